@@ -1433,8 +1433,18 @@ struct TbVel {
           r.x_off[s] = (float)(sub_w * (float)s + sub_w / 2.);
           r.x_pos[s] = (float)(r.x_off[s] / (box_mpc / (float)N));
         }
+        // columns per workgroup: the fewest that leave the fewest idle threads
+        // in its rounds of kNT cells, up to 768 cells (36 KiB of LDS)
+        int ncol = 1;
+        auto idle = [](int c) { return (double)((c * N + kNT - 1) / kNT * kNT) / (c * N); };
+        for (int c = 2; c <= 16 && c * N <= 768; c *= 2)
+          if (idle(c) < idle(ncol)) ncol = c;
+        uint8_t* todo = ctx->state;  // N^2 column flags
         PROF("rsd_los");
-        k_rsd_los<<<(unsigned)(((long)N * N + kNT - 1) / kNT), kNT, 0, ctx->stream>>>(dT, xH, vel, grad + np, r);
+        k_rsd_gather<<<(unsigned)(N * N / ncol), kNT, rsd_gather_lds(ncol * N), ctx->stream>>>(dT, xH, vel, todo, ncol,
+                                                                                            r);
+        MRX_TRY(check_launch(ctx, "k_rsd_gather"));
+        k_rsd_los<<<(unsigned)(((long)N * N + kNT - 1) / kNT), kNT, 0, ctx->stream>>>(dT, xH, vel, grad + np, todo, r);
         MRX_TRY(check_launch(ctx, "k_rsd_los"));
       }
       MRX_TRY(ensure_partials(ctx, 1024 + 8));

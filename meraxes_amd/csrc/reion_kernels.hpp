@@ -1708,13 +1708,16 @@ struct RsdGlobalSink {
   }
 };
 
+// The columns k_rsd_gather leaves to it (todo[col] != 0: displacements beyond
+// its reach, or not finite), one thread per column, in the reference's order.
 __global__ __launch_bounds__(kNT) void k_rsd_los(float* __restrict__ dT, const float* __restrict__ xH,
-                                                const float* __restrict__ vel, float* __restrict__ bins, RsdArgs a)
+                                                const float* __restrict__ vel, float* __restrict__ bins,
+                                                const uint8_t* __restrict__ todo, RsdArgs a)
 {
   const long col = (long)blockIdx.x * kNT + threadIdx.x;
   const int N = a.N;
   const long NN = (long)N * N;
-  if (col >= NN) return;
+  if (col >= NN || !todo[col]) return;
   const float* dt = dT + col * N;
   const float* xh = xH + col * N;
   const float* vl = vel + col * (N + 2);
@@ -1729,6 +1732,210 @@ __global__ __launch_bounds__(kNT) void k_rsd_los(float* __restrict__ dT, const f
     rsd_cell(k, N, d, vl[km] / a.H_z, vl[k] / a.H_z, vl[k] / a.H_z, vl[kp] / a.H_z, a, g);
   }
   for (int k = 0; k < N; ++k) o[k] = b[k * NN];
+}
+
+// The re-binning as a gather, one thread per bin.  rsd_cell's loop is serial
+// along a column only because a bin's float sum must be formed in the order
+// (cell, sub-cell); a bin hears from the few cells that reach it, so every bin
+// can form its own sum in that order.  One thread per column kept 4 waves per
+// SIMD busy with dependent read-modify-writes and 6.7e9 FP64 placements at
+// 512^3 (37 ms; at 32^3, 1024 threads in all, 2.3 ms).  At 256^3 the whole
+// delta_T call went from 10.4 to 1.31 ms.
+//
+// Phase 1, one thread per cell: each of the 50 sub-cells gets a class, "whole
+// in bin k + a" or "across k + a and k + a + 1", held as five 64-bit planes in
+// LDS (sub-cell s is bit s).  Within a half cell the position is linear in s
+// up to rounding (the float tables x_pos and x_off move it by < 1e-6 cells),
+// so the sub-cells at least kRsdMargin inside a bin are classified in runs by
+// solving for s; only the others (one or two per cell edge) are placed by the
+// reference's double expressions, which alone decide near an edge.
+// Phase 2, one thread per bin: over the cells that can reach it, in the
+// reference's order of k (the wrapped ones where the reference meets them),
+// the runs of whole sub-cells are float additions of d / 50 and the divided
+// ones take the reference's double fractions.
+// Reach: kRsdReach bins either way; a column with a larger (or non-finite)
+// displacement is flagged in `todo` and left untouched for k_rsd_los.
+constexpr int kRsdReach = 7;         // 2 (2 * 7 + 1) - 1 = 29 classes, ids 1..29 in five bits
+constexpr int kRsdPlanes = 5;
+constexpr double kRsdMaxDisp = 5.9;  // cells; floor(-5.9) = -6, floor(1 + 5.9) + 1 = 7
+constexpr float kRsdMargin = 1e-4f;
+
+// Class id of a sub-cell: whole in bin a, or divided between a and a + 1.
+__device__ __forceinline__ int rsd_id(int a, bool split) { return 2 * (a + kRsdReach) + (split ? 2 : 1); }
+
+// Edges of sub-cell s, and its lower bin with rsd_cell's cases: returns its class.
+__device__ __forceinline__ void rsd_edges(int s, double d1_low, double d2_low, double d2_high, const RsdArgs& a,
+                                          double& lo, double& hi)
+{
+  const double xp = a.x_pos[s];
+  const double disp = (xp <= 0.5) ? d1_low + ((xp + 0.5) - 0.) * (d2_low - d1_low) / (1. - 0.)
+                                  : d2_low + ((xp - 0.5) - 0.) * (d2_high - d2_low) / (1. - 0.);
+  const double pos = ((double)a.x_off[s] + disp) / a.cell;
+  lo = pos - a.half;
+  hi = pos + a.half;
+}
+
+__device__ __forceinline__ int rsd_class(double lo, double hi)
+{
+  if (lo >= 0.0 && hi < 1.0) return rsd_id(0, false);
+  if (lo < 0.0 && hi < 0.0) {
+    const double cd = ceil(fabs(lo)) - 1.;
+    return rsd_id(-((int)cd + 1), !(fabs(hi) > cd));
+  }
+  if (lo < 0.0 && (hi > 0.0 && hi < 1.0)) return rsd_id(-1, true);
+  if ((lo >= 0.0 && lo < 1.0) && hi >= 1.0) return rsd_id(0, true);
+  const double cd = floor(fabs(hi));
+  const int c = (int)cd;
+  return (lo >= cd) ? rsd_id(c, false) : rsd_id(c - 1, true);
+}
+
+// The double share of a divided sub-cell in its lower or upper bin.
+__device__ __forceinline__ double rsd_share(double lo, double hi, bool upper, float d, const RsdArgs& a)
+{
+  double up, dn;
+  if (lo < 0.0 && hi < 0.0) {
+    dn = (fabs(lo) - (ceil(fabs(lo)) - 1.)) / a.frac_w;
+    up = 1. - dn;
+  } else if (lo < 0.0 && (hi > 0.0 && hi < 1.0)) {
+    up = hi / a.frac_w;
+    dn = 1. - up;
+  } else if ((lo >= 0.0 && lo < 1.0) && hi >= 1.0) {
+    up = (hi - 1.) / a.frac_w;
+    dn = 1. - up;
+  } else {
+    up = (hi - floor(fabs(hi))) / a.frac_w;
+    dn = 1. - up;
+  }
+  return (upper ? up : dn) * (double)d / (double)(float)kRsdSteps;
+}
+
+// ncol columns per workgroup (ncol * N cells); dynamic LDS rsd_gather_lds(ncol * N).
+constexpr size_t rsd_gather_lds(int cells) { return (size_t)cells * (kRsdPlanes * 8 + 8); }
+
+__global__ __launch_bounds__(kNT) void k_rsd_gather(float* __restrict__ dT, const float* __restrict__ xH,
+                                                   const float* __restrict__ vel, uint8_t* __restrict__ todo,
+                                                   int ncol, RsdArgs a)
+{
+  extern __shared__ uint64_t rsd_lds[];
+  __shared__ int reach[16], bad[16];  // per column of the workgroup (ncol <= 16)
+  const int N = a.N, tid = threadIdx.x;
+  const int cells = ncol * N;
+  uint64_t* plane = rsd_lds;                                             // [kRsdPlanes][cells]
+  float* dv = reinterpret_cast<float*>(rsd_lds + (size_t)kRsdPlanes * cells);  // delta_T; 0 planes: contributes nothing
+  float* dsp = dv + cells;                                               // displacement v / H
+  const long col0 = (long)blockIdx.x * ncol;
+  if (tid < ncol) reach[tid] = bad[tid] = 0;
+  __syncthreads();
+  for (int e = tid; e < cells; e += kNT) {
+    const int cl = e / N, k = e - cl * N;
+    const float v = vel[(col0 + cl) * (N + 2) + k] / a.H_z;
+    dv[e] = dT[(col0 + cl) * N + k];
+    dsp[e] = v;
+    if (!(fabs((double)v) <= kRsdMaxDisp * a.cell)) bad[cl] = 1;
+  }
+  __syncthreads();
+  const float inv_cell = (float)(1.0 / a.cell);
+  constexpr float w = 1.0f / kRsdSteps;
+  // phase 1
+  for (int e = tid; e < cells; e += kNT) {
+    const int cl = e / N, k = e - cl * N;
+    uint64_t pl[kRsdPlanes] = {0, 0, 0, 0, 0};
+    const float d = dv[e];
+    if (!bad[cl] && fabs((double)d) >= 1e-7 && (double)xH[(col0 + cl) * N + k] >= 1e-7) {
+      const float fl = dsp[k == 0 ? e + N - 1 : e - 1], fc = dsp[e], fh = dsp[k == N - 1 ? e - (N - 1) : e + 1];
+      const double dl = fl, dc = fc, dh = fh;
+      uint64_t todo_s = (1ull << kRsdSteps) - 1;
+      int amax = 0;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        // lo(s) ~ lo0 + s dp over the sub-cells [s0, s0 + 25) of this half
+        constexpr int HS = kRsdSteps / 2;
+        const int s0 = h * HS;
+        const float da = (h ? fc : fl) * inv_cell, db = (h ? fh : fc) * inv_cell;
+        const float x0 = (s0 + 0.5f) * w;
+        const float dp = w * (1.0f + (db - da));
+        const float lo0 = x0 - 0.5f * w + da + (x0 + (h ? -0.5f : 0.5f)) * (db - da);
+        if (!(dp > 0.1f * w)) continue;  // (nearly) crossing sub-cells: place each
+        const float inv_dp = 1.0f / dp;
+        const int a1 = (int)floorf(lo0 + (HS - 1) * dp);
+        for (int q = (int)floorf(lo0); q <= a1; ++q) {
+          const int i1 = max((int)ceilf(((float)q + kRsdMargin - lo0) * inv_dp), 0);
+          const int i2 = min((int)floorf(((float)(q + 1) - kRsdMargin - w - lo0) * inv_dp), HS - 1);
+          if (i1 > i2) continue;
+          const uint64_t run = ((1ull << (i2 - i1 + 1)) - 1) << (s0 + i1);
+          const int id = rsd_id(q, false);
+#pragma unroll
+          for (int p = 0; p < kRsdPlanes; ++p)
+            if ((id >> p) & 1) pl[p] |= run;
+          todo_s &= ~run;
+          amax = max(amax, q < 0 ? -q : q);
+        }
+      }
+      while (todo_s) {
+        const int s = __ffsll((unsigned long long)todo_s) - 1;
+        todo_s &= todo_s - 1;
+        double lo, hi;
+        rsd_edges(s, dl, dc, dh, a, lo, hi);
+        const int id = rsd_class(lo, hi);
+#pragma unroll
+        for (int p = 0; p < kRsdPlanes; ++p) pl[p] |= (uint64_t)((id >> p) & 1) << s;
+        const int q = (id - 1) / 2 - kRsdReach;  // lower bin
+        amax = max(amax, max(-q, (id & 1) ? q : q + 1));
+      }
+      if (amax > reach[cl]) atomicMax(&reach[cl], amax);
+    }
+#pragma unroll
+    for (int p = 0; p < kRsdPlanes; ++p) plane[(size_t)p * cells + e] = pl[p];
+  }
+  __syncthreads();
+  // phase 2
+  for (int e = tid; e < cells; e += kNT) {
+    const int cl = e / N, b = e - cl * N;
+    if (bad[cl]) continue;
+    const int W = reach[cl], n = 2 * W + 1;
+    // sources b - W .. b + W, taken modulo N in increasing order
+    const int rot = (b < W) ? W - b : (b + W >= N ? N - (b - W) : 0);
+    float acc = 0.0f;
+    for (int j = 0; j < n; ++j) {
+      int jj = j + rot;
+      if (jj >= n) jj -= n;
+      int k = b - W + jj;
+      const int o = W - jj;  // the bin's offset from its source cell
+      if (k < 0) k += N;
+      if (k >= N) k -= N;
+      const int src = cl * N + k;
+      const int id = rsd_id(o, false);
+      uint64_t mf = (1ull << kRsdSteps) - 1, mlo = mf, mup = mf;  // whole; divided, lower bin; divided, upper bin
+#pragma unroll
+      for (int p = 0; p < kRsdPlanes; ++p) {
+        const uint64_t v = plane[(size_t)p * cells + src];
+        mf &= ((id >> p) & 1) ? v : ~v;
+        mlo &= (((id + 1) >> p) & 1) ? v : ~v;
+        mup &= (((id - 1) >> p) & 1) ? v : ~v;
+      }
+      uint64_t m = mf | mlo | mup;
+      if (!m) continue;
+      const float d = dv[src];
+      const float share = d / (float)kRsdSteps;
+      while (m) {
+        const int s = __ffsll((unsigned long long)m) - 1;
+        if ((mf >> s) & 1) {
+          const int run = __ffsll((unsigned long long)~(mf >> s)) - 1;
+          for (int i = 0; i < run; ++i) acc = acc + share;
+          m &= ~(((1ull << run) - 1) << s);
+        } else {
+          const double dl = dsp[k == 0 ? src + N - 1 : src - 1], dc = dsp[src],
+                       dh = dsp[k == N - 1 ? src - (N - 1) : src + 1];
+          double lo, hi;
+          rsd_edges(s, dl, dc, dh, a, lo, hi);
+          acc = (float)((double)acc + rsd_share(lo, hi, (mup >> s) & 1, d, a));
+          m &= m - 1;
+        }
+      }
+    }
+    dT[(col0 + cl) * N + b] = acc;
+  }
+  if (tid < ncol) todo[col0 + tid] = (uint8_t)bad[tid];
 }
 #pragma clang fp contract(on)
 

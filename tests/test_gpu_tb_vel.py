@@ -112,6 +112,22 @@ def test_tb_vel_large_displacements_rebinning_exact(ctx):
     assert moved > 0.1 * np.abs(g2).max()  # multi-cell moves happened
 
 
+@pytest.mark.parametrize("N,disp,width", [(32, 0.2, 4.0), (48, 1.0, 2.0), (96, 2.0, 1.5), (160, 0.4, 3.0),
+                                          (320, 0.3, 3.0), (32, 4.0, 1.0), (64, 30.0, 2.0)])
+def test_tb_vel_rebinning_gather_exact(ctx, N, disp, width):
+    """The gathered re-binning against the oracle's serial one, bit for bit, on the GPU's own
+    pec_vels 2 field: one to sixteen columns per workgroup, cells that cross each other
+    (steep velocities), and columns on either side of the gather's reach of 7 cells
+    (displacements of 4 and 30 cells rms: some and nearly all beyond it)."""
+    xH, d, TS, vel = inputs(N, 100.0 * N / 64, 51 + N, 0, disp_rms=disp, width=width)
+    p2 = P.tb_vel_params(N, 100.0 * N / 64, 8.0, pec_vels=2, trees_id=0)
+    p3 = P.tb_vel_params(N, 100.0 * N / 64, 8.0, pec_vels=3, trees_id=0)
+    g2, _, g_vel = run_gpu(ctx, p2, xH, d, TS, vel, True)
+    g3, _, _ = run_gpu(ctx, p3, xH, d, TS, vel, True)
+    o3 = O.rsd_los(p3, xH, g_vel, g2)
+    assert np.array_equal(g3.view(np.uint32), o3.view(np.uint32)), int((g3 != o3).sum())
+
+
 def test_tb_vel_without_spin_temperature_is_plain_tb(ctx):
     N = 32
     xH, d, TS, vel = inputs(N, 50.0, 3, 1)
