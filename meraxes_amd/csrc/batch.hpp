@@ -89,6 +89,7 @@ struct Cohort {
   uint8_t* state = nullptr;
   float2* tw = nullptr;
   float* Rtab = nullptr;
+  StepDev* steps = nullptr;
   float* wtab = nullptr;
   double* partials = nullptr;
   double* sums = nullptr;
@@ -108,6 +109,7 @@ void free_cohort(Cohort& c)
   dfree(c.state);
   dfree(c.tw);
   dfree(c.Rtab);
+  dfree(c.steps);
   dfree(c.wtab);
   dfree(c.partials);
   dfree(c.sums);
@@ -119,15 +121,6 @@ void free_cohort(Cohort& c)
   c.stream = nullptr;
   if (c.done) (void)hipEventDestroy(c.done);
   c.done = nullptr;
-}
-
-// J_21 constant of find_HII_bubbles.c:317-320 at radius R, evaluated exactly
-// as the single-box path does.
-double j21_const(const mrx_hii_params* p, double R)
-{
-  const double z = p->redshift;
-  return (1.0 + z) * (1.0 + z) / (4.0 * M_PI) * p->alpha_uv * kPlanck * 1e21 * R * p->unit_length_cm *
-         p->nion_phot_per_bary / kProtonMass * p->unit_mass_g / pow(p->unit_length_cm, 3) / p->unit_time_s;
 }
 
 bool same_cohort(const mrx_hii_params& a, const mrx_hii_params& b)
@@ -142,7 +135,7 @@ template <int N>
 struct BatchPipe {
   static constexpr int NH = N / 2;
   static constexpr long nc = (long)N * N * NH;
-  static int nb_threshold() { return N * N / ThrCfg<N>::RZ; }
+  static int nb_threshold() { return N * N / RowCfg<N>::ROWS; }
 
   struct Fwd {
     mrx_ctx* ctx;
@@ -225,18 +218,15 @@ struct BatchPipe {
       const bool last = (s == c.S - 1);
       const WinArgs w = win_args(p->box_size, (float)c.R[s], p->filter_type, 1);
       MRX_TRY(inverse_xy(ctx, c, last ? nullptr : &w, c.variant));
-      a.M_mean = RtoM(p, c.R[s]);
-      a.R_cubed = c.R[s] * c.R[s] * c.R[s];
-      a.kfc = (4.0 / 3.0) * M_PI * a.R_cubed / a.pixel_volume / a.M_mean;
       a.step = s;
       a.last = last ? 1 : 0;
-      constexpr int NT = ThrCfg<N>::NT;
+      constexpr int NT = RowCfg<N>::NT;
       if (c.F == 4)
         k_c2r_threshold_batch<N, 4><<<dim3(nb, c.nbox), NT, 0, c.stream>>>(
-          c.T, nc, (long)c.F * nc, c.tw, c.boxes_dev, c.state, c.Rtab, c.J21c, c.S, c.partials, a);
+          c.T, nc, (long)c.F * nc, c.tw, c.boxes_dev, c.state, c.Rtab, c.steps, c.J21c, c.S, c.partials, a);
       else
         k_c2r_threshold_batch<N, 3><<<dim3(nb, c.nbox), NT, 0, c.stream>>>(
-          c.T, nc, (long)c.F * nc, c.tw, c.boxes_dev, c.state, c.Rtab, c.J21c, c.S, c.partials, a);
+          c.T, nc, (long)c.F * nc, c.tw, c.boxes_dev, c.state, c.Rtab, c.steps, c.J21c, c.S, c.partials, a);
       MRX_TRY(check_launch(ctx, "k_c2r_threshold_batch"));
     }
     // the same reduction as the single-box path, so each box's globals are identical to it
@@ -260,6 +250,7 @@ struct BatchPipe {
     MRX_TRY(alloc((void**)&c.state, (size_t)N * N * N * c.nbox));
     MRX_TRY(alloc((void**)&c.tw, sizeof(float2) * N));
     MRX_TRY(alloc((void**)&c.Rtab, sizeof(float) * c.S));
+    MRX_TRY(alloc((void**)&c.steps, sizeof(StepDev) * c.S));
     MRX_TRY(alloc((void**)&c.wtab, sizeof(float) * (size_t)(NH + 1) * (NH + 1) * (NH + 1)));
     MRX_TRY(alloc((void**)&c.partials,
                   sizeof(double) * ((size_t)nb_threshold() * 4 + (size_t)kRedBlocks * kRedMaxV) * c.nbox));
@@ -276,6 +267,9 @@ struct BatchPipe {
     std::vector<float> Rf(c.S);
     for (int s = 0; s < c.S; ++s) Rf[s] = (float)c.R[s];
     HIP_TRY(hipMemcpy(c.Rtab, Rf.data(), sizeof(float) * c.S, hipMemcpyHostToDevice));
+    std::vector<StepDev> sd(c.S);
+    for (int s = 0; s < c.S; ++s) sd[s] = step_consts(&c.p0, c.R[s], false);
+    HIP_TRY(hipMemcpy(c.steps, sd.data(), sizeof(StepDev) * c.S, hipMemcpyHostToDevice));
     std::vector<BoxDev> bd(c.nbox);
     std::vector<double> j(c.nbox * c.S);
     std::vector<const float*> in(nf);
@@ -290,7 +284,7 @@ struct BatchPipe {
       bd[i].eff = b.params.efficiency;
       bd[i].redshift = b.params.redshift;
       bd[i].bias = b.params.gamma_halo_bias;
-      for (int s = 0; s < c.S; ++s) j[(size_t)i * c.S + s] = j21_const(&b.params, c.R[s]);
+      for (int s = 0; s < c.S; ++s) j[(size_t)i * c.S + s] = step_consts(&b.params, c.R[s], false).J21c;
       const float* src[4] = {b.deltax, b.stars, b.weighted_sfr, b.x_e};
       for (int f = 0; f < c.F; ++f) in[(size_t)i * c.F + f] = src[f];
     }

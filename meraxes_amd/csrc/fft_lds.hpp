@@ -337,6 +337,8 @@ struct SchedV;
 #define MRX_SCHED(L_, V_, ...)                                                                             \
   template <>                                                                                             \
   struct SchedV<L_, V_> {                                                                                 \
+    static constexpr int radix[] = {__VA_ARGS__};                                                         \
+    static constexpr int nradix = sizeof(radix) / sizeof(int);                                            \
     template <int NCOL, int NT, bool INV, int SN, int SC, bool CFAST, int TWS, bool PAD>                  \
     __device__ __forceinline__ static void run(float2* s, const float2* tw, int tid)                      \
     {                                                                                                     \

@@ -94,7 +94,8 @@ struct mrx_ctx {
   float2* V = nullptr;
   uint8_t* state = nullptr;
   float2* tw = nullptr;
-  float* Rtab = nullptr;
+  StepDev* steps = nullptr;  // the ladder's steps (kMaxSteps + 1 entries), then its radii (Rtab)
+  float* Rtab = nullptr;     // within the steps allocation
   double* partials = nullptr;
   size_t partials_cap = 0;
   double* sums = nullptr;
@@ -627,44 +628,52 @@ struct Pipe {
                                                                               (long)N * N * pitch, clamp, pitch, kzlive);
       return check_launch(ctx, "k_c2r_z_reg");
     }
-    const dim3 gz(N * N / Cfg<N>::RZ, nfield);
-    k_c2r_z<N><<<gz, kNT, 0, ctx->stream>>>(T, out, ctx->tw, nc, (long)N * N * pitch, clamp, pitch, kzlive);
+    const dim3 gz(N * N / RowCfg<N>::ROWS, nfield);
+    k_c2r_z<N><<<gz, RowCfg<N>::NT, 0, ctx->stream>>>(T, out, ctx->tw, nc, (long)N * N * pitch, clamp, pitch, kzlive);
     return check_launch(ctx, "k_c2r_z");
   }
 
-  // the ladder's last pass; fields deltax, stars, sfr (+ x_e) (+ N_rec when rec)
+  // the last pass of K ladder steps, step k's spectra at Tsrc + k tstride;
+  // fields deltax, stars, sfr (+ x_e) (+ N_rec when rec)
   // 256^3 and 512^3 without recombinations: the row transforms in registers
-  // (k_c2r_threshold_reg); otherwise staged in LDS (k_c2r_threshold)
+  // (k_c2r_threshold_reg); otherwise row_fft.hpp's (k_c2r_threshold)
   static constexpr bool kRegThr = (N == 256 || N == 512);
-  static int threshold(mrx_ctx* ctx, const float2* Tsrc, const float* deltax, float* xH, float* rb, float* J21,
-                       float* zin, float* J21i, float* Gamma12, bool rec, const StepArgs& a)
+  static int threshold(mrx_ctx* ctx, const float2* Tsrc, long tstride, int K, const float* deltax, float* xH,
+                       float* rb, float* J21, float* zin, float* J21i, float* Gamma12, bool rec, const StepArgs& a)
   {
     const int nb = nblocks_threshold(rec);
-    PROF("c2r_threshold");
+    const ThrGrids g{deltax, ctx->state, xH, rb, J21, zin, J21i, Gamma12, ctx->Rtab};
     if constexpr (kRegThr) {
       if (!rec) {
         constexpr int A = N / 32;
-        if (a.nfield == 4)
-          k_c2r_threshold_reg<A, 4><<<nb, 256, 0, ctx->stream>>>(Tsrc, nc, ctx->tw, deltax, ctx->state, xH, rb, J21,
-                                                                zin, J21i, ctx->Rtab, ctx->partials, a);
-        else
-          k_c2r_threshold_reg<A, 3><<<nb, 256, 0, ctx->stream>>>(Tsrc, nc, ctx->tw, deltax, ctx->state, xH, rb, J21,
-                                                                zin, J21i, ctx->Rtab, ctx->partials, a);
+        StepArgs ak = a;
+        for (int k = 0; k < K; ++k, ++ak.step) {
+          PROF("c2r_threshold");
+          const float2* Tk = Tsrc + k * tstride;
+          if (a.nfield == 4)
+            k_c2r_threshold_reg<A, 4><<<nb, 256, 0, ctx->stream>>>(Tk, nc, ctx->tw, ctx->steps, g, ctx->partials, ak);
+          else
+            k_c2r_threshold_reg<A, 3><<<nb, 256, 0, ctx->stream>>>(Tk, nc, ctx->tw, ctx->steps, g, ctx->partials, ak);
+        }
         return check_launch(ctx, "k_c2r_threshold_reg");
       }
     }
-    constexpr int NT = ThrCfg<N>::NT;
-#define MRX_THR(NF_, REC_)                                                                                          \
-  k_c2r_threshold<N, NF_, REC_><<<nb, NT, 0, ctx->stream>>>(Tsrc, nc, ctx->tw, deltax, ctx->state, xH, rb, J21,   \
-                                                           zin, J21i, Gamma12, ctx->Rtab, ctx->partials, a)
-    if (!rec && a.nfield == 4)
-      MRX_THR(4, false);
-    else if (!rec)
-      MRX_THR(3, false);
-    else if (a.nfield == 5)
-      MRX_THR(5, true);
-    else
-      MRX_THR(4, true);
+    PROF("c2r_threshold");
+    constexpr int NT = RowCfg<N>::NT;
+#define MRX_THR(NF_, REC_)                                                                                  \
+  k_c2r_threshold<N, NF_, REC_><<<nb, NT, 0, ctx->stream>>>(Tsrc, nc, tstride, K, ctx->tw, ctx->steps, g, \
+                                                           ctx->partials, a)
+    if (rec) {
+      if (a.nfield == 5)
+        MRX_THR(5, true);
+      else
+        MRX_THR(4, true);
+    } else if constexpr (!kRegThr) {
+      if (a.nfield == 4)
+        MRX_THR(4, false);
+      else
+        MRX_THR(3, false);
+    }
 #undef MRX_THR
     return check_launch(ctx, "k_c2r_threshold");
   }
@@ -674,7 +683,7 @@ struct Pipe {
     if constexpr (kRegThr) {
       if (!rec) return N * N / RegThr<N / 32>::RWG;
     }
-    return N * N / ThrCfg<N>::RZ;
+    return N * N / RowCfg<N>::ROWS;
   }
 
   static int pack_herm(mrx_ctx* ctx, const float2* H, float2* U)
@@ -791,6 +800,29 @@ int rr_tables(mrx_ctx* ctx, const mrx_hii_params* p, const RRDev** out)
   return MRX_OK;
 }
 
+// The constants of one ladder step at radius R (find_HII_bubbles.c:317-340).
+StepDev step_consts(const mrx_hii_params* p, double R, bool rec)
+{
+  const double z = p->redshift;
+  const double pixel_volume = pow(p->box_size / (double)p->grid_dim, 3);
+  StepDev d;
+  d.J21c = (1.0 + z) * (1.0 + z) / (4.0 * M_PI) * p->alpha_uv * kPlanck * 1e21 * R * p->unit_length_cm *
+           p->nion_phot_per_bary / kProtonMass * p->unit_mass_g / pow(p->unit_length_cm, 3) / p->unit_time_s;
+  d.M_mean = RtoM(p, R);
+  d.R_cubed = R * R * R;
+  d.kfc = (4.0 / 3.0) * M_PI * d.R_cubed / pixel_volume / d.M_mean;
+  d.gamma_pref = 0.0;
+  if (rec) {
+    // Gamma_R_prefactor (find_HII_bubbles.c:325-334): R h^-1 to R, pixel volume (Mpc/h)^3 to cm^3
+    double gp = (1.0 + z) * (1.0 + z) * R * (p->unit_length_cm / p->hubble_h) * kSigmaHI * p->alpha_uv /
+                (p->alpha_uv + 2.75) / 1.0e-12;
+    gp *= (p->unit_mass_g / p->unit_time_s) * pow(p->unit_length_cm / p->hubble_h, -3.) * p->nion_phot_per_bary /
+          kProtonMass;
+    d.gamma_pref = gp;
+  }
+  return d;
+}
+
 struct HiiRun {
   template <int N>
   struct At {
@@ -809,11 +841,23 @@ struct HiiRun {
       if (S < 1) return set_err(ctx, MRX_EINVAL, "radius ladder is empty");
       if (S > kMaxSteps) return set_err(ctx, MRX_EUNSUPPORTED, "radius ladder has %d steps (max %d)", S, kMaxSteps);
       MRX_TRY(ensure_partials(ctx, (size_t)P::nblocks_threshold(rec) * 4 + 8 + kRedBlocks * kRedMaxV));
-      if (!ctx->Rtab) HIP_TRY(hipMalloc(&ctx->Rtab, sizeof(float) * 256));
       if (!ctx->sums) HIP_TRY(hipMalloc(&ctx->sums, sizeof(double) * 8));
-      std::vector<float> Rf(S);
-      for (int s = 0; s < S; ++s) Rf[s] = (float)R[s];
-      HIP_TRY(hipMemcpyAsync(ctx->Rtab, Rf.data(), sizeof(float) * S, hipMemcpyHostToDevice, ctx->stream));
+      // the steps' constants and radii, in one upload
+      constexpr size_t kStepBytes = sizeof(StepDev) * (kMaxSteps + 1);
+      if (!ctx->steps) {
+        HIP_TRY(hipMalloc(&ctx->steps, kStepBytes + sizeof(float) * (kMaxSteps + 1)));
+        ctx->Rtab = reinterpret_cast<float*>(reinterpret_cast<char*>(ctx->steps) + kStepBytes);
+      }
+      std::vector<char> htab(kStepBytes + sizeof(float) * S);
+      {
+        StepDev* hs = reinterpret_cast<StepDev*>(htab.data());
+        float* hr = reinterpret_cast<float*>(htab.data() + kStepBytes);
+        for (int s = 0; s < S; ++s) {
+          hs[s] = step_consts(p, R[s], rec);
+          hr[s] = (float)R[s];
+        }
+      }
+      HIP_TRY(hipMemcpyAsync(ctx->steps, htab.data(), htab.size(), hipMemcpyHostToDevice, ctx->stream));
 
       // inputs: deltax, stars, weighted_sfr, x_e are padded and laid out at a
       // fixed stride when staged; device pointers are used where they lie.
@@ -871,6 +915,7 @@ struct HiiRun {
       (void)fs;
       const double pixel_volume = pow(box_size / (double)N, 3);
       StepArgs a;
+      memset(&a, 0, sizeof a);
       a.pixel_volume = pixel_volume;
       a.eff = p->efficiency;
       a.redshift = p->redshift;
@@ -878,7 +923,6 @@ struct HiiRun {
       a.uvb = p->uvb_flag;
       a.use_xe = p->include_spin_temp;
       a.nfield = nfield;
-      const double z = p->redshift;
       // the filtered radii go through the x pass ladder_radii at a time
       // (tabulated windows; KL = 0: sharp-k, one radius per pass over its live
       // tiles) when the spectra of that many radii fit, else one at a time
@@ -896,33 +940,15 @@ struct HiiRun {
           float2* TK = KL > 1 ? ctx->TK : ctx->T;
           MRX_TRY(P::inverse_xy_k(ctx, ctx->U, ctx->V, TK, tstride, nfield, ws, K, wpre ? wpre + s * nt : nullptr));
           a.kzlive = N / 2;
+          Tsrc = TK;
+        } else {
+          const WinArgs w = win_args(box_size, (float)R[s], p->filter_type, last ? 0 : 1);
+          MRX_TRY(P::inverse_xy(ctx, ctx->U, ctx->V, ctx->T, nfield, w, a.kzlive));
         }
-        for (int k = 0; k < K; ++k, ++s) {
-          if (KL >= 1 && !last) {
-            Tsrc = (KL > 1 ? ctx->TK : ctx->T) + k * tstride;
-          } else {
-            const WinArgs w = win_args(box_size, (float)R[s], p->filter_type, last ? 0 : 1);
-            MRX_TRY(P::inverse_xy(ctx, ctx->U, ctx->V, ctx->T, nfield, w, a.kzlive));
-          }
-          a.J21c = (1.0 + z) * (1.0 + z) / (4.0 * M_PI) * p->alpha_uv * kPlanck * 1e21 * R[s] * p->unit_length_cm *
-                   p->nion_phot_per_bary / kProtonMass * p->unit_mass_g / pow(p->unit_length_cm, 3) / p->unit_time_s;
-          a.M_mean = RtoM(p, R[s]);
-          a.R_cubed = R[s] * R[s] * R[s];
-          a.kfc = (4.0 / 3.0) * M_PI * a.R_cubed / a.pixel_volume / a.M_mean;
-          if (rec) {
-            // Gamma_R_prefactor (find_HII_bubbles.c:325-334): R h^-1 to R, pixel volume (Mpc/h)^3 to cm^3
-            double gp = (1.0 + z) * (1.0 + z) * R[s] * (p->unit_length_cm / p->hubble_h) * kSigmaHI * p->alpha_uv /
-                        (p->alpha_uv + 2.75) / 1.0e-12;
-            gp *= (p->unit_mass_g / p->unit_time_s) * pow(p->unit_length_cm / p->hubble_h, -3.) *
-                  p->nion_phot_per_bary / kProtonMass;
-            a.gamma_pref = gp;
-          } else {
-            a.gamma_pref = 0.0;
-          }
-          a.step = s;
-          a.last = last ? 1 : 0;
-          MRX_TRY(P::threshold(ctx, Tsrc, deltax, out[0], out[1], out[2], out[3], out[4], out[5], rec, a));
-        }
+        a.step = s;
+        a.last = last ? 1 : 0;
+        MRX_TRY(P::threshold(ctx, Tsrc, tstride, K, deltax, out[0], out[1], out[2], out[3], out[4], out[5], rec, a));
+        s += K;
       }
       if (rec) {
         // N_rec += dNrec after the ladder (:472-477)
@@ -1896,7 +1922,7 @@ int mrx_free(mrx_ctx* ctx)
   dfree(ctx->V);
   dfree(ctx->state);
   dfree(ctx->tw);
-  dfree(ctx->Rtab);
+  dfree(ctx->steps);
   dfree(ctx->partials);
   dfree(ctx->sums);
   dfree(ctx->stage);

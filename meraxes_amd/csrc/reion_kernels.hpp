@@ -23,6 +23,7 @@
 #include <stdint.h>
 
 #include "fft_lds.hpp"
+#include "row_fft.hpp"
 
 namespace mrx {
 
@@ -47,15 +48,6 @@ constexpr int z_rows(int NH)
 {
   int r = (NH >= kZE) ? 1 : pow2_floor(kZE / NH);
   while ((r * NH) % 512 != 0) r *= 2;
-  return r;
-}
-
-// The fewest rows of NH complex holding a multiple of 128 elements (4-cell
-// groups over one 64-thread wave).
-constexpr int z_rows_wave(int NH)
-{
-  int r = 1;
-  while ((r * NH) % 128 != 0) r *= 2;
   return r;
 }
 
@@ -220,67 +212,6 @@ __global__ __launch_bounds__(kNT) void k_r2c_z_tab(const float* const* __restric
   r2c_z_tile<N>(in_tab[blockIdx.y], out + blockIdx.y * out_fstride, twN);
 }
 
-// ---------------------------------------------------- z: C2R load + FFT
-// Untwists ROWS packed rows held in LDS and runs the inverse length-N/2 FFT
-// on all of them with NT threads; afterwards the tile, read as floats, holds
-// ROWS real rows of N.
-template <int N, int ROWS, int NT>
-__device__ __forceinline__ void c2r_untwist_rows(float2* s, const float2* tw, int tid)
-{
-  constexpr int NH = N / 2;
-  constexpr int NP = NH / 2 + 1;
-  for (int q = tid; q < ROWS * NP; q += NT) {
-    const int r = q / NP, k = q % NP;
-    const int rb = r * NH;
-    if (k == 0) {
-      const float2 p = s[lds_addr<true>(rb)];  // (X_0, X_{N/2}), both real
-      s[lds_addr<true>(rb)] = make_float2(p.x + p.y, p.x - p.y);
-    } else {
-      const float2 xk = s[lds_addr<true>(rb + k)], xm = cconj(s[lds_addr<true>(rb + NH - k)]);
-      const float2 E = cadd(xk, xm);
-      const float2 O = cmul(csub(xk, xm), cconj(tw[k]));  // * exp(+2 pi i k / N)
-      s[lds_addr<true>(rb + k)] = make_float2(E.x - O.y, E.y + O.x);  // E + i O
-      if (k != NH - k) s[lds_addr<true>(rb + NH - k)] = make_float2(E.x + O.y, -E.y + O.x);  // conj(E) + i conj(O)
-    }
-  }
-  __syncthreads();
-  fft_lds<NH, ROWS, NT, true, 1, NH, false, 2, true>(s, tw, tid);
-}
-
-template <int N>
-__device__ __forceinline__ void c2r_untwist_fft(float2* s, const float2* tw, int tid)
-{
-  c2r_untwist_rows<N, Cfg<N>::RZ, kNT>(s, tw, tid);
-}
-
-// Loads RZ packed rows, untwists them and runs the inverse length-N/2 FFT in
-// LDS; afterwards real cell e of the tile is lds_real<N>(s, e).  Slots kz >=
-// kzlive are read as zero (not loaded).
-template <int N>
-__device__ __forceinline__ void c2r_rows_lds(float2* s, const float2* tw, const float2* __restrict__ src, long row0,
-                                             int tid, int kzlive)
-{
-  using C = Cfg<N>;
-  constexpr int NH = C::NH, ZE = C::ZE;
-  constexpr int EPZ = ZE / kNT;
-  float2 v[EPZ];
-#pragma unroll
-  for (int i = 0; i < EPZ; ++i) {
-    const int e = tid + i * kNT;
-    v[i] = (e % NH < kzlive) ? src[row0 * NH + e] : make_float2(0.0f, 0.0f);
-  }
-#pragma unroll
-  for (int i = 0; i < EPZ; ++i) s[lds_addr<true>(tid + i * kNT)] = v[i];
-  __syncthreads();
-  c2r_untwist_fft<N>(s, tw, tid);
-}
-
-__device__ __forceinline__ float lds_real(const float2* s, int e)
-{
-  const float2 v = s[lds_addr<true>(e >> 1)];
-  return (e & 1) ? v.y : v.x;
-}
-
 // aliasing clamps of find_HII_bubbles.c:272-311.  Kinds 0-2 are written as
 // compares and selects with fmaxf/fminf's results for every input, NaN
 // included (fmaxf(NaN, c) = c, and a compare with NaN is false): a max of a
@@ -305,41 +236,38 @@ __device__ __forceinline__ float clamp_kind(float v, int kind)
   }
 }
 
-// Plain C2R z pass: packed rows -> padded real rows, with an optional clamp;
-// slots kz >= kzlive of the input are zero.
+// ------------------------------------------------------------- z: C2R pass
+// Packed rows -> real rows of pitch floats (the padding zeroed), with an
+// optional clamp; slots kz >= kzlive of the input are zero.  ROWS rows per
+// workgroup (row_fft.hpp); blockIdx.y selects the field.
 template <int N>
-__global__ __launch_bounds__(kNT) void k_c2r_z(const float2* __restrict__ in, float* __restrict__ out,
-                                              const float2* __restrict__ twN, long in_fstride, long out_fstride,
-                                              int clamp, int pitch, int kzlive)
+__global__ __launch_bounds__(RowCfg<N>::NT) void k_c2r_z(const float2* __restrict__ in, float* __restrict__ out,
+                                                         const float2* __restrict__ twN, long in_fstride,
+                                                         long out_fstride, int clamp, int pitch, int kzlive)
 {
-  using C = Cfg<N>;
-  constexpr int RZ = C::RZ, ZE = C::ZE;
-  __shared__ float2 s[ZE + ZE / 32];
+  using C = RowCfg<N>;
+  constexpr int NH = C::NH, ROWS = C::ROWS, NT = C::NT, NBL = C::NBL, RL = C::RL;
+  __shared__ float2 s[row_lds<N>(ROWS)];
   __shared__ float2 tw[N];
   const int tid = threadIdx.x;
-  for (int i = tid; i < N; i += kNT) tw[i] = twN[i];
-  const long row0 = (long)blockIdx.x * RZ;
-  c2r_rows_lds<N>(s, tw, in + blockIdx.y * in_fstride, row0, tid, kzlive);
-  float* o = out + blockIdx.y * out_fstride;
-  if (pitch == N) {
-    // unpadded rows: each thread stores groups of 4 cells (two complex slots
-    // of one 32-slot LDS bank row) as one 16-byte write
-    constexpr int Q = N / 4;
-    static_assert((RZ * Q) % kNT == 0, "4-cell groups must split evenly over the threads");
-    float4* o4 = reinterpret_cast<float4*>(o + row0 * N);
+  for (int i = tid; i < N; i += NT) tw[i] = twN[i];
+  __syncthreads();
+  const long row0 = (long)blockIdx.x * ROWS;
+  const float2* src = in + blockIdx.y * in_fstride + row0 * NH;
+  rows_first<N, ROWS>(s, tw, tid, [&](int c, int k) {
+    return (k < kzlive) ? src[c * NH + k] : make_float2(0.0f, 0.0f);
+  });
+  rows_middle<N, ROWS, 1, C::R1>(s, tw, tid);
+  for (int e = tid; e < ROWS * NBL; e += NT) {
+    const int r = e / NBL, j = e % NBL;
+    float2 v[RL];
+    rows_last<N>(s, tw, r, j, v);
+    float* o = out + blockIdx.y * out_fstride + (row0 + r) * pitch;
 #pragma unroll
-    for (int i = 0; i < RZ * Q / kNT; ++i) {
-      const int q = tid + i * kNT;
-      const int c0 = (q / Q) * (N / 2) + 2 * (q % Q);
-      const float2 a = s[lds_addr<true>(c0)], b = s[lds_addr<true>(c0 + 1)];
-      o4[q] = make_float4(clamp_kind(a.x, clamp), clamp_kind(a.y, clamp), clamp_kind(b.x, clamp),
-                          clamp_kind(b.y, clamp));
-    }
-    return;
-  }
-  for (int e = tid; e < RZ * pitch; e += kNT) {
-    const int r = e / pitch, z = e % pitch;
-    o[(row0 + r) * pitch + z] = (z < N) ? clamp_kind(lds_real(s, r * N + z), clamp) : 0.0f;
+    for (int m = 0; m < RL; ++m)
+      *reinterpret_cast<float2*>(o + 2 * (j + m * NBL)) =
+        make_float2(clamp_kind(v[m].x, clamp), clamp_kind(v[m].y, clamp));
+    if (pitch > N && j == 0) *reinterpret_cast<float2*>(o + N) = make_float2(0.0f, 0.0f);
   }
 }
 
@@ -900,34 +828,20 @@ struct StepArgs {
   int kzlive;           // spectrum slots kz >= kzlive are zero (sharp-k)
 };
 
-// One ladder step of _find_HII_bubbles (find_HII_bubbles.c:255-443) for RZ
-// rows: inverse z pass of every field, clamp, then the per-cell test in double
-// exactly as the reference writes it.  Per-cell state between steps is one
-// byte (0xFF = never crossed, else the step of the latest crossing); xH,
-// r_bubble and the J_21 zeros are written once, on the last step, and the
-// first crossing writes J_21 / z_at_ionization / J_21_at_ionization directly.
-// Threads and 4-cell groups of the fused z pass + threshold: all NF fields of
-// RZ rows sit in LDS together and are transformed as NF*RZ pencils, so the
-// fields share every barrier of the transform.
-// Power-of-two grids take 512 complex elements of rows per field (16 KiB of
-// LDS for four fields: measured at 512^3, 512 beats 1024 by 10% and 2048 by
-// 38%, more resident workgroups hiding the transform's barriers); the others
-// keep the z pass's row blocks.
-template <int N>
-struct ThrCfg {
-  static constexpr int NH = N / 2;
-  static constexpr bool P2 = (Cfg<N>::ZE % 1024 == 0) && NH <= 512;
-  // Row blocks longer than kZE elements (2560 for a factor 5 in NH) would take
-  // 80 KiB of LDS for four fields: those grids run one wave per workgroup over
-  // the fewest rows whose elements split into 4-cell groups over 64 threads.
-  static constexpr bool WAVE = !P2 && Cfg<N>::ZE > kZE;
-  static constexpr int RZ = P2 ? 512 / NH : (WAVE ? z_rows_wave(NH) : Cfg<N>::RZ);
-  static constexpr int ZE = RZ * NH;
-  static constexpr int NT = WAVE ? 64 : 256;
-  static constexpr int G = ZE / (2 * NT);  // groups of 4 cells per thread
-  static_assert(ZE % (2 * NT) == 0, "z tile must split into 4-cell groups");
-  static_assert((N * N) % RZ == 0, "threshold workgroups must tile the rows");
+// What differs from step to step of a ladder (device table, one entry per step).
+struct StepDev {
+  double M_mean, R_cubed, kfc, J21c, gamma_pref;  // as in StepArgs
 };
+
+__device__ __forceinline__ void step_load(StepArgs& a, const StepDev* __restrict__ steps)
+{
+  const StepDev& d = steps[a.step];
+  a.M_mean = d.M_mean;
+  a.R_cubed = d.R_cubed;
+  a.kfc = d.kfc;
+  a.J21c = d.J21c;
+  a.gamma_pref = d.gamma_pref;
+}
 
 // The ladder step's test of one cell (find_HII_bubbles.c:313-443).  v: the
 // cell's clamped filtered fields (deltax, stars, weighted_sfr, then x_e when
@@ -1025,147 +939,183 @@ __device__ __forceinline__ uint32_t threshold_cell(const float* v, uint32_t st, 
   return st_new;
 }
 
-// Fields in T: deltax, stars, weighted_sfr, then x_e when XE (NF - REC = 4),
-// then N_rec when REC (inhomogeneous recombinations).
+// The grids of one box that the ladder's test reads and writes.
+struct ThrGrids {
+  const float* __restrict__ deltax_in;
+  uint8_t* __restrict__ state;
+  float* __restrict__ xH;
+  float* __restrict__ r_bubble;
+  float* __restrict__ J21;
+  float* __restrict__ z_in;
+  float* __restrict__ J21_ion;
+  float* __restrict__ Gamma12;
+  const float* __restrict__ Rtab;
+};
+
+// Two neighbouring cells (c0, c0 + 1 of grid row `row`) of one ladder step:
+// threshold_cell on each, and on the last step the output grids and the
+// cells' terms of the four block sums (xH, xH weighted by density, density,
+// J_21).  v: the cells' clamped fields.  Returns the two new state bytes.
 template <int N, int NF, bool REC>
-__device__ __forceinline__ void c2r_threshold_tile(const float2* __restrict__ T, long fstride,
-                                                   const float2* __restrict__ twN,
-                                                   const float* __restrict__ deltax_in,
-                                                   uint8_t* __restrict__ state, float* __restrict__ xH,
-                                                   float* __restrict__ r_bubble, float* __restrict__ J21,
-                                                   float* __restrict__ z_in, float* __restrict__ J21_ion,
-                                                   float* __restrict__ Gamma12, const float* __restrict__ Rtab,
-                                                   double* __restrict__ partials, const StepArgs& a)
+__device__ __forceinline__ uint32_t threshold_pair(const float (&v)[2][NF], uint32_t st_old, long row, int c0,
+                                                   const StepArgs& a, const ThrGrids& g, double (&sum)[4])
 {
 #pragma clang fp contract(off)
-  using TC = ThrCfg<N>;
-  constexpr int NH = TC::NH, RZ = TC::RZ, ZE = TC::ZE, NT = TC::NT, G = TC::G;
-  constexpr bool XE = (NF - (REC ? 1 : 0)) == 4;
-  static_assert(NF - (REC ? 1 : 0) == 3 || NF - (REC ? 1 : 0) == 4, "three or four fields besides N_rec");
-  constexpr int TOT = NF * ZE;  // complex elements of every field's rows
-  constexpr int EPT = TOT / NT;
-  static_assert(TOT % NT == 0, "fields must split evenly over the threads");
-  __shared__ float2 s[TOT + TOT / 32];
-  __shared__ float2 tw[N];
-  __shared__ double red[NT];
-  const int tid = threadIdx.x;
-  const long row0 = (long)blockIdx.x * RZ;
-  // the cells' ladder state, loaded with the spectra (the barriers of the
-  // transform would otherwise leave its latency exposed)
-  uint32_t st_pre[G];
+  const long ir0 = row * N + c0;
+  uint32_t st_new = st_old;
+  float xh2[2], rb2[2], j2[2], ja2[2];
+  bool zc2[2];
 #pragma unroll
-  for (int j = 0; j < G; ++j)
-    st_pre[j] = (a.step == 0) ? 0xFFFFFFFFu
-                              : *reinterpret_cast<const uint32_t*>(state + row0 * N + 4 * (tid + j * NT));
-  {
-    float2 v[EPT];
-#pragma unroll
-    for (int i = 0; i < EPT; ++i) {
-      const int e = tid + i * NT, f = e / ZE, k = e % ZE;
-      v[i] = (k % NH < a.kzlive) ? T[f * fstride + row0 * NH + k] : make_float2(0.0f, 0.0f);
-    }
-    for (int i = tid; i < N; i += NT) tw[i] = twN[i];
-#pragma unroll
-    for (int i = 0; i < EPT; ++i) s[lds_addr<true>(tid + i * NT)] = v[i];
+  for (int e = 0; e < 2; ++e) {
+    xh2[e] = rb2[e] = j2[e] = 0.0f;
+    const uint32_t st = (st_old >> (8 * e)) & 0xFFu;
+    const uint32_t sn = threshold_cell<NF, REC>(v[e], st, ir0 + e, a, g.J21, g.Gamma12, g.Rtab, xh2[e], rb2[e], j2[e],
+                                                zc2[e], ja2[e]);
+    st_new = (st_new & ~(0xFFu << (8 * e))) | (sn << (8 * e));
   }
-  __syncthreads();
-  c2r_untwist_rows<N, NF * RZ, NT>(s, tw, tid);
-  // thread t owns the cell groups 4 * (t + j * NT) + q, q < 4, j < G: four
-  // consecutive cells of one row, so state is one word and the outputs are
-  // 16-byte stores
-  constexpr int CPT = 4 * G;
-  float val[NF][CPT];
+  if (a.last) {
+    *reinterpret_cast<float2*>(g.xH + ir0) = make_float2(xh2[0], xh2[1]);
+    *reinterpret_cast<float2*>(g.r_bubble + ir0) = make_float2(rb2[0], rb2[1]);
+    const float2 dx = *reinterpret_cast<const float2*>(g.deltax_in + row * (N + 2) + c0);
+    const float dx2[2] = {dx.x, dx.y};
+    float2 jv = make_float2(0.f, 0.f);
+    if (a.uvb) jv = *reinterpret_cast<const float2*>(g.J21 + ir0);
+    const float jj[2] = {jv.x, jv.y};
+    float jo[2];
 #pragma unroll
-  for (int f = 0; f < NF; ++f) {
-    // clamps of :272-311: deltax, x_e, the rest (stars, N_rec); the weighted
-    // SFR is clamped in threshold_cell, at its uses
-    const int kind = (f == 0) ? 0 : (f == 2 ? -1 : ((XE && f == 3) ? 2 : 1));
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-      const int h = f * ZE + 2 * (tid + j * NT);  // float2 index of the group's first pair
-      const float2 p0 = s[lds_addr<true>(h)], p1 = s[lds_addr<true>(h + 1)];
-      val[f][4 * j + 0] = clamp_kind(p0.x, kind);
-      val[f][4 * j + 1] = clamp_kind(p0.y, kind);
-      val[f][4 * j + 2] = clamp_kind(p1.x, kind);
-      val[f][4 * j + 3] = clamp_kind(p1.y, kind);
+    for (int e = 0; e < 2; ++e) {
+      const double dm = 1.0 + (double)dx2[e];
+      sum[0] += (double)xh2[e];
+      sum[1] += (double)xh2[e] * dm;
+      sum[2] += dm;
+      jo[e] = (j2[e] != 0.0f) ? jj[e] : 0.0f;
+      if (a.uvb) sum[3] += (double)jo[e];
     }
-  }
-  double s_xH = 0.0, s_xHm = 0.0, s_m = 0.0, s_J = 0.0;
-  const long cell0 = row0 * N;
+    if (a.uvb) *reinterpret_cast<float2*>(g.J21 + ir0) = make_float2(jo[0], jo[1]);
+    if (zc2[0] || zc2[1]) {
+      const float2 zi = *reinterpret_cast<const float2*>(g.z_in + ir0);
+      const float zi2[2] = {zi.x, zi.y};
 #pragma unroll
-  for (int j = 0; j < G; ++j) {
-    const int e0 = 4 * (tid + j * NT);
-    const long ir0 = cell0 + e0;
-    const uint32_t st_old = st_pre[j];
-    uint32_t st_new = st_old;
-    float xh4[4], rb4[4], j4[4];
-    int zcheck4 = 0;
-    float jaux4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int i = 4 * j + q;
-      float v[NF];
-#pragma unroll
-      for (int f = 0; f < NF; ++f) v[f] = val[f][i];
-      float xh = 0.0f, rb = 0.0f, jf = 0.0f, ja = 0.0f;
-      bool zc = false;
-      const uint32_t st = (st_old >> (8 * q)) & 0xFFu;
-      const uint32_t sn = threshold_cell<NF, REC>(v, st, ir0 + q, a, J21, Gamma12, Rtab, xh, rb, jf, zc, ja);
-      st_new = (st_new & ~(0xFFu << (8 * q))) | (sn << (8 * q));
-      if (a.last) {
-        xh4[q] = xh;
-        rb4[q] = rb;
-        j4[q] = jf;
-      }
-      jaux4[q] = ja;
-      zcheck4 |= (zc ? 1 : 0) << q;
-    }
-    if (st_new != st_old || a.step == 0) *reinterpret_cast<uint32_t*>(state + ir0) = st_new;
-    if (a.last) {
-      *reinterpret_cast<float4*>(xH + ir0) = make_float4(xh4[0], xh4[1], xh4[2], xh4[3]);
-      *reinterpret_cast<float4*>(r_bubble + ir0) = make_float4(rb4[0], rb4[1], rb4[2], rb4[3]);
-      const int r = e0 / N, z = e0 % N;
-      const float* dxp = deltax_in + (row0 + r) * (N + 2) + z;
-      const float2 d01 = *reinterpret_cast<const float2*>(dxp);
-      const float2 d23 = *reinterpret_cast<const float2*>(dxp + 2);
-      const float dx4[4] = {d01.x, d01.y, d23.x, d23.y};
-      float4 jv = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (a.uvb) jv = *reinterpret_cast<const float4*>(J21 + ir0);
-      const float jj[4] = {jv.x, jv.y, jv.z, jv.w};
-      float jo[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const double dm = 1.0 + (double)dx4[q];
-        s_xH += (double)xh4[q];
-        s_xHm += (double)xh4[q] * dm;
-        s_m += dm;
-        jo[q] = (j4[q] != 0.0f) ? jj[q] : 0.0f;
-        if (a.uvb) s_J += (double)jo[q];
-      }
-      if (a.uvb) *reinterpret_cast<float4*>(J21 + ir0) = make_float4(jo[0], jo[1], jo[2], jo[3]);
-      if (zcheck4) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const long ir = ir0 + q;
-          if (((zcheck4 >> q) & 1) && z_in[ir] < 0) {
-            z_in[ir] = (float)a.redshift;
-            if (a.uvb) J21_ion[ir] = ((j4[q] != 0.0f) ? jj[q] : jaux4[q]) * (float)a.bias;
-          }
+      for (int e = 0; e < 2; ++e) {
+        if (zc2[e] && zi2[e] < 0) {
+          g.z_in[ir0 + e] = (float)a.redshift;
+          if (a.uvb) g.J21_ion[ir0 + e] = ((j2[e] != 0.0f) ? jj[e] : ja2[e]) * (float)a.bias;
         }
       }
     }
   }
+  return st_new;
+}
+
+// The clamps of :272-311 by field: deltax, x_e, the rest (stars, N_rec); the
+// weighted SFR is clamped in threshold_cell, at its uses.
+template <bool XE>
+__device__ __forceinline__ float clamp_field(float v, int f)
+{
+  return clamp_kind(v, (f == 0) ? 0 : (f == 2 ? -1 : ((XE && f == 3) ? 2 : 1)));
+}
+
+// waves per SIMD the threshold kernels are held to: 128 VGPRs hold three or
+// four fields' last-stage outputs, five take 168
+constexpr int thr_waves(int nf) { return nf == 5 ? 3 : 4; }
+
+// K ladder steps of _find_HII_bubbles (find_HII_bubbles.c:255-443), a.step,
+// a.step + 1 ..., for ROWS rows: inverse z pass of every field (row_fft.hpp),
+// clamp, then the per-cell test in double exactly as the reference writes it.
+// Per-cell state between launches is one byte (0xFF = never crossed, else the
+// step of the latest crossing), held in registers from step to step of a
+// launch; xH, r_bubble and the J_21 zeros are written once, on the last step.
+// Fields in T: deltax, stars, weighted_sfr, then x_e when XE (NF - REC = 4),
+// then N_rec when REC (inhomogeneous recombinations); step k's at T + k
+// kstride.  j21 (or null): the box's own J_21 constants by step.
+template <int N, int NF, bool REC>
+__device__ __forceinline__ void c2r_threshold_rows(const float2* __restrict__ T, long fstride, long kstride, int K,
+                                                   const float2* __restrict__ twN,
+                                                   const StepDev* __restrict__ steps, const double* __restrict__ j21,
+                                                   const ThrGrids& g, double* __restrict__ partials, StepArgs a)
+{
+  using C = RowCfg<N>;
+  constexpr int NH = C::NH, ROWS = C::ROWS, NT = C::NT, NBL = C::NBL, RL = C::RL;
+  constexpr int P = NF * ROWS;
+  constexpr bool XE = (NF - (REC ? 1 : 0)) == 4;
+  static_assert(NF - (REC ? 1 : 0) == 3 || NF - (REC ? 1 : 0) == 4, "three or four fields besides N_rec");
+  __shared__ float2 s[row_lds<N>(P)];
+  __shared__ float2 tw[N];
+  __shared__ double red[4 * NT / 64];
+  int tid = threadIdx.x;
+  const long row0 = (long)blockIdx.x * ROWS;
+  // the cell pairs 2n, 2n + 1 a thread tests: the outputs n = j + m NBL of its
+  // last-stage butterfly (r, j), or pairs tid + m NT of the rows when they
+  // meet in LDS
+  constexpr int PAIRS = C::kViaLds ? ROWS * NH / NT : RL;
+  static_assert(!C::kViaLds || (ROWS * NH) % NT == 0, "pairs must split evenly over the threads");
+  const bool live = C::kViaLds || tid < ROWS * NBL;  // the others help with the transforms only
+  auto pair_row = [](int t, int m) { return C::kViaLds ? (t + m * NT) / NH : t / NBL; };
+  auto pair_n = [](int t, int m) { return C::kViaLds ? (t + m * NT) % NH : t % NBL + m * NBL; };
+  auto pair_state = [&](int t, int m) {
+    return reinterpret_cast<uint16_t*>(g.state + (row0 + pair_row(t, m)) * N + 2 * pair_n(t, m));
+  };
+  uint32_t st_in[PAIRS], st[PAIRS];
+#pragma unroll
+  for (int m = 0; m < PAIRS; ++m) st[m] = st_in[m] = (a.step == 0 || !live) ? 0xFFFFu : *pair_state(tid, m);
+  const bool fresh = a.step == 0;
+  for (int i = tid; i < N; i += NT) tw[i] = twN[i];
+  double sum[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int k = 0; k < K; ++k, ++a.step) {
+    step_load(a, steps);
+    if (j21) a.J21c = j21[a.step];
+    // the LDS addresses are formed anew in every step: kept over the loop they
+    // take the registers of a whole wave per SIMD (116 -> 190 at N = 320)
+    asm volatile("" : "+v"(tid));
+    __syncthreads();  // the twiddle table; the last step's reads of s
+    const float2* Tk = T + k * kstride + row0 * NH;
+    rows_first<N, P>(s, tw, tid, [&](int c, int n) {
+      const int f = c / ROWS, rr = c % ROWS;
+      return (n < a.kzlive) ? Tk[f * fstride + rr * NH + n] : make_float2(0.0f, 0.0f);
+    });
+    rows_middle<N, P, 1, C::R1>(s, tw, tid);
+    auto test = [&](int m, const float2 (&v)[NF]) {
+      float c[2][NF];
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+        c[0][f] = clamp_field<XE>(v[f].x, f);
+        c[1][f] = clamp_field<XE>(v[f].y, f);
+      }
+      st[m] = threshold_pair<N, NF, REC>(c, st[m], row0 + pair_row(tid, m), 2 * pair_n(tid, m), a, g, sum);
+    };
+    if constexpr (C::kViaLds) {
+      rows_last_lds<N, P>(s, tw, tid);
+#pragma unroll
+      for (int m = 0; m < PAIRS; ++m) {
+        float2 v[NF];
+#pragma unroll
+        for (int f = 0; f < NF; ++f) v[f] = s[lds_addr<true>((f * ROWS + pair_row(tid, m)) * NH + pair_n(tid, m))];
+        test(m, v);
+      }
+    } else if (live) {
+      float2 o[NF][RL];
+#pragma unroll
+      for (int f = 0; f < NF; ++f) rows_last<N>(s, tw, f * ROWS + tid / NBL, tid % NBL, o[f]);
+#pragma unroll
+      for (int m = 0; m < PAIRS; ++m) {
+        float2 v[NF];
+#pragma unroll
+        for (int f = 0; f < NF; ++f) v[f] = o[f][m];
+        test(m, v);
+      }
+    }
+  }
+  if (live) {
+#pragma unroll
+    for (int m = 0; m < PAIRS; ++m)
+      if (fresh || st[m] != st_in[m]) *pair_state(tid, m) = (uint16_t)st[m];
+  }
   if (a.last) {
-    double* p = partials + (long)blockIdx.x * 4;
-    double v0 = block_sum<NT>(s_xH, red);
-    double v1 = block_sum<NT>(s_xHm, red);
-    double v2 = block_sum<NT>(s_m, red);
-    double v3 = block_sum<NT>(s_J, red);
+    block_sum_n<NT, 4>(sum, red);
     if (tid == 0) {
-      p[0] = v0;
-      p[1] = v1;
-      p[2] = v2;
-      p[3] = v3;
+      double* p = partials + (long)blockIdx.x * 4;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) p[q] = sum[q];
     }
   }
 }
@@ -1182,7 +1132,8 @@ __device__ __forceinline__ void c2r_threshold_tile(const float2* __restrict__ T,
 // (g, t) tests the cells of n = t + A j, j in [4g, 4g + 4).  Three barriers
 // per workgroup and two LDS round trips, where staging the rows in LDS for a
 // Stockham transform takes eight and five.  Per cell the test is
-// threshold_cell's, as in c2r_threshold_tile.
+// threshold_cell's, as in c2r_threshold_rows, one step per launch (a loop over
+// two steps spilled at four waves per SIMD: 541 -> 560 us per step at 512^3).
 // Inverse real transform (C2R) of packed rows of NH = 16 A complex held by A
 // lanes each: lane t = lane mod A holds points t + A m of its row in x[m] (m <
 // 16), and gets z[j] = point t + A j of the row's complex output (real cells
@@ -1190,7 +1141,7 @@ __device__ __forceinline__ void c2r_threshold_tile(const float2* __restrict__ T,
 // lane (A - t) mod A holds (a lane shuffle); then a 16-point DFT of the lane's
 // registers, the twiddle exp(+2 pi i t k1 / NH), one exchange through the
 // row's LDS rows xr (16 x A, pitch A + 1) and A-point DFTs over the lanes.
-// The untwist is c2r_untwist_rows's; tw is the N-entry table exp(-2 pi i j /
+// The untwist is row_fft.hpp's; tw is the N-entry table exp(-2 pi i j /
 // N) in LDS.  Every thread of the workgroup calls it (one barrier inside).
 template <int A>
 __device__ __forceinline__ void row_c2r_reg(const float2 (&x)[16], float2 (&z)[16], const float2* tw, float2* xr,
@@ -1280,134 +1231,79 @@ struct RegThr {
 template <int A, int NF>
 __global__ __launch_bounds__(256) void k_c2r_threshold_reg(const float2* __restrict__ T, long fstride,
                                                            const float2* __restrict__ twN,
-                                                           const float* __restrict__ deltax_in,
-                                                           uint8_t* __restrict__ state, float* __restrict__ xH,
-                                                           float* __restrict__ r_bubble, float* __restrict__ J21,
-                                                           float* __restrict__ z_in, float* __restrict__ J21_ion,
-                                                           const float* __restrict__ Rtab,
+                                                           const StepDev* __restrict__ steps, ThrGrids g,
                                                            double* __restrict__ partials, StepArgs a)
 {
-#pragma clang fp contract(off)
   using C = RegThr<A>;
   constexpr int NH = C::NH, N = C::N, RW = C::RW, RWG = C::RWG, XP = C::XP;
   static_assert(NF == 3 || NF == 4, "three or four fields");
   constexpr bool XE = NF == 4;
   __shared__ float2 tw[N];
   __shared__ float2 xb[RWG][4][16 * XP];  // [row of the workgroup][field group][16 x A, pitch XP]
-  __shared__ double red[256];
+  __shared__ double red[4 * 256 / 64];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int t = lane % A, g = (lane / A) % 4;
+  const int t = lane % A, fg = (lane / A) % 4;
   const int rl = (tid >> 6) * RW + lane / (4 * A);  // row within the workgroup
   const long row = (long)blockIdx.x * RWG + rl;     // x N + y
+  step_load(a, steps);
   for (int i = tid; i < N; i += 256) tw[i] = twN[i];
-  // the ladder state of this lane's cells, two bytes at cell 2n, n = t + A (4g + q)
+  // the ladder state of this lane's cells, two bytes at cell 2n, n = t + A (4 fg + q)
   uint32_t st_pre[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q)
     st_pre[q] = (a.step == 0) ? 0xFFFFu
-                              : *reinterpret_cast<const uint16_t*>(state + row * N + 2 * (t + A * (4 * g + q)));
-  // field g's row; the fourth group carries zeros when there are three fields
+                              : *reinterpret_cast<const uint16_t*>(g.state + row * N + 2 * (t + A * (4 * fg + q)));
+  // field fg's row; the fourth group carries zeros when there are three fields
   float2 x[16];
   {
-    const float2* src = T + (long)(g < NF ? g : 0) * fstride + row * NH + t;
+    const float2* src = T + (long)(fg < NF ? fg : 0) * fstride + row * NH + t;
 #pragma unroll
     for (int m = 0; m < 16; ++m)
-      x[m] = (g < NF && t + A * m < a.kzlive) ? src[A * m] : make_float2(0.0f, 0.0f);
+      x[m] = (fg < NF && t + A * m < a.kzlive) ? src[A * m] : make_float2(0.0f, 0.0f);
   }
   __syncthreads();  // the twiddle table
-  float2* xr = xb[rl][g];
+  float2* xr = xb[rl][fg];
   float2 z[16];
   row_c2r_reg<A>(x, z, tw, xr, lane);
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < 16; ++j) xr[j * XP + t] = z[j];
   __syncthreads();
-  // the cells n = t + A j, j = 4g + q: all fields of the row from LDS
-  double s_xH = 0.0, s_xHm = 0.0, s_m = 0.0, s_J = 0.0;
-  const long cell0 = row * N;
+  // the cells n = t + A j, j = 4 fg + q: all fields of the row from LDS
+  double sum[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const int j = 4 * g + q;
+    const int j = 4 * fg + q;
     const int c0 = 2 * (t + A * j);  // first of the two cells
-    float v[2][NF];
+    float c[2][NF];
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
-      // clamps of :272-311; the weighted SFR's is threshold_cell's
-      const int kind = (f == 0) ? 0 : (f == 2 ? -1 : ((XE && f == 3) ? 2 : 1));
       const float2 p = xb[rl][f][j * XP + t];
-      v[0][f] = clamp_kind(p.x, kind);
-      v[1][f] = clamp_kind(p.y, kind);
+      c[0][f] = clamp_field<XE>(p.x, f);
+      c[1][f] = clamp_field<XE>(p.y, f);
     }
-    const uint32_t st_old = st_pre[q];
-    uint32_t st_new = st_old;
-    float xh2[2], rb2[2], j2[2], ja2[2];
-    bool zc2[2];
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      xh2[e] = rb2[e] = j2[e] = 0.0f;
-      const uint32_t st = (st_old >> (8 * e)) & 0xFFu;
-      const uint32_t sn = threshold_cell<NF, false>(v[e], st, cell0 + c0 + e, a, J21, nullptr, Rtab, xh2[e], rb2[e],
-                                                    j2[e], zc2[e], ja2[e]);
-      st_new = (st_new & ~(0xFFu << (8 * e))) | (sn << (8 * e));
-    }
-    const long ir0 = cell0 + c0;
-    if (st_new != st_old || a.step == 0) *reinterpret_cast<uint16_t*>(state + ir0) = (uint16_t)st_new;
-    if (a.last) {
-      *reinterpret_cast<float2*>(xH + ir0) = make_float2(xh2[0], xh2[1]);
-      *reinterpret_cast<float2*>(r_bubble + ir0) = make_float2(rb2[0], rb2[1]);
-      const float2 dx = *reinterpret_cast<const float2*>(deltax_in + row * (N + 2) + c0);
-      const float dx2[2] = {dx.x, dx.y};
-      float2 jv = make_float2(0.f, 0.f);
-      if (a.uvb) jv = *reinterpret_cast<const float2*>(J21 + ir0);
-      const float jj[2] = {jv.x, jv.y};
-      float jo[2];
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const double dm = 1.0 + (double)dx2[e];
-        s_xH += (double)xh2[e];
-        s_xHm += (double)xh2[e] * dm;
-        s_m += dm;
-        jo[e] = (j2[e] != 0.0f) ? jj[e] : 0.0f;
-        if (a.uvb) s_J += (double)jo[e];
-      }
-      if (a.uvb) *reinterpret_cast<float2*>(J21 + ir0) = make_float2(jo[0], jo[1]);
-      if (zc2[0] || zc2[1]) {
-        const float2 zi = *reinterpret_cast<const float2*>(z_in + ir0);
-        const float zi2[2] = {zi.x, zi.y};
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          if (zc2[e] && zi2[e] < 0) {
-            z_in[ir0 + e] = (float)a.redshift;
-            if (a.uvb) J21_ion[ir0 + e] = ((j2[e] != 0.0f) ? jj[e] : ja2[e]) * (float)a.bias;
-          }
-        }
-      }
-    }
+    const uint32_t st = threshold_pair<N, NF, false>(c, st_pre[q], row, c0, a, g, sum);
+    if (st != st_pre[q] || a.step == 0) *reinterpret_cast<uint16_t*>(g.state + row * N + c0) = (uint16_t)st;
   }
   if (a.last) {
-    double v[4] = {s_xH, s_xHm, s_m, s_J};
-    block_sum_n<256, 4>(v, red);
+    block_sum_n<256, 4>(sum, red);
     if (tid == 0) {
       double* p = partials + (long)blockIdx.x * 4;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) p[k] = v[k];
+      for (int q = 0; q < 4; ++q) p[q] = sum[q];
     }
   }
 }
 
 template <int N, int NF, bool REC = false>
-__global__ __launch_bounds__(ThrCfg<N>::NT) void k_c2r_threshold(const float2* __restrict__ T, long fstride,
-                                                      const float2* __restrict__ twN,
-                                                      const float* __restrict__ deltax_in,
-                                                      uint8_t* __restrict__ state, float* __restrict__ xH,
-                                                      float* __restrict__ r_bubble, float* __restrict__ J21,
-                                                      float* __restrict__ z_in, float* __restrict__ J21_ion,
-                                                      float* __restrict__ Gamma12, const float* __restrict__ Rtab,
-                                                      double* __restrict__ partials, StepArgs a)
+__global__ __launch_bounds__(RowCfg<N>::NT, thr_waves(NF)) void k_c2r_threshold(const float2* __restrict__ T, long fstride,
+                                                                 long kstride, int K,
+                                                                 const float2* __restrict__ twN,
+                                                                 const StepDev* __restrict__ steps, ThrGrids g,
+                                                                 double* __restrict__ partials, StepArgs a)
 {
-  c2r_threshold_tile<N, NF, REC>(T, fstride, twN, deltax_in, state, xH, r_bubble, J21, z_in, J21_ion, Gamma12, Rtab,
-                                 partials, a);
+  c2r_threshold_rows<N, NF, REC>(T, fstride, kstride, K, twN, steps, nullptr, g, partials, a);
 }
 
 // Per-box grids and scalars of a batch (device array, one entry per box).
@@ -1427,22 +1323,20 @@ struct BoxDev {
 // nfield spectra per box (box stride bstride); state and partials are
 // contiguous per box; J21c_tab[box * nstep + step] is the box's J_21 constant.
 template <int N, int NF>
-__global__ __launch_bounds__(ThrCfg<N>::NT) void k_c2r_threshold_batch(const float2* __restrict__ T, long fstride, long bstride,
-                                                            const float2* __restrict__ twN,
-                                                            const BoxDev* __restrict__ boxes,
-                                                            uint8_t* __restrict__ state,
-                                                            const float* __restrict__ Rtab,
-                                                            const double* __restrict__ J21c_tab, int nstep,
-                                                            double* __restrict__ partials, StepArgs a)
+__global__ __launch_bounds__(RowCfg<N>::NT, thr_waves(NF)) void k_c2r_threshold_batch(
+  const float2* __restrict__ T, long fstride, long bstride, const float2* __restrict__ twN,
+  const BoxDev* __restrict__ boxes, uint8_t* __restrict__ state, const float* __restrict__ Rtab,
+  const StepDev* __restrict__ steps, const double* __restrict__ J21c_tab, int nstep, double* __restrict__ partials,
+  StepArgs a)
 {
   const int box = blockIdx.y;
   const BoxDev bx = boxes[box];
   a.eff = bx.eff;
   a.redshift = bx.redshift;
   a.bias = bx.bias;
-  a.J21c = J21c_tab[(long)box * nstep + a.step];
-  c2r_threshold_tile<N, NF, false>(T + box * bstride, fstride, twN, bx.deltax, state + (long)box * N * N * N, bx.xH,
-                                   bx.r_bubble, bx.J21, bx.z_in, bx.J21_ion, nullptr, Rtab,
+  const ThrGrids g{bx.deltax, state + (long)box * N * N * N, bx.xH, bx.r_bubble, bx.J21, bx.z_in, bx.J21_ion, nullptr,
+                   Rtab};
+  c2r_threshold_rows<N, NF, false>(T + box * bstride, fstride, 0, 1, twN, steps, J21c_tab + (long)box * nstep, g,
                                    partials + (long)box * gridDim.x * 4, a);
 }
 
