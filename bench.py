@@ -56,8 +56,10 @@ def kernel_bytes(name, N, F, radii=1.0):
 
     Names with a ts_ prefix are launches of the spin-temperature shell loop,
     one field each; the others are the bubble finder's, F fields each.
-    ``radii`` is the average number of ladder radii one ix_filter_k launch
-    covers (it reads each field's spectrum once and writes one per radius).
+    ``radii`` is the average number of ladder radii one launch of this kernel
+    covers (ladder_radii): ix_filter_k reads each field's spectrum once and
+    writes one per radius, the y pass reads and writes each radius's, and the
+    threshold pass reads each radius's and one byte of state per cell once.
     """
     if name.startswith("ts_"):
         name, F = name[3:], 1
@@ -73,20 +75,29 @@ def kernel_bytes(name, N, F, radii=1.0):
     Nr = N**3
     table = {
         # strided pencil passes: read + write one spectrum per field
-        "colpass_y_inv": 2 * F * spec,
-        "colpass_y_fwd": 2 * spec,  # forward passes run one field per launch
+        "colpass_y_inv": 2 * F * spec * radii,
+        "colpass_y_fwd": 2 * F * spec,
         "ts_cell": 40 * 4 * Nr + 4 * N * N * (N + 2) * 3 + 3 * 4 * Nr,
-        "colpass_x_fwd": 2 * spec,
+        "colpass_x_fwd": 2 * F * spec,
         # window + inverse x pass: read unfiltered (+ Nyquist plane) and write per field
         "ix_filter": F * (2 * spec + 8 * N * N),
         "ix_filter_k": F * ((1 + radii) * spec + 8 * N * N),
         # inverse z pass + threshold: read each field's spectrum, 1 byte of step state per cell
-        "c2r_threshold": F * spec + 2 * Nr,
-        "r2c_z": 4 * N * N * (N + 2) + spec,
+        "c2r_threshold": F * spec * radii + 2 * Nr,
+        "r2c_z": F * (4 * N * N * (N + 2) + spec),
         "window_table": 4 * (N // 2 + 1) ** 3,
         "brightness_temp": 4 * N * N * (N + 2) + 2 * 4 * Nr,
     }
     return table.get(name)
+
+
+def ladder_radii(name, S, prof, steps):
+    """Ladder radii per launch of a kernel, from the launches of a profiled run:
+    the S - 1 filtered radii over ix_filter_k's, all S over the y and threshold passes'."""
+    n = prof.get(name, (0, 0))[1] / steps
+    if not n or name not in ("ix_filter_k", "colpass_y_inv", "c2r_threshold"):
+        return 1.0
+    return (S - 1 if name == "ix_filter_k" else S) / n
 
 
 def path_bytes_hii(N, F, S):
@@ -95,7 +106,7 @@ def path_bytes_hii(N, F, S):
     pass, the inverse y pass and the z pass + threshold; the window tables
     (shared by the boxes of a batch cohort) are left out."""
     spec = 8 * N * N * (N // 2)
-    fwd = F * (kernel_bytes("r2c_z", N, F) + 2 * 2 * spec)
+    fwd = kernel_bytes("r2c_z", N, F) + F * 2 * 2 * spec
     per_radius = kernel_bytes("ix_filter", N, F) + kernel_bytes("colpass_y_inv", N, F) + kernel_bytes(
         "c2r_threshold", N, F)
     return fwd + S * per_radius
@@ -750,16 +761,14 @@ def main():
     dom = max(prof.items(), key=lambda kv: kv[1][0])
     name, (ms_tot, cnt) = dom
     avg_s = ms_tot / cnt / 1e3
-    # radii per multi-radius x pass: the S - 1 filtered radii over its launches
-    nk = prof.get("ix_filter_k", (0, 0))[1] // args.steps
-    radii = (S - 1) / nk if nk else 1.0
-    b = kernel_bytes(name, N, F, radii)
+    kbytes = lambda k: kernel_bytes(k, N, F, ladder_radii(k, S, prof, args.steps))  # noqa: E731
+    b = kbytes(name)
     roof = {"kernel": name, "bound": "hbm", "achieved": (b / avg_s / 1e9) if b else None, "peak": HBM_PEAK / 1e9,
             "unit": "GB/s", "frac": (b / avg_s / HBM_PEAK) if b else None, "traffic": measured_traffic(name, N),
             "avg_launch_us": avg_s * 1e6, "bytes_per_launch": b}
     per_kernel = {}
     for k, (ms, n) in prof.items():
-        kb = kernel_bytes(k, N, F, radii)
+        kb = kbytes(k)
         per_kernel[k] = {"ms_per_step": ms / args.steps, "launches_per_step": n // args.steps,
                          "us_per_launch": ms / n * 1e3,
                          "GB_s": (kb * n / (ms / 1e3) / 1e9) if kb else None,
@@ -807,8 +816,8 @@ def main():
     }
     # the path at the kernels' own algorithmic bytes: every launch whose bytes are
     # known (the sharp-k shells' pruned passes are not counted) over the step time
-    known = sum((kernel_bytes(k, N, F, radii) or 0) * n for k, (ms, n) in prof.items()) / args.steps
-    known_ms = sum(ms for k, (ms, n) in prof.items() if kernel_bytes(k, N, F, radii)) / args.steps
+    known = sum((kbytes(k) or 0) * n for k, (ms, n) in prof.items()) / args.steps
+    known_ms = sum(ms for k, (ms, n) in prof.items() if kbytes(k)) / args.steps
     out["path_kernel_bytes"] = {
         "bytes_per_step": known, "frac_of_peak": known / dt / HBM_PEAK,
         "device_ms_of_those_kernels": known_ms, "frac_of_peak_over_their_device_time": known / (known_ms / 1e3) / HBM_PEAK,

@@ -165,7 +165,9 @@ struct BatchPipe {
       const bool win = (w != nullptr);
       if (win) {  // the table layout follows the tile width
         const long nt = (long)(NH + 1) * (NH + 1) * (NH + 1);
-        k_window_table<N, TW><<<window_table_blocks<N, TW>(), kNT, 0, c->stream>>>(c->wtab, *w);
+        WinRadii r;
+        r.R[0] = w->R;
+        k_window_table<N, TW><<<window_table_blocks<N, TW>(), kNT, 0, c->stream>>>(c->wtab, *w, r);
         MRX_TRY(check_launch(ctx, "k_window_table (batch)"));
       }
       const dim3 gx(N * M::NKZB, c->nbox);

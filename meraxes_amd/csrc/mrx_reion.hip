@@ -72,13 +72,20 @@ double* resolve_scratch(int device)
 }
 }  // namespace
 
-// Radii per inverse x pass of the bubble ladder (1..kLadderRadiiMax); the
-// MRX_LADDER_RADII environment variable, read when a context is created,
-// overrides it.  Two radii per pass bring the x pass to the y pass's rate at
-// 512^3 (more gain nothing); the second radius's spectra cost nfield
-// N^2 (N/2) float2 of device memory.
-constexpr int kLadderRadii = 2;
-constexpr int kLadderRadiiMax = 8;
+// Radii per group of passes of the bubble ladder (one x pass, one y pass and
+// one threshold pass cover a group).  The MRX_LADDER_RADII environment
+// variable (1..kLadderRadiiMax), read when a context is created, sets it;
+// otherwise it is as many as keep the group's spectra within kLadderBytes, two
+// at least.  Two bring the x pass to the y pass's rate at 512^3 (more gain
+// nothing there).  On small grids a pass over one radius is a few microseconds
+// of work behind a launch of the same length: 64^3 with three fields runs all
+// 37 filtered radii in one group (711 -> 315 us per call; 373 with 8 per
+// group).  The bound keeps a group's spectra in the 256 MB Infinity Cache from
+// pass to pass: 128^3 with four fields takes 1553, 1440, 1485, 1588 and 1684
+// us with 2, 4, 6, 8 and 12 radii per group; from 160^3 up the number matters
+// by less than 3 %.
+constexpr int kLadderRadiiMax = 64;
+constexpr size_t kLadderBytes = (size_t)128 << 20;
 
 struct mrx_ctx {
   int device = 0;
@@ -130,9 +137,9 @@ struct mrx_ctx {
   size_t wtab_all_cap = 0;
   hipStream_t side = nullptr;
   hipEvent_t side_ev[2] = {nullptr, nullptr};
-  // the bubble ladder's inverse x pass covers ladder_radii radii per launch
-  // (tabulated windows): their x-pass outputs, ladder_radii x nfield spectra
-  int ladder_radii = kLadderRadii;
+  // the bubble ladder's passes cover a group of radii per launch (tabulated
+  // windows): the group's x-pass outputs, radii x nfield spectra in TK
+  int ladder_radii = 0;  // radii per group; 0: chosen by size (kLadderBytes)
   float2* TK = nullptr;
   size_t TK_cap = 0;  // float2
   float ts_h_xe0 = 0.f, ts_h_T0 = 0.f;  // RECFAST x_e, T_K of the homogeneous branch
@@ -455,14 +462,20 @@ struct Pipe {
   }
 
   // padded real fields -> unfiltered packed spectra U (scaled by 1/N^3 when
-  // `scale`), Nyquist planes split into V.
-  static int forward(mrx_ctx* ctx, const float* in, long in_fstride, int nfield, bool scale, float2* U, float2* V,
+  // `scale`), Nyquist planes split into V; one launch per pass for all fields.
+  static int forward(mrx_ctx* ctx, const float* in, bool scale, float2* U, float2* V, bool float_scale = false)
+  {
+    FieldTab t{};
+    t.p[0] = in;
+    return forward(ctx, t, 1, scale, U, V, float_scale);
+  }
+  static int forward(mrx_ctx* ctx, const FieldTab& in, int nfield, bool scale, float2* U, float2* V,
                      bool float_scale = false)
   {
     const dim3 gz(N * N / Cfg<N>::RZ, nfield);
     {
     PROF("r2c_z");
-    k_r2c_z<N><<<gz, kNT, 0, ctx->stream>>>(in, U, ctx->tw, in_fstride, nc);
+    k_r2c_z<N><<<gz, kNT, 0, ctx->stream>>>(in, U, ctx->tw, nc);
     }
     MRX_TRY(check_launch(ctx, "k_r2c_z"));
     const dim3 gc(N * (NH / Cfg<N>::TW), nfield);
@@ -498,7 +511,9 @@ struct Pipe {
     const int nkzb = std::min(NH / TW, nmax / TW + 1);
     {
       PROF("r2c_z");
-      k_r2c_z<N><<<dim3(N * N / Cfg<N>::RZ, 1), kNT, 0, ctx->stream>>>(in, U, ctx->tw, 0, nc);
+      FieldTab t{};
+      t.p[0] = in;
+      k_r2c_z<N><<<dim3(N * N / Cfg<N>::RZ, 1), kNT, 0, ctx->stream>>>(t, U, ctx->tw, nc);
     }
     MRX_TRY(check_launch(ctx, "k_r2c_z"));
     {
@@ -552,11 +567,7 @@ struct Pipe {
     if (w.apply) {
       const long nt = (long)(NH + 1) * (NH + 1) * (NH + 1);
       MRX_TRY(ensure_buf(ctx, ctx->wtab, ctx->wtab_cap, (size_t)nt));
-      {
-        PROF("window_table");
-        k_window_table<N, Cfg<N>::TW><<<window_table_blocks<N, Cfg<N>::TW>(), kNT, 0, ctx->stream>>>(ctx->wtab, w);
-      }
-      MRX_TRY(check_launch(ctx, "k_window_table"));
+      MRX_TRY(window_tables(ctx, ctx->wtab, &w, 1));
       Wt = ctx->wtab;
     }
     const dim3 gc(N * (NH / Cfg<N>::TW), 1);
@@ -577,8 +588,8 @@ struct Pipe {
 
   // The inverse x and y passes of K ladder radii with tabulated windows ws[k]
   // (not sharp-k): one x pass reads U once and writes the K spectra TK + k
-  // tstride, then each radius's y pass runs in place.  Per radius the spectra
-  // are inverse_xy's.
+  // tstride, then one y pass runs in place over them all.  Per radius the
+  // spectra are inverse_xy's.
   // wpre: the K radii's window tables already built (window_tables), or null
   static int inverse_xy_k(mrx_ctx* ctx, const float2* U, const float2* V, float2* TK, long tstride, int nfield,
                           const WinArgs* ws, int K, const float* wpre = nullptr)
@@ -597,10 +608,8 @@ struct Pipe {
         U, V, TK, ctx->tw, wt, nt, nc, (long)N * N, tstride, nfield, K);
     }
     MRX_TRY(check_launch(ctx, "k_ix_filter_k"));
-    for (int k = 0; k < K; ++k) {
-      PROF("colpass_y_inv");
-      colpass_y<true>(ctx, TK + k * tstride, nfield, 0.0);
-    }
+    PROF("colpass_y_inv");
+    colpass_y<true>(ctx, TK, K * nfield, 0.0);  // the group's spectra lie back to back (tstride = nfield nc)
     return check_launch(ctx, "k_colpass y inv");
   }
 
@@ -610,9 +619,12 @@ struct Pipe {
   {
     constexpr int TW = Cfg<N>::TW;
     const long nt = (long)(NH + 1) * (NH + 1) * (NH + 1);
-    for (int k = 0; k < K; ++k) {
+    for (int k0 = 0; k0 < K; k0 += kWinRadii) {
+      const int n = std::min(kWinRadii, K - k0);
+      WinRadii r;
+      for (int k = 0; k < n; ++k) r.R[k] = ws[k0 + k].R;
       PROF("window_table");
-      k_window_table<N, TW><<<window_table_blocks<N, TW>(), kNT, 0, ctx->stream>>>(Wt + k * nt, ws[k]);
+      k_window_table<N, TW><<<dim3(window_table_blocks<N, TW>(), n), kNT, 0, ctx->stream>>>(Wt + k0 * nt, ws[0], r);
     }
     return check_launch(ctx, "k_window_table");
   }
@@ -861,7 +873,6 @@ struct HiiRun {
 
       // inputs: deltax, stars, weighted_sfr, x_e are padded and laid out at a
       // fixed stride when staged; device pointers are used where they lie.
-      const long fs = (long)npad(N);
       const float* deltax = in[0];
       const float* src[5] = {in[0], in[1], in[2], p->include_spin_temp ? in[3] : in[4], in[4]};
       const double box_size = p->box_size;
@@ -871,26 +882,34 @@ struct HiiRun {
       // (up to 4 GiB of tables; beyond that each x pass builds its own)
       const long nt = (long)(N / 2 + 1) * (N / 2 + 1) * (N / 2 + 1);
       const float* wpre = nullptr;
-      if (p->filter_type != MRX_FILTER_SHARPK && ctx->ladder_radii >= 1 && S > 1 &&
+      bool use_side = false;
+      if (p->filter_type != MRX_FILTER_SHARPK && S > 1 &&
           (size_t)nt * (S - 1) * sizeof(float) <= ((size_t)4 << 30) &&
           ensure_buf(ctx, ctx->wtab_all, ctx->wtab_all_cap, (size_t)nt * (S - 1)) == MRX_OK) {
-        if (!ctx->side) HIP_TRY(hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking));
-        for (auto& e : ctx->side_ev)
-          if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         std::vector<WinArgs> ws(S - 1);
         for (int k = 0; k < S - 1; ++k) ws[k] = win_args(box_size, (float)R[k], p->filter_type, 1);
-        HIP_TRY(hipEventRecord(ctx->side_ev[0], ctx->stream));
-        HIP_TRY(hipStreamWaitEvent(ctx->side, ctx->side_ev[0], 0));
-        hipStream_t const main_stream = ctx->stream;
-        ctx->stream = ctx->side;
-        const int rc = P::window_tables(ctx, ctx->wtab_all, ws.data(), S - 1);
-        ctx->stream = main_stream;
-        const hipError_t er = (rc == MRX_OK) ? hipEventRecord(ctx->side_ev[1], ctx->side) : hipSuccess;
-        if (rc != MRX_OK || er != hipSuccess) {
-          // the tables already launched finish before the buffer can be reused
-          (void)hipStreamSynchronize(ctx->side);
-          if (rc != MRX_OK) return rc;
-          return set_err(ctx, MRX_EDEVICE, "hipEventRecord (window tables) failed: %s", hipGetErrorString(er));
+        // below 128^3 the tables are a few microseconds of one launch, less
+        // than the two events that order a side stream
+        use_side = N >= 128;
+        if (!use_side) {
+          MRX_TRY(P::window_tables(ctx, ctx->wtab_all, ws.data(), S - 1));
+        } else {
+          if (!ctx->side) HIP_TRY(hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking));
+          for (auto& e : ctx->side_ev)
+            if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+          HIP_TRY(hipEventRecord(ctx->side_ev[0], ctx->stream));
+          HIP_TRY(hipStreamWaitEvent(ctx->side, ctx->side_ev[0], 0));
+          hipStream_t const main_stream = ctx->stream;
+          ctx->stream = ctx->side;
+          const int rc = P::window_tables(ctx, ctx->wtab_all, ws.data(), S - 1);
+          ctx->stream = main_stream;
+          const hipError_t er = (rc == MRX_OK) ? hipEventRecord(ctx->side_ev[1], ctx->side) : hipSuccess;
+          if (rc != MRX_OK || er != hipSuccess) {
+            // the tables already launched finish before the buffer can be reused
+            (void)hipStreamSynchronize(ctx->side);
+            if (rc != MRX_OK) return rc;
+            return set_err(ctx, MRX_EDEVICE, "hipEventRecord (window tables) failed: %s", hipGetErrorString(er));
+          }
         }
         wpre = ctx->wtab_all;
       }
@@ -903,16 +922,15 @@ struct HiiRun {
         {
           if (on) (void)hipStreamWaitEvent(c->stream, c->side_ev[1], 0);
         }
-      } wait_side{ctx, wpre != nullptr};
-      for (int f = 0; f < nfield; ++f) {
-        // forward transform of each field into its U slot
-        MRX_TRY(P::forward(ctx, src[f], 0, 1, true, ctx->U + (long)f * P::nc, ctx->V + (long)f * N * N));
-      }
-      if (wpre) {
+      } wait_side{ctx, use_side};
+      // forward transform of every field into its U slot
+      FieldTab ft{};
+      for (int f = 0; f < nfield; ++f) ft.p[f] = src[f];
+      MRX_TRY(P::forward(ctx, ft, nfield, true, ctx->U, ctx->V));
+      if (use_side) {
         HIP_TRY(hipStreamWaitEvent(ctx->stream, ctx->side_ev[1], 0));
         wait_side.on = false;
       }
-      (void)fs;
       const double pixel_volume = pow(box_size / (double)N, 3);
       StepArgs a;
       memset(&a, 0, sizeof a);
@@ -923,11 +941,16 @@ struct HiiRun {
       a.uvb = p->uvb_flag;
       a.use_xe = p->include_spin_temp;
       a.nfield = nfield;
-      // the filtered radii go through the x pass ladder_radii at a time
-      // (tabulated windows; KL = 0: sharp-k, one radius per pass over its live
-      // tiles) when the spectra of that many radii fit, else one at a time
-      int KL = (p->filter_type == MRX_FILTER_SHARPK) ? 0 : ctx->ladder_radii;
+      // the filtered radii go through the passes KL at a time (tabulated
+      // windows; KL = 0: sharp-k, one radius per pass over its live tiles)
+      // when the spectra of that many radii fit, else one at a time
       const long tstride = (long)nfield * P::nc;
+      int KL = 0;
+      if (p->filter_type != MRX_FILTER_SHARPK) {
+        KL = ctx->ladder_radii ? ctx->ladder_radii
+                               : (int)std::max<size_t>(2, kLadderBytes / (sizeof(float2) * (size_t)tstride));
+        KL = std::max(1, std::min(KL, S - 1));
+      }
       if (KL > 1 && ensure_tk(ctx, (size_t)KL * tstride) != MRX_OK) KL = 1;
       for (int s = 0; s < S;) {
         const bool last = (s == S - 1);
@@ -935,10 +958,10 @@ struct HiiRun {
         const float2* Tsrc = ctx->T;
         if (!last && KL >= 1) {
           K = std::min(KL, S - 1 - s);
-          WinArgs ws[kLadderRadiiMax];
-          for (int k = 0; k < K; ++k) ws[k] = win_args(box_size, (float)R[s + k], p->filter_type, 1);
+          std::vector<WinArgs> ws(wpre ? 0 : K);
+          for (int k = 0; k < (int)ws.size(); ++k) ws[k] = win_args(box_size, (float)R[s + k], p->filter_type, 1);
           float2* TK = KL > 1 ? ctx->TK : ctx->T;
-          MRX_TRY(P::inverse_xy_k(ctx, ctx->U, ctx->V, TK, tstride, nfield, ws, K, wpre ? wpre + s * nt : nullptr));
+          MRX_TRY(P::inverse_xy_k(ctx, ctx->U, ctx->V, TK, tstride, nfield, ws.data(), K, wpre ? wpre + s * nt : nullptr));
           a.kzlive = N / 2;
           Tsrc = TK;
         } else {
@@ -994,7 +1017,7 @@ struct FilteredField {
     {
       using P = Pipe<N>;
       MRX_TRY(ensure_buffers(ctx, N, 1));
-      MRX_TRY(P::forward(ctx, in, 0, 1, true, ctx->U, ctx->V));
+      MRX_TRY(P::forward(ctx, in, true, ctx->U, ctx->V));
       const WinArgs w = win_args(box_size, (float)R, filter_type, apply);
       int kzlive;
       MRX_TRY(P::inverse_xy(ctx, ctx->U, ctx->V, ctx->T, 1, w, kzlive));
@@ -1010,7 +1033,7 @@ struct R2C {
     {
       using P = Pipe<N>;
       MRX_TRY(ensure_buffers(ctx, N, 1));
-      MRX_TRY(P::forward(ctx, in, 0, 1, false, ctx->U, ctx->V));
+      MRX_TRY(P::forward(ctx, in, false, ctx->U, ctx->V));
       return P::unpack_herm(ctx, ctx->U, ctx->V, out);
     }
   };
@@ -1280,7 +1303,7 @@ struct TsRun {
             if (nmax < N / 2)
               MRX_TRY(P::forward_sharpk(ctx, wgrid, ctx->U, ctx->V, nmax));
             else
-              MRX_TRY(P::forward(ctx, wgrid, 0, 1, true, ctx->U, ctx->V, true));
+              MRX_TRY(P::forward(ctx, wgrid, true, ctx->U, ctx->V, true));
           }
           int kzlive;
           MRX_TRY(P::inverse_xy(ctx, ctx->U, ctx->V, ctx->T, 1, w, kzlive));
@@ -1430,7 +1453,7 @@ struct TbVel {
         k_vel_convert<<<nb, kNT, 0, ctx->stream>>>(vel, N, a.redshift, a.trees_id);
       }
       MRX_TRY(check_launch(ctx, "k_vel_convert"));
-      MRX_TRY(P::forward(ctx, vel, 0, 1, true, ctx->U, ctx->V));
+      MRX_TRY(P::forward(ctx, vel, true, ctx->U, ctx->V));
       const float box_f = (float)p->box_size;
       const float delta_k = (float)(2.0 * M_PI / box_f);
       {
@@ -1524,7 +1547,7 @@ struct PowerSpec {
       float* work = ctx->adj_work;
       k_ps_prep<<<(unsigned)((ncell + 255) / 256), 256, 0, ctx->stream>>>(dT, work, N, ave, (float)a.volume);
       MRX_TRY(check_launch(ctx, "k_ps_prep"));
-      MRX_TRY(P::forward(ctx, work, 0, 1, false, ctx->U, ctx->V));
+      MRX_TRY(P::forward(ctx, work, false, ctx->U, ctx->V));
       k_ps_bin<<<nblk, kNT, 0, ctx->stream>>>(ctx->U, ctx->V, ctx->partials, a);
       MRX_TRY(check_launch(ctx, "k_ps_bin"));
       k_reduce_partials<<<1, kNT, 0, ctx->stream>>>(ctx->partials, nblk, nb * 3, sums_big);
@@ -1743,7 +1766,7 @@ struct SnapAdj {
         MRX_TRY(check_launch(ctx, "k_ts_shell_grad"));
         const float* add = gshell;
         if (ct > 0) {  // shell 0 is the unfiltered grid
-          MRX_TRY(P::forward(ctx, gshell, 0, 1, true, ctx->U, ctx->V, true));
+          MRX_TRY(P::forward(ctx, gshell, true, ctx->U, ctx->V, true));
           const WinArgs w = win_args(tp->box_size, (float)s->R[ct], tp->heating_filter_type, 1);
           int kzlive;
           MRX_TRY(P::inverse_xy(ctx, ctx->U, ctx->V, ctx->T, 1, w, kzlive));

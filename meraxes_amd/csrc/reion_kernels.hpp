@@ -195,12 +195,17 @@ __device__ __forceinline__ void r2c_z_tile(const float* __restrict__ in, float2*
   }
 }
 
-// blockIdx.y selects the field (strides in_fstride, out_fstride)
+// The input grids of up to five fields (separate allocations), by value.
+struct FieldTab {
+  const float* p[5];
+};
+
+// blockIdx.y selects the field (outputs at stride out_fstride)
 template <int N>
-__global__ __launch_bounds__(kNT) void k_r2c_z(const float* __restrict__ in, float2* __restrict__ out,
-                                              const float2* __restrict__ twN, long in_fstride, long out_fstride)
+__global__ __launch_bounds__(kNT) void k_r2c_z(FieldTab in, float2* __restrict__ out, const float2* __restrict__ twN,
+                                              long out_fstride)
 {
-  r2c_z_tile<N>(in + blockIdx.y * in_fstride, out + blockIdx.y * out_fstride, twN);
+  r2c_z_tile<N>(in.p[blockIdx.y], out + blockIdx.y * out_fstride, twN);
 }
 
 // blockIdx.y selects the field through a table of input pointers (batches of
@@ -384,11 +389,19 @@ constexpr unsigned window_table_blocks()
   return (unsigned)((N / 2 + 1) * ((N / 2) / TW) + (N / 2 + 1));
 }
 
+// The radii of one launch (blockIdx.y), by value; w.R is replaced by theirs.
+constexpr int kWinRadii = 64;
+struct WinRadii {
+  float R[kWinRadii];
+};
+
 template <int N, int TW>
-__global__ __launch_bounds__(kNT) void k_window_table(float* __restrict__ Wt, WinArgs w)
+__global__ __launch_bounds__(kNT) void k_window_table(float* __restrict__ Wt, WinArgs w, WinRadii radii)
 {
   constexpr int NH = N / 2, NH1 = NH + 1, NKZB = NH / TW;
   const int blk = blockIdx.x;
+  w.R = radii.R[blockIdx.y];
+  Wt += (long)blockIdx.y * NH1 * NH1 * NH1;
   if (blk < NH1 * NKZB) {
     const int b = blk / NKZB, kb = blk % NKZB;
     float* out = Wt + (long)blk * NH1 * TW;

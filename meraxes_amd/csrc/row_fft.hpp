@@ -18,7 +18,7 @@
 // pass had 7 to 12 waves per CU at the lengths with a factor 3 or 5; per step
 // it went from 336 to 146 us (320^3, four fields, now at its vector
 // instructions: about 80 per complex point, 130 us), from 77 to 35 us (160^3,
-// five fields), from 65 to 42 us (192^3) and from 13.9 to 9.1 us (128^3).
+// five fields), from 65 to 32 us (192^3) and from 13.9 to 9.1 us (128^3).
 #pragma once
 #include "fft_lds.hpp"
 
