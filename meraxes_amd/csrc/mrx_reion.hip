@@ -17,7 +17,6 @@
 #include <memory>
 #include <mutex>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "../../include/mrx_reion.h"
@@ -25,6 +24,7 @@
 #include "reion_kernels.hpp"
 #include "ts_kernels.hpp"
 #include "adjoint.hpp"
+#include "ts_quad.hpp"
 #include "ts_tables.h"
 #include "recomb_tables.h"
 
@@ -122,8 +122,14 @@ struct mrx_ctx {
   mrx_ts_data* tsd = nullptr;
   std::string ts_key;
   mrx_ts_snap* tss = nullptr;
-  TsDev* ts_host = nullptr;
+  TsDev* ts_host = nullptr;  // pinned: its upload does not stop the host
   TsDev* ts_dev = nullptr;
+  // the frequency integrals on the device (ts_quad.hpp): their tables, for the
+  // table set quad_key, and the results of up to kQuadBuilds builds
+  TsQuadDev* quad_dev = nullptr;
+  std::string quad_key;
+  double* quad_out = nullptr;   // device
+  double* quad_host = nullptr;  // pinned
   float* ts_work = nullptr;
   size_t ts_work_cap = 0;
   float* ts_shells = nullptr;
@@ -131,8 +137,9 @@ struct mrx_ctx {
   int ts_shells_N = 0, ts_shells_n = 0;  // grid and shell count ts_shells holds (0: none)
   float* wtab = nullptr;  // window tables of the current radii, (N/2+1)^3 floats each
   size_t wtab_cap = 0;
-  // the bubble ladder's window tables of every filtered radius, built on a
-  // stream of their own (default priority) while the fields are transformed
+  // a second stream (default priority): the bubble ladder's window tables of
+  // every filtered radius are built on it while the fields are transformed, and
+  // the spin temperature's frequency integrals while its shells are filtered
   float* wtab_all = nullptr;
   size_t wtab_all_cap = 0;
   hipStream_t side = nullptr;
@@ -396,6 +403,14 @@ int ensure_buf(mrx_ctx* ctx, float*& p, size_t& cap, size_t nfloat)
     return set_err(ctx, MRX_ENOMEM, "device allocation of %zu floats failed", nfloat);
   }
   cap = nfloat;
+  return MRX_OK;
+}
+
+int ensure_side(mrx_ctx* ctx)
+{
+  if (!ctx->side) HIP_TRY(hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking));
+  for (auto& e : ctx->side_ev)
+    if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   return MRX_OK;
 }
 
@@ -894,9 +909,7 @@ struct HiiRun {
         if (!use_side) {
           MRX_TRY(P::window_tables(ctx, ctx->wtab_all, ws.data(), S - 1));
         } else {
-          if (!ctx->side) HIP_TRY(hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking));
-          for (auto& e : ctx->side_ev)
-            if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+          MRX_TRY(ensure_side(ctx));
           HIP_TRY(hipEventRecord(ctx->side_ev[0], ctx->stream));
           HIP_TRY(hipStreamWaitEvent(ctx->side, ctx->side_ev[0], 0));
           hipStream_t const main_stream = ctx->stream;
@@ -1164,6 +1177,103 @@ double ts_RtoM(const mrx_ts_params* p, double R)
   return pow(2 * M_PI, 1.5) * p->omega_m * p->rho_crit * pow(R, 3);
 }
 
+// Queues the lower frequency limits and frequency integrals of nbuild table
+// builds (their collapse fractions cf and <x_e> xe) on the side stream; they
+// read no grid.  quad_results waits for them.
+int quad_launch(mrx_ctx* ctx, const mrx_ts_params* p, const mrx_ts_snap* s, int nbuild, const double* cf,
+                const double* xe)
+{
+  MRX_TRY(ensure_side(ctx));
+  const size_t out_bytes = sizeof(double) * kQuadBuilds * kQuadOut;
+  if (!ctx->quad_dev) HIP_TRY(hipMalloc(&ctx->quad_dev, sizeof(TsQuadDev)));
+  if (!ctx->quad_out) HIP_TRY(hipMalloc(&ctx->quad_out, out_bytes));
+  if (!ctx->quad_host) HIP_TRY(hipHostMalloc(&ctx->quad_host, out_bytes, hipHostMallocDefault));
+  const mrx_ts_data* d = ctx->tsd;
+  if (ctx->quad_key != ctx->ts_key) {
+    std::unique_ptr<TsQuadDev> t(new TsQuadDev());
+    for (int l = 0; l < 61; ++l) {  // lanes 0-29 below the centre, 30-59 above, 60 the centre
+      const int j = l < 60 ? l % 30 : 30;
+      t->node[l] = (l < 30 ? -1.0 : 1.0) * mrx_gk61_xgk[j];
+      t->wk[l] = mrx_gk61_wgk[j];
+      t->wg[l] = (l < 60 && (j & 1)) ? mrx_gk61_wg[j / 2] : 0.0;
+    }
+    t->f_H = d->f_H;
+    t->f_He = d->f_He;
+    t->N_b0 = d->N_b0;
+    t->hubble_h = d->hubble_h;
+    t->omega_m = d->omega_m;
+    t->omega_l = d->omega_l;
+    t->ion_eff = d->reion_efficiency;
+    memcpy(t->XH, d->xi_XHII, sizeof t->XH);
+    memcpy(t->E, d->xi_E, sizeof t->E);
+    memcpy(t->fheat, d->xi_fheat, sizeof t->fheat);
+    memcpy(t->nLya, d->xi_nLya, sizeof t->nLya);
+    memcpy(t->nHI, d->xi_nHI, sizeof t->nHI);
+    memcpy(t->nHeI, d->xi_nHeI, sizeof t->nHeI);
+    memcpy(t->nHeII, d->xi_nHeII, sizeof t->nHeII);
+    HIP_TRY(hipStreamSynchronize(ctx->side));  // an earlier launch may still read the old tables
+    ctx->quad_key.clear();
+    HIP_TRY(hipMemcpy(ctx->quad_dev, t.get(), sizeof(TsQuadDev), hipMemcpyHostToDevice));
+    ctx->quad_key = ctx->ts_key;
+  }
+  TsQuadArgs a;
+  memset(&a, 0, sizeof a);
+  const double nu_over_ev = quad::kNuOverEv;
+  a.nsteps = s->nsteps;
+  a.nbuild = nbuild;
+  a.first_snapshot = (p->snapshot == 0) ? 1 : 0;
+  a.zp = s->zp;
+  a.Z1 = p->redshifts[p->snapshot];
+  a.Z0 = a.first_snapshot ? a.Z1 : p->redshifts[p->snapshot - 1];
+  a.F0 = a.first_snapshot ? 0.0 : p->stored_fcoll[p->snapshot - 1];
+  for (int b = 0; b < nbuild; ++b) {
+    a.F1[b] = cf[b];
+    a.x_e[b] = xe[b];
+  }
+  a.nu_min = p->nu_xray_gal_threshold * nu_over_ev;
+  a.nu_max = p->nu_xray_max * nu_over_ev;
+  a.spec_index = p->spec_index_xray_gal;
+  for (int ct = 0; ct < s->nsteps; ++ct)
+    a.zpp[ct] = (s->zpp_edge[ct] + (ct == 0 ? s->zp : s->zpp_edge[ct - 1])) * 0.5;
+  struct OnSide {  // kernel timings are recorded on the launch stream
+    mrx_ctx* c;
+    hipStream_t main;
+    explicit OnSide(mrx_ctx* x) : c(x), main(x->stream) { c->stream = c->side; }
+    ~OnSide() { c->stream = main; }
+  } on_side(ctx);
+  {
+    PROF("nu_lower");
+    k_ts_nu_lower<<<dim3(s->nsteps, nbuild), 64, 0, ctx->stream>>>(ctx->quad_dev, a, ctx->quad_out);
+  }
+  MRX_TRY(check_launch(ctx, "k_ts_nu_lower"));
+  {
+    PROF("freq_integrals");
+    k_ts_freq_integrals<<<dim3(s->nsteps, 3 * kNXHII, nbuild), 64, 0, ctx->stream>>>(ctx->quad_dev, a, ctx->quad_out);
+  }
+  MRX_TRY(check_launch(ctx, "k_ts_freq_integrals"));
+  HIP_TRY(hipMemcpyAsync(ctx->quad_host, ctx->quad_out, sizeof(double) * nbuild * kQuadOut, hipMemcpyDeviceToHost,
+                         ctx->stream));
+  return MRX_OK;
+}
+
+// Build b of the last quad_launch into s.
+int quad_results(mrx_ctx* ctx, int b, mrx_ts_snap* s)
+{
+  HIP_TRY(hipStreamSynchronize(ctx->side));
+  const mrx_ts_data* d = ctx->tsd;
+  const double* o = ctx->quad_host + (size_t)b * kQuadOut;
+  const double H = mrx_ts_hubble(d, (float)s->zp);
+  for (int ct = 0; ct < s->nsteps; ++ct) {
+    s->nu_lower[ct] = o[ct];
+    for (int x = 0; x < kNXHII; ++x) {
+      s->freq_heat[x][ct] = o[quad_index(0, x, ct)];
+      s->freq_ion[x][ct] = o[quad_index(1, x, ct)];
+      s->freq_lya[x][ct] = o[quad_index(2, x, ct)] * quad::kSpeedOfLight / (4 * M_PI) / 2.46606727e15 / H;
+    }
+  }
+  return MRX_OK;
+}
+
 struct TsRun {
   template <int N>
   struct At {
@@ -1243,8 +1353,7 @@ struct TsRun {
         ctx->ts_shells_N = ctx->ts_shells_n = 0;
         MRX_TRY(ensure_buf(ctx, ctx->ts_shells, ctx->ts_shells_cap, (size_t)s->nsteps * ncell));
         // f_coll and <x_e> of the first shell (ComputeTs.c:413-475) read the
-        // input grids only: taken first, so the host builds the tables while
-        // the device filters the shells
+        // input grids only: taken first, for the tables
         if (!p->fixed_globals) MRX_TRY(fcoll(s->R[0], 1));
         if (p->fixed_globals) {
           collapse_fraction = p->fixed_collapse_fraction;
@@ -1252,23 +1361,9 @@ struct TsRun {
         }
         s->collapse_fraction = collapse_fraction;
         s->x_e_ave = x_e_ave;
-        // the host tables are built on a thread of their own while this one
-        // queues the shells' kernels (the build reads the plan's radii and
-        // edges and writes only the tables; the shell loop reads the plan)
-        int tab_rc = MRX_OK;
-        std::thread tab;
-        try {
-          tab = std::thread([&tab_rc, s, d, p] { tab_rc = mrx_ts_build_tables(s, d, p); });
-        } catch (...) {  // no thread to be had: build them here, before the shells
-          tab_rc = mrx_ts_build_tables(s, d, p);
-        }
-        struct Join {
-          std::thread& t;
-          ~Join()
-          {
-            if (t.joinable()) t.join();
-          }
-        } join_tab{tab};
+        // the shells' frequency integrals run on the side stream while this
+        // one filters the shells
+        MRX_TRY(quad_launch(ctx, p, s, 1, &s->collapse_fraction, &s->x_e_ave));
         const long half = (long)N * N * (N / 2 + 1);
         // the working grid starts as the input sfr grid: it is read in place
         // until the first shell with operations writes ts_work from it
@@ -1311,8 +1406,8 @@ struct TsRun {
         }
         ctx->ts_shells_N = N;
         ctx->ts_shells_n = s->nsteps;
-        if (tab.joinable()) tab.join();
-        if (tab_rc != MRX_OK) return set_err(ctx, tab_rc, "spin-temperature tables failed");
+        if (mrx_ts_finish_tables(s, d, p) != MRX_OK) return set_err(ctx, MRX_EINVAL, "spin-temperature tables failed");
+        MRX_TRY(quad_results(ctx, 0, s));
         fill_ts_dev(*ctx->ts_host, d, s, p);
         HIP_TRY(hipMemcpyAsync(ctx->ts_dev, ctx->ts_host, sizeof(TsDev), hipMemcpyHostToDevice, ctx->stream));
         if (prepare_only) return MRX_OK;
@@ -1587,11 +1682,27 @@ struct SnapAdj {
     // The gradient through the shell tables' two grid means, the collapse
     // fraction and <x_e> (ComputeTs.c:413-475), which the tables take through
     // tau_X: the derivatives of the six x_e tables with respect to each mean
-    // by central differences of the host table build (relative step 1e-4),
+    // by central differences of the table build (relative step 1e-4),
     // contracted on the device with every cell's shell values and shell-sum
     // adjoints (k_ts_means_grad), then spread back over the cells the means
     // are taken from (k_ts_means_apply).  <x_e> only when its gradient
     // (g_xe_prev) is wanted.
+    static constexpr double kMeansStep = 1e-4;
+    static double means_h(double x0) { return kMeansStep * std::max(std::fabs(x0), 1e-8); }
+    // the 2 nm table builds (each mean + and - its step), on the side stream
+    static int means_launch(mrx_ctx* ctx, const mrx_ts_params* tp, const mrx_ts_snap* s, int nm)
+    {
+      static_assert(kQuadBuilds >= 4, "two means, two sides");
+      double cf[4], xe[4];
+      for (int m = 0; m < nm; ++m)
+        for (int sg = 0; sg < 2; ++sg) {
+          cf[2 * m + sg] = s->collapse_fraction;
+          xe[2 * m + sg] = s->x_e_ave;
+          double& v = (m == 0) ? cf[2 * m + sg] : xe[2 * m + sg];
+          v += (sg ? -1 : 1) * means_h(v);
+        }
+      return quad_launch(ctx, tp, s, 2 * nm, cf, xe);
+    }
     static int means_tables(mrx_ctx* ctx, const mrx_ts_params* tp, const mrx_ts_snap* s, int nm,
                             std::vector<double>& E)
     {
@@ -1600,17 +1711,18 @@ struct SnapAdj {
       std::unique_ptr<mrx_ts_snap> sc(new mrx_ts_snap);
       std::unique_ptr<TsDev> tplus(new TsDev), tminus(new TsDev);
       const TsDev& t0 = *ctx->ts_host;  // the forward's constants
-      // the table build records the collapse fraction in the caller's history
+      // finishing a build records its collapse fraction in the caller's history
       double* fc_slot = tp->stored_fcoll ? tp->stored_fcoll + tp->snapshot : nullptr;
       const double fc_saved = fc_slot ? *fc_slot : 0.0;
       int rc = MRX_OK;
       for (int m = 0; m < nm && rc == MRX_OK; ++m) {
         const double x0 = (m == 0) ? s->collapse_fraction : s->x_e_ave;
-        const double h = 1e-4 * std::max(std::fabs(x0), 1e-8);
+        const double h = means_h(x0);
         for (int sg = 0; sg < 2 && rc == MRX_OK; ++sg) {
           *sc = *s;
           (m == 0 ? sc->collapse_fraction : sc->x_e_ave) = x0 + (sg ? -h : h);
-          rc = mrx_ts_build_tables(sc.get(), ctx->tsd, tp);
+          rc = mrx_ts_finish_tables(sc.get(), ctx->tsd, tp);
+          if (rc == MRX_OK) rc = quad_results(ctx, 2 * m + sg, sc.get());
           if (rc == MRX_OK) fill_ts_dev(sg ? *tminus : *tplus, ctx->tsd, sc.get(), tp);
         }
         if (rc != MRX_OK) break;
@@ -1696,32 +1808,16 @@ struct SnapAdj {
       }
       const bool shells = (a.ts_mode == 2) && !s->no_light;
       if (a.ts_mode == 2) MRX_TRY(ensure_dev(ctx, ctx->adj_gS, ctx->adj_gS_cap, 4 * (size_t)ncell));
-      // the tables' derivatives with respect to their grid means are host
-      // work: built on a thread of their own while the device runs the
-      // adjoint, and used after the shells' adjoints
+      // the tables' derivatives with respect to their grid means: the builds
+      // run on the side stream beside the adjoint and are used after the
+      // shells' adjoints
       const bool means = shells && !tp->fixed_globals;
       const int nm = g_xe_prev ? 2 : 1;
       std::vector<double> E;
-      int E_rc = MRX_OK;
-      std::thread E_thread;
-      if (means) {
-        try {
-          E_thread = std::thread([&E_rc, &E, ctx, tp, s, nm] { E_rc = means_tables(ctx, tp, s, nm, E); });
-        } catch (...) {
-          E_rc = means_tables(ctx, tp, s, nm, E);
-        }
-      }
-      struct JoinE {
-        std::thread& t;
-        ~JoinE()
-        {
-          if (t.joinable()) t.join();
-        }
-      } join_E{E_thread};
+      if (means) MRX_TRY(means_launch(ctx, tp, s, nm));
       auto finish_means = [&]() -> int {
         if (!means) return MRX_OK;
-        if (E_thread.joinable()) E_thread.join();
-        if (E_rc != MRX_OK) return set_err(ctx, E_rc, "spin-temperature tables (grid-mean derivatives) failed");
+        MRX_TRY(means_tables(ctx, tp, s, nm, E));
         return means_term(ctx, tp, s, nm, E, deltax, stars, xe_prev, g_delta, g_stars, g_xe_prev);
       };
       const unsigned nbc = (unsigned)((ncell + kNT - 1) / kNT);
@@ -1970,7 +2066,10 @@ int mrx_free(mrx_ctx* ctx)
   for (auto& e : ctx->ext) dfree(e);
   delete ctx->tsd;
   delete ctx->tss;
-  delete ctx->ts_host;
+  if (ctx->ts_host) (void)hipHostFree(ctx->ts_host);
+  dfree(ctx->quad_dev);
+  dfree(ctx->quad_out);
+  if (ctx->quad_host) (void)hipHostFree(ctx->quad_host);
   for (auto& r : ctx->prof_recs) {
     (void)hipEventDestroy(r.a);
     (void)hipEventDestroy(r.b);
@@ -2199,7 +2298,7 @@ int mrx_compute_ts(mrx_ctx* ctx, const mrx_ts_params* p, const float* deltax, co
     ctx->ts_key = key;
   }
   if (!ctx->tss) ctx->tss = new mrx_ts_snap();
-  if (!ctx->ts_host) ctx->ts_host = new TsDev();
+  if (!ctx->ts_host) HIP_TRY(hipHostMalloc(&ctx->ts_host, sizeof(TsDev), hipHostMallocDefault));
   if (const int prc = mrx_ts_plan(ctx->tss, ctx->tsd, p); prc != MRX_OK)
     return prc == MRX_EUNSUPPORTED
              ? set_err(ctx, prc, "a spin-temperature shell needs more than %d SFR-history operations",
@@ -2470,7 +2569,7 @@ int mrx_snapshot_adjoint(mrx_ctx* ctx, const mrx_ts_params* ts, const mrx_hii_pa
       ctx->ts_key = key;
     }
     if (!ctx->tss) ctx->tss = new mrx_ts_snap();
-    if (!ctx->ts_host) ctx->ts_host = new TsDev();
+    if (!ctx->ts_host) HIP_TRY(hipHostMalloc(&ctx->ts_host, sizeof(TsDev), hipHostMallocDefault));
     if (const int prc = mrx_ts_plan(ctx->tss, ctx->tsd, ts); prc != MRX_OK)
       return prc == MRX_EUNSUPPORTED
                ? set_err(ctx, prc, "a spin-temperature shell needs more than %d SFR-history operations",

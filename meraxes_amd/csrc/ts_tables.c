@@ -1012,11 +1012,11 @@ int mrx_ts_plan(mrx_ts_snap* s, const mrx_ts_data* d, const mrx_ts_params* p)
   return MRX_OK;
 }
 
-/* The shells' tables are independent of one another: one work item is a
- * shell, its lower frequency limit, raw Ly-n sum and 3 x 14 frequency
- * integrals (which share one table of node values); items are handed out one
- * at a time to up to 16 host threads.  Each item is computed exactly as the
- * serial loop would, so the tables do not depend on the thread count. */
+/* The shells' integrals are independent of one another: one work item is a
+ * shell, its lower frequency limit and 3 x 14 frequency integrals (which share
+ * one table of node values); items are handed out one at a time to up to 16
+ * host threads.  Each item is computed exactly as the serial loop would, so
+ * the tables do not depend on the thread count. */
 typedef struct {
   mrx_ts_snap* s;
   const mrx_ts_data* d;
@@ -1036,13 +1036,6 @@ static void tab_item(tab_job* j, int ct, nu_cache* cache)
   const double lower =
     fmax(mrx_ts_nu_tau_one(d, p, zp, zpp, s->x_e_ave, s->x_e_ave), p->nu_xray_gal_threshold * K_NU_over_EV);
   s->nu_lower[ct] = lower;
-  double sum = 0;
-  for (int n_ct = MRX_NSPEC_MAX; n_ct >= 2; n_ct--) {
-    if (zpp > zmax((float)zp, n_ct)) continue;
-    const double nuprime = nu_n(n_ct) * (1 + zpp) / (1.0 + zp);
-    sum += frecycle(n_ct) * mrx_ts_spectral_emissivity(d, nuprime);
-  }
-  s->sum_lyn[ct] = sum;
   if (cache) nu_cache_clear(cache);
   for (int x = 0; x < MRX_X_INT_NXHII; x++) {
     s->freq_heat[x][ct] = integrate_over_nu(d, p, zp, d->xi_XHII[x], lower, 0, cache);
@@ -1079,7 +1072,39 @@ static void tab_run(tab_job* j)
   for (int t = 0; t < started; t++) pthread_join(th[t], NULL);
 }
 
+/* The raw Ly-n sums of the shells (ComputeTs.c:590-612) */
+static void lyn_sums(mrx_ts_snap* s, const mrx_ts_data* d)
+{
+  const double zp = s->zp;
+  double top[MRX_NSPEC_MAX + 1], nu[MRX_NSPEC_MAX + 1], rec[MRX_NSPEC_MAX + 1];
+  for (int n = 2; n <= MRX_NSPEC_MAX; n++) {
+    top[n] = zmax((float)zp, n);
+    nu[n] = nu_n(n);
+    rec[n] = frecycle(n);
+  }
+  for (int ct = 0; ct < s->nsteps; ct++) {
+    const double prev_zpp = (ct == 0) ? zp : s->zpp_edge[ct - 1];
+    const double zpp = (s->zpp_edge[ct] + prev_zpp) * 0.5;
+    double sum = 0;
+    for (int n = MRX_NSPEC_MAX; n >= 2; n--) {
+      if (zpp > top[n]) continue;
+      const double nuprime = nu[n] * (1 + zpp) / (1.0 + zp);
+      sum += rec[n] * mrx_ts_spectral_emissivity(d, nuprime);
+    }
+    s->sum_lyn[ct] = sum;
+  }
+}
+
 int mrx_ts_build_tables(mrx_ts_snap* s, const mrx_ts_data* d, const mrx_ts_params* p)
+{
+  if (s->homogeneous) return MRX_OK;
+  if (p->stored_fcoll) p->stored_fcoll[p->snapshot] = s->collapse_fraction; /* tau_X interpolates to it */
+  tab_job job = {s, d, p, s->nsteps, 0};
+  tab_run(&job);
+  return mrx_ts_finish_tables(s, d, p);
+}
+
+int mrx_ts_finish_tables(mrx_ts_snap* s, const mrx_ts_data* d, const mrx_ts_params* p)
 {
   if (s->homogeneous) return MRX_OK;
   const double zp = s->zp;
@@ -1089,8 +1114,7 @@ int mrx_ts_build_tables(mrx_ts_snap* s, const mrx_ts_data* d, const mrx_ts_param
   int first_radii = 1, first_zero = 1;
   const int n_pts_radii = 1000;
   double weight = s->final_weight; /* the shell loop's last weight (one variable in the reference) */
-  tab_job job = {s, d, p, s->nsteps, 0};
-  tab_run(&job);
+  lyn_sums(s, d);
   for (int ct = 0; ct < s->nsteps; ct++) {
     double prev_zpp, prev_R;
     if (ct == 0) {

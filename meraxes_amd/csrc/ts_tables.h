@@ -109,6 +109,10 @@ int mrx_ts_plan(mrx_ts_snap* s, const mrx_ts_data* d, const mrx_ts_params* p);
  * x_e_ave of the first shell are known; writes stored_fcoll[snapshot]. */
 int mrx_ts_build_tables(mrx_ts_snap* s, const mrx_ts_data* d, const mrx_ts_params* p);
 
+/* mrx_ts_build_tables without the lower frequency limits and the integrals
+ * (nu_lower, freq_*), for a caller that has them from the device (ts_quad.hpp). */
+int mrx_ts_finish_tables(mrx_ts_snap* s, const mrx_ts_data* d, const mrx_ts_params* p);
+
 /* dt/dz of the flat LCDM cosmology (XRayHeatingFunctions.c:377-392) */
 double mrx_cosmo_dtdz(double omega_l, double omega_m, double hubble_h, float z);
 
