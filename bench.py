@@ -576,7 +576,8 @@ def bench_batched(ctx, steps, warmup, per_size=BATCH_PER_SIZE):
         torch.cuda.synchronize()
         tp = time.perf_counter() - t0
         bs.close()
-        alg = sum(path_bytes_hii(N, 3, len(P.radius_ladder(b["params"]))) for b in sub)
+        # without the UVB the ladder transforms two fields (the weighted SFR only feeds J_21)
+        alg = sum(path_bytes_hii(N, 2, len(P.radius_ladder(b["params"]))) for b in sub)
         per_size[str(N)] = {"batched_ms": tb * 1e3, "plain_loop_ms": tp * 1e3, "speedup": tp / tb,
                             "alg_bytes": alg, "batched_GB_s": alg / tb / 1e9, "batched_frac": alg / tb / HBM_PEAK,
                             "plain_loop_GB_s": alg / tp / 1e9, "plain_loop_frac": alg / tp / HBM_PEAK}

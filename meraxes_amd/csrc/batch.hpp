@@ -212,8 +212,6 @@ struct BatchPipe {
     memset(&a, 0, sizeof a);
     a.pixel_volume = pow(p->box_size / (double)N, 3);
     a.uvb = p->uvb_flag;
-    a.use_xe = p->include_spin_temp;
-    a.nfield = c.F;
     a.kzlive = N / 2;
     const int nb = nb_threshold();
     for (int s = 0; s < c.S; ++s) {
@@ -223,12 +221,14 @@ struct BatchPipe {
       a.step = s;
       a.last = last ? 1 : 0;
       constexpr int NT = RowCfg<N>::NT;
-      if (c.F == 4)
-        k_c2r_threshold_batch<N, 4><<<dim3(nb, c.nbox), NT, 0, c.stream>>>(
+      auto thr = [&](auto fs) {
+        k_c2r_threshold_batch<N, decltype(fs)><<<dim3(nb, c.nbox), NT, 0, c.stream>>>(
           c.T, nc, (long)c.F * nc, c.tw, c.boxes_dev, c.state, c.Rtab, c.steps, c.J21c, c.S, c.partials, a);
+      };
+      if (p->uvb_flag)
+        p->include_spin_temp ? thr(Fields<true, true, false>()) : thr(Fields<false, true, false>());
       else
-        k_c2r_threshold_batch<N, 3><<<dim3(nb, c.nbox), NT, 0, c.stream>>>(
-          c.T, nc, (long)c.F * nc, c.tw, c.boxes_dev, c.state, c.Rtab, c.steps, c.J21c, c.S, c.partials, a);
+        p->include_spin_temp ? thr(Fields<true, false, false>()) : thr(Fields<false, false, false>());
       MRX_TRY(check_launch(ctx, "k_c2r_threshold_batch"));
     }
     // the same reduction as the single-box path, so each box's globals are identical to it
@@ -287,8 +287,10 @@ struct BatchPipe {
       bd[i].redshift = b.params.redshift;
       bd[i].bias = b.params.gamma_halo_bias;
       for (int s = 0; s < c.S; ++s) j[(size_t)i * c.S + s] = step_consts(&b.params, c.R[s], false).J21c;
-      const float* src[4] = {b.deltax, b.stars, b.weighted_sfr, b.x_e};
-      for (int f = 0; f < c.F; ++f) in[(size_t)i * c.F + f] = src[f];
+      int f = 0;
+      for (const float* q : {b.deltax, b.stars, c.p0.uvb_flag ? b.weighted_sfr : nullptr,
+                             c.p0.include_spin_temp ? b.x_e : nullptr})
+        if (q) in[(size_t)i * c.F + f++] = q;
     }
     HIP_TRY(hipMemcpy(c.boxes_dev, bd.data(), sizeof(BoxDev) * c.nbox, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c.J21c, j.data(), sizeof(double) * j.size(), hipMemcpyHostToDevice));

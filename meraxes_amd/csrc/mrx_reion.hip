@@ -660,55 +660,47 @@ struct Pipe {
     return check_launch(ctx, "k_c2r_z");
   }
 
-  // the last pass of K ladder steps, step k's spectra at Tsrc + k tstride;
-  // fields deltax, stars, sfr (+ x_e) (+ N_rec when rec)
-  // 256^3 and 512^3 without recombinations: the row transforms in registers
-  // (k_c2r_threshold_reg); otherwise row_fft.hpp's (k_c2r_threshold)
+  // the last pass of K ladder steps, step k's spectra (Fields' order) at Tsrc
+  // + k tstride.  256^3 and 512^3 without recombinations: the row transforms in
+  // registers (k_c2r_threshold_reg); otherwise row_fft.hpp's (k_c2r_threshold)
   static constexpr bool kRegThr = (N == 256 || N == 512);
-  static int threshold(mrx_ctx* ctx, const float2* Tsrc, long tstride, int K, const float* deltax, float* xH,
-                       float* rb, float* J21, float* zin, float* J21i, float* Gamma12, bool rec, const StepArgs& a)
+  template <class FS>
+  static int threshold_fs(mrx_ctx* ctx, const float2* Tsrc, long tstride, int K, const ThrGrids& g, const StepArgs& a)
   {
-    const int nb = nblocks_threshold(rec);
-    const ThrGrids g{deltax, ctx->state, xH, rb, J21, zin, J21i, Gamma12, ctx->Rtab};
-    if constexpr (kRegThr) {
-      if (!rec) {
-        constexpr int A = N / 32;
-        StepArgs ak = a;
-        for (int k = 0; k < K; ++k, ++ak.step) {
-          PROF("c2r_threshold");
-          const float2* Tk = Tsrc + k * tstride;
-          if (a.nfield == 4)
-            k_c2r_threshold_reg<A, 4><<<nb, 256, 0, ctx->stream>>>(Tk, nc, ctx->tw, ctx->steps, g, ctx->partials, ak);
-          else
-            k_c2r_threshold_reg<A, 3><<<nb, 256, 0, ctx->stream>>>(Tk, nc, ctx->tw, ctx->steps, g, ctx->partials, ak);
-        }
-        return check_launch(ctx, "k_c2r_threshold_reg");
+    if constexpr (kRegThr && !FS::REC) {
+      constexpr int A = N / 32;
+      using C = RegThr<A, FS::N>;
+      StepArgs ak = a;
+      for (int k = 0; k < K; ++k, ++ak.step) {
+        PROF("c2r_threshold");
+        k_c2r_threshold_reg<A, FS><<<N * N / C::RWG, C::NT, 0, ctx->stream>>>(Tsrc + k * tstride, nc, ctx->tw,
+                                                                             ctx->steps, g, ctx->partials, ak);
       }
+      return check_launch(ctx, "k_c2r_threshold_reg");
+    } else {
+      PROF("c2r_threshold");
+      k_c2r_threshold<N, FS><<<N * N / RowCfg<N>::ROWS, RowCfg<N>::NT, 0, ctx->stream>>>(
+        Tsrc, nc, tstride, K, ctx->tw, ctx->steps, g, ctx->partials, a);
+      return check_launch(ctx, "k_c2r_threshold");
     }
-    PROF("c2r_threshold");
-    constexpr int NT = RowCfg<N>::NT;
-#define MRX_THR(NF_, REC_)                                                                                  \
-  k_c2r_threshold<N, NF_, REC_><<<nb, NT, 0, ctx->stream>>>(Tsrc, nc, tstride, K, ctx->tw, ctx->steps, g, \
-                                                           ctx->partials, a)
-    if (rec) {
-      if (a.nfield == 5)
-        MRX_THR(5, true);
-      else
-        MRX_THR(4, true);
-    } else if constexpr (!kRegThr) {
-      if (a.nfield == 4)
-        MRX_THR(4, false);
-      else
-        MRX_THR(3, false);
-    }
-#undef MRX_THR
-    return check_launch(ctx, "k_c2r_threshold");
+  }
+  static int threshold(mrx_ctx* ctx, const float2* Tsrc, long tstride, int K, const ThrGrids& g, bool xe, bool sfr,
+                       bool rec, const StepArgs& a)
+  {
+    if (rec)
+      return xe ? threshold_fs<Fields<true, true, true>>(ctx, Tsrc, tstride, K, g, a)
+                : threshold_fs<Fields<false, true, true>>(ctx, Tsrc, tstride, K, g, a);
+    if (sfr)
+      return xe ? threshold_fs<Fields<true, true, false>>(ctx, Tsrc, tstride, K, g, a)
+                : threshold_fs<Fields<false, true, false>>(ctx, Tsrc, tstride, K, g, a);
+    return xe ? threshold_fs<Fields<true, false, false>>(ctx, Tsrc, tstride, K, g, a)
+              : threshold_fs<Fields<false, false, false>>(ctx, Tsrc, tstride, K, g, a);
   }
 
   static int nblocks_threshold(bool rec)
   {
     if constexpr (kRegThr) {
-      if (!rec) return N * N / RegThr<N / 32>::RWG;
+      if (!rec) return N * N / RegThr<N / 32, 4>::RWG;  // the rows do not depend on the fields
     }
     return N * N / RowCfg<N>::ROWS;
   }
@@ -861,7 +853,8 @@ struct HiiRun {
     {
       using P = Pipe<N>;
       const bool rec = p->include_recombinations != 0;
-      const int nfield = 3 + (p->include_spin_temp ? 1 : 0) + (rec ? 1 : 0);
+      const bool xe = p->include_spin_temp != 0, wsfr = p->uvb_flag != 0 || rec;  // Fields
+      const int nfield = 2 + (wsfr ? 1 : 0) + (xe ? 1 : 0) + (rec ? 1 : 0);
       MRX_TRY(ensure_buffers(ctx, N, nfield > 4 ? nfield : 4));
       std::vector<double> R;
       const int S = ladder(p, R);
@@ -889,7 +882,6 @@ struct HiiRun {
       // inputs: deltax, stars, weighted_sfr, x_e are padded and laid out at a
       // fixed stride when staged; device pointers are used where they lie.
       const float* deltax = in[0];
-      const float* src[5] = {in[0], in[1], in[2], p->include_spin_temp ? in[3] : in[4], in[4]};
       const double box_size = p->box_size;
       // the tabulated windows (top-hat, Gaussian) of every filtered radius
       // are built on the side stream while the fields are transformed: the
@@ -938,7 +930,12 @@ struct HiiRun {
       } wait_side{ctx, use_side};
       // forward transform of every field into its U slot
       FieldTab ft{};
-      for (int f = 0; f < nfield; ++f) ft.p[f] = src[f];
+      int nf = 0;
+      ft.p[nf++] = in[0];
+      ft.p[nf++] = in[1];
+      if (wsfr) ft.p[nf++] = in[2];
+      if (xe) ft.p[nf++] = in[3];
+      if (rec) ft.p[nf++] = in[4];
       MRX_TRY(P::forward(ctx, ft, nfield, true, ctx->U, ctx->V));
       if (use_side) {
         HIP_TRY(hipStreamWaitEvent(ctx->stream, ctx->side_ev[1], 0));
@@ -952,8 +949,7 @@ struct HiiRun {
       a.redshift = p->redshift;
       a.bias = p->gamma_halo_bias;
       a.uvb = p->uvb_flag;
-      a.use_xe = p->include_spin_temp;
-      a.nfield = nfield;
+      const ThrGrids grids{deltax, ctx->state, out[0], out[1], out[2], out[3], out[4], out[5], ctx->Rtab};
       // the filtered radii go through the passes KL at a time (tabulated
       // windows; KL = 0: sharp-k, one radius per pass over its live tiles)
       // when the spectra of that many radii fit, else one at a time
@@ -983,7 +979,7 @@ struct HiiRun {
         }
         a.step = s;
         a.last = last ? 1 : 0;
-        MRX_TRY(P::threshold(ctx, Tsrc, tstride, K, deltax, out[0], out[1], out[2], out[3], out[4], out[5], rec, a));
+        MRX_TRY(P::threshold(ctx, Tsrc, tstride, K, grids, xe, wsfr, rec, a));
         s += K;
       }
       if (rec) {
@@ -2634,7 +2630,7 @@ int mrx_hii_batch_create(mrx_ctx* ctx, const mrx_hii_batch_box* boxes, int n_box
   for (auto& c : b->cohorts) {
     if (rc != MRX_OK) break;
     c.N = c.p0.grid_dim;
-    c.F = c.p0.include_spin_temp ? 4 : 3;
+    c.F = 2 + (c.p0.uvb_flag ? 1 : 0) + (c.p0.include_spin_temp ? 1 : 0);  // Fields
     c.nbox = (int)c.boxes.size();
     c.S = ladder(&c.p0, c.R);
     if (c.S < 1) rc = set_err(ctx, MRX_EINVAL, "batch: radius ladder is empty");
@@ -2702,7 +2698,7 @@ int mrx_hii_batch_describe(const mrx_hii_batch* b, char* buf, int len)
     (void)cohort_dispatch(c.N, sh);
     char tmp[256];
     snprintf(tmp, sizeof tmp, "%s{\"grid_dim\": %d, \"boxes\": %d, \"fields\": %d, \"radii\": %d, \"variant\": %d, "
-             "\"tile_width\": %d, \"radix_schedule\": %d, \"tune_ms\": [", k ? ", " : "", c.N, c.nbox, c.F, c.S,
+             "\"tile_width\": %d, \"radix_schedule\": %d, \"tune_ms\": [", k ? ", " : "", c.N, c.nbox, c.p0.include_spin_temp ? 4 : 3, c.S,
              c.variant, sh.tw, sh.sv);
     s += tmp;
     for (size_t v = 0; v < c.tune_ms.size(); ++v) {

@@ -836,8 +836,6 @@ struct StepArgs {
   int step;             // ladder index (0 = largest R)
   int last;             // unfiltered final step
   int uvb;
-  int use_xe;
-  int nfield;
   int kzlive;           // spectrum slots kz >= kzlive are zero (sharp-k)
 };
 
@@ -856,9 +854,20 @@ __device__ __forceinline__ void step_load(StepArgs& a, const StepDev* __restrict
   a.gamma_pref = d.gamma_pref;
 }
 
+// The fields a ladder transforms, in order: deltax, stars, then weighted_sfr
+// (SFR), x_e (XE) and N_rec (REC).  The weighted SFR enters only J_21 (uvb) and
+// Gamma_12 (REC): a ladder with neither leaves it out, a quarter to a third of
+// every pass, and its outputs are the same.
+template <bool XE_, bool SFR_, bool REC_>
+struct Fields {
+  static constexpr bool XE = XE_, SFR = SFR_, REC = REC_;
+  static_assert(SFR || !REC, "Gamma_12 takes the weighted SFR");
+  static constexpr int W = 2, X = 2 + SFR, R = 2 + SFR + XE;  // their places
+  static constexpr int N = 2 + SFR + XE + REC;
+};
+
 // The ladder step's test of one cell (find_HII_bubbles.c:313-443).  v: the
-// cell's clamped filtered fields (deltax, stars, weighted_sfr, then x_e when
-// there are four besides N_rec, then N_rec when REC); st: its state byte.  The
+// cell's clamped filtered fields (Fields' order); st: its state byte.  The
 // first crossing writes the cell's J_21 (and Gamma_12 with REC); on the last
 // step xh, rb and jflag (1 where the cell's J_21 is kept) are set, and zcheck
 // says whether z_at_ionization is to be set if still unset (:427-434), with
@@ -869,21 +878,20 @@ __device__ __forceinline__ void step_load(StepArgs& a, const StepDev* __restrict
 // J_21: for those (jflag = 1) the caller takes jaux from J21, read after this
 // call.  Deferring the check keeps a dependent load of z_at_ionization out of
 // every ladder step.  Returns the new state byte.
-template <int NF, bool REC>
+template <class FS>
 __device__ __forceinline__ uint32_t threshold_cell(const float* v, uint32_t st, long ir, const StepArgs& a,
                                                    float* __restrict__ J21, float* __restrict__ Gamma12,
                                                    const float* __restrict__ Rtab, float& xh, float& rb,
                                                    float& jflag, bool& zcheck, float& jaux)
 {
 #pragma clang fp contract(off)
-  constexpr bool XE = (NF - (REC ? 1 : 0)) == 4;
-  constexpr int RI = XE ? 4 : 3;  // field of N_rec
+  constexpr bool XE = FS::XE, REC = FS::REC;
   // the double quantities are formed in the branches that use them: the
   // single-precision test below decides almost every cell without them
   auto density_over_mean = [&]() { return 1.0 + (double)v[0]; };
-  auto neutral_fraction = [&]() { return XE ? 1.0 - (double)v[3] : 1.0; };
+  auto neutral_fraction = [&]() { return XE ? 1.0 - (double)v[FS::X] : 1.0; };
   // recombinations in the cell (:360-363)
-  auto rec = [&]() { return REC ? (double)v[RI] / density_over_mean() : 0.0; };
+  auto rec = [&]() { return REC ? (double)v[FS::R] / density_over_mean() : 0.0; };
   // the reference's f_coll (four roundings of its exact value), evaluated
   // where needed: the last step's partial xH and near-threshold cells
   auto f_coll = [&]() {
@@ -899,7 +907,7 @@ __device__ __forceinline__ uint32_t threshold_cell(const float* v, uint32_t st, 
     // (relative) of the exact sides, so a gap above the band's 9.5e-7 gives
     // the double test's outcome; cells inside the band take the double test
     const float kfe = (float)(a.kfc * a.eff);
-    const float lf = v[1] * kfe, rf = (XE ? 1.0f - v[3] : 1.0f) * (1.0f + v[0]);
+    const float lf = v[1] * kfe, rf = (XE ? 1.0f - v[FS::X] : 1.0f) * (1.0f + v[0]);
     if (lf > rf * 1.000001f) {
       cross = true;
       decided = true;
@@ -919,7 +927,7 @@ __device__ __forceinline__ uint32_t threshold_cell(const float* v, uint32_t st, 
   }
   // the weighted SFR is clamped here, where it is used (the clamp is
   // idempotent, so a caller may pass it clamped or not)
-  auto sfr = [&]() { return clamp_kind(v[2], 1); };
+  auto sfr = [&]() { return FS::SFR ? clamp_kind(v[FS::W], 1) : 0.0f; };
   // J_21 of the cell at this radius (:317-320, :331-337)
   auto j21_aux = [&]() { return a.uvb ? (float)((double)sfr() / a.pixel_volume * a.J21c) : 0.0f; };
   const bool never = (st == 0xFFu);
@@ -969,8 +977,8 @@ struct ThrGrids {
 // threshold_cell on each, and on the last step the output grids and the
 // cells' terms of the four block sums (xH, xH weighted by density, density,
 // J_21).  v: the cells' clamped fields.  Returns the two new state bytes.
-template <int N, int NF, bool REC>
-__device__ __forceinline__ uint32_t threshold_pair(const float (&v)[2][NF], uint32_t st_old, long row, int c0,
+template <int N, class FS>
+__device__ __forceinline__ uint32_t threshold_pair(const float (&v)[2][FS::N], uint32_t st_old, long row, int c0,
                                                    const StepArgs& a, const ThrGrids& g, double (&sum)[4])
 {
 #pragma clang fp contract(off)
@@ -982,7 +990,7 @@ __device__ __forceinline__ uint32_t threshold_pair(const float (&v)[2][NF], uint
   for (int e = 0; e < 2; ++e) {
     xh2[e] = rb2[e] = j2[e] = 0.0f;
     const uint32_t st = (st_old >> (8 * e)) & 0xFFu;
-    const uint32_t sn = threshold_cell<NF, REC>(v[e], st, ir0 + e, a, g.J21, g.Gamma12, g.Rtab, xh2[e], rb2[e], j2[e],
+    const uint32_t sn = threshold_cell<FS>(v[e], st, ir0 + e, a, g.J21, g.Gamma12, g.Rtab, xh2[e], rb2[e], j2[e],
                                                 zc2[e], ja2[e]);
     st_new = (st_new & ~(0xFFu << (8 * e))) | (sn << (8 * e));
   }
@@ -1022,10 +1030,10 @@ __device__ __forceinline__ uint32_t threshold_pair(const float (&v)[2][NF], uint
 
 // The clamps of :272-311 by field: deltax, x_e, the rest (stars, N_rec); the
 // weighted SFR is clamped in threshold_cell, at its uses.
-template <bool XE>
+template <class FS>
 __device__ __forceinline__ float clamp_field(float v, int f)
 {
-  return clamp_kind(v, (f == 0) ? 0 : (f == 2 ? -1 : ((XE && f == 3) ? 2 : 1)));
+  return clamp_kind(v, (f == 0) ? 0 : ((FS::SFR && f == FS::W) ? -1 : ((FS::XE && f == FS::X) ? 2 : 1)));
 }
 
 // waves per SIMD the threshold kernels are held to: 128 VGPRs hold three or
@@ -1038,10 +1046,8 @@ constexpr int thr_waves(int nf) { return nf == 5 ? 3 : 4; }
 // Per-cell state between launches is one byte (0xFF = never crossed, else the
 // step of the latest crossing), held in registers from step to step of a
 // launch; xH, r_bubble and the J_21 zeros are written once, on the last step.
-// Fields in T: deltax, stars, weighted_sfr, then x_e when XE (NF - REC = 4),
-// then N_rec when REC (inhomogeneous recombinations); step k's at T + k
-// kstride.  j21 (or null): the box's own J_21 constants by step.
-template <int N, int NF, bool REC>
+// Step k's fields (FS) at T + k kstride.  j21 (or null): the box's own J_21 constants by step.
+template <int N, class FS>
 __device__ __forceinline__ void c2r_threshold_rows(const float2* __restrict__ T, long fstride, long kstride, int K,
                                                    const float2* __restrict__ twN,
                                                    const StepDev* __restrict__ steps, const double* __restrict__ j21,
@@ -1049,9 +1055,7 @@ __device__ __forceinline__ void c2r_threshold_rows(const float2* __restrict__ T,
 {
   using C = RowCfg<N>;
   constexpr int NH = C::NH, ROWS = C::ROWS, NT = C::NT, NBL = C::NBL, RL = C::RL;
-  constexpr int P = NF * ROWS;
-  constexpr bool XE = (NF - (REC ? 1 : 0)) == 4;
-  static_assert(NF - (REC ? 1 : 0) == 3 || NF - (REC ? 1 : 0) == 4, "three or four fields besides N_rec");
+  constexpr int NF = FS::N, P = NF * ROWS;
   __shared__ float2 s[row_lds<N>(P)];
   __shared__ float2 tw[N];
   __shared__ double red[4 * NT / 64];
@@ -1091,10 +1095,10 @@ __device__ __forceinline__ void c2r_threshold_rows(const float2* __restrict__ T,
       float c[2][NF];
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
-        c[0][f] = clamp_field<XE>(v[f].x, f);
-        c[1][f] = clamp_field<XE>(v[f].y, f);
+        c[0][f] = clamp_field<FS>(v[f].x, f);
+        c[1][f] = clamp_field<FS>(v[f].y, f);
       }
-      st[m] = threshold_pair<N, NF, REC>(c, st[m], row0 + pair_row(tid, m), 2 * pair_n(tid, m), a, g, sum);
+      st[m] = threshold_pair<N, FS>(c, st[m], row0 + pair_row(tid, m), 2 * pair_n(tid, m), a, g, sum);
     };
     if constexpr (C::kViaLds) {
       rows_last_lds<N, P>(s, tw, tid);
@@ -1134,16 +1138,16 @@ __device__ __forceinline__ void c2r_threshold_rows(const float2* __restrict__ T,
 }
 
 // The fused z pass + threshold with the row transforms in registers, for
-// rows of NH = 16 A complex (A = 16: 512^3, A = 8: 256^3) and three or four
+// rows of NH = 16 A complex (A = 16: 512^3, A = 8: 256^3) and two to four
 // fields (no N_rec).  A field's packed row is held by A lanes, lane t holding
 // points t + A m, m < 16.  The C2R untwist pairs point k with NH - k, held by
 // lane (A - t) mod A (a lane shuffle); the length-NH inverse transform is a
 // 16-point DFT of each lane's registers, a twiddle, one exchange through LDS,
 // and A-point DFTs, after which lane t holds z[t + A j], j < 16, the real
-// cells 2n and 2n + 1 of n = t + A j.  A wave holds four field groups of A
-// lanes per row (64 / 4A rows); the fields of a cell meet through LDS: lane
-// (g, t) tests the cells of n = t + A j, j in [4g, 4g + 4).  Three barriers
-// per workgroup and two LDS round trips, where staging the rows in LDS for a
+// cells 2n and 2n + 1 of n = t + A j.  A workgroup is one wave per field, its
+// groups of A lanes dealt to (row, field) pairs, so no lane idles with two or
+// three fields; the fields of a cell meet through LDS, and the points j of a
+// row are split over its lane groups.  Three barriers per workgroup and two LDS round trips, where staging the rows in LDS for a
 // Stockham transform takes eight and five.  Per cell the test is
 // threshold_cell's, as in c2r_threshold_rows, one step per launch (a loop over
 // two steps spilled at four waves per SIMD: 541 -> 560 us per step at 512^3).
@@ -1232,48 +1236,51 @@ __global__ __launch_bounds__(256) void k_c2r_z_reg(const float2* __restrict__ in
   if (pitch > N && t == 0) *reinterpret_cast<float2*>(o + N) = make_float2(0.0f, 0.0f);
 }
 
-template <int A>
+template <int A, int NF>
 struct RegThr {
   static constexpr int NH = 16 * A, N = 2 * NH;
-  static constexpr int RW = 64 / (4 * A);  // rows per wave
-  static constexpr int RWG = 4 * RW;        // rows per 256-thread workgroup
-  static constexpr int XP = A + 1;          // LDS pitch of an exchange row
+  static constexpr int NT = 64 * NF;                 // one wave per field's worth of rows
+  static constexpr int RWG = NT / (A * NF);          // rows per workgroup
+  static constexpr int XP = A + 1;                   // LDS pitch of an exchange row
+  // points j of a row each of its NF lane groups tests: 16 / NF, rounded up
+  static constexpr int QN = (16 + NF - 1) / NF;
+  static constexpr int first(int f) { return (16 * f + NF - 1) / NF; }
   static_assert(A == 8 || A == 16, "rows of 128 or 256 complex");
 };
 
-template <int A, int NF>
-__global__ __launch_bounds__(256) void k_c2r_threshold_reg(const float2* __restrict__ T, long fstride,
+template <int A, class FS>
+__global__ __launch_bounds__((RegThr<A, FS::N>::NT)) void k_c2r_threshold_reg(const float2* __restrict__ T, long fstride,
                                                            const float2* __restrict__ twN,
                                                            const StepDev* __restrict__ steps, ThrGrids g,
                                                            double* __restrict__ partials, StepArgs a)
 {
-  using C = RegThr<A>;
-  constexpr int NH = C::NH, N = C::N, RW = C::RW, RWG = C::RWG, XP = C::XP;
-  static_assert(NF == 3 || NF == 4, "three or four fields");
-  constexpr bool XE = NF == 4;
+  constexpr int NF = FS::N;
+  using C = RegThr<A, NF>;
+  constexpr int NH = C::NH, N = C::N, NT = C::NT, RWG = C::RWG, XP = C::XP, QN = C::QN;
   __shared__ float2 tw[N];
-  __shared__ float2 xb[RWG][4][16 * XP];  // [row of the workgroup][field group][16 x A, pitch XP]
-  __shared__ double red[4 * 256 / 64];
+  __shared__ float2 xb[RWG][NF][16 * XP];  // [row of the workgroup][field][16 x A, pitch XP]
+  __shared__ double red[4 * NT / 64];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int t = lane % A, fg = (lane / A) % 4;
-  const int rl = (tid >> 6) * RW + lane / (4 * A);  // row within the workgroup
-  const long row = (long)blockIdx.x * RWG + rl;     // x N + y
+  const int t = lane % A, slot = tid / A;
+  const int fg = slot % NF, rl = slot / NF;      // field; row within the workgroup
+  const long row = (long)blockIdx.x * RWG + rl;  // x N + y
+  // this lane's cells: n = t + A j, j in [j0, j0 + nq)
+  const int j0 = C::first(fg), nq = C::first(fg + 1) - j0;
   step_load(a, steps);
-  for (int i = tid; i < N; i += 256) tw[i] = twN[i];
-  // the ladder state of this lane's cells, two bytes at cell 2n, n = t + A (4 fg + q)
-  uint32_t st_pre[4];
+  for (int i = tid; i < N; i += NT) tw[i] = twN[i];
+  // their ladder state, two bytes at cell 2n
+  uint32_t st_pre[QN];
 #pragma unroll
-  for (int q = 0; q < 4; ++q)
-    st_pre[q] = (a.step == 0) ? 0xFFFFu
-                              : *reinterpret_cast<const uint16_t*>(g.state + row * N + 2 * (t + A * (4 * fg + q)));
-  // field fg's row; the fourth group carries zeros when there are three fields
+  for (int q = 0; q < QN; ++q)
+    st_pre[q] = (a.step == 0 || q >= nq) ? 0xFFFFu
+                                         : *reinterpret_cast<const uint16_t*>(g.state + row * N + 2 * (t + A * (j0 + q)));
+  // field fg's row
   float2 x[16];
   {
-    const float2* src = T + (long)(fg < NF ? fg : 0) * fstride + row * NH + t;
+    const float2* src = T + (long)fg * fstride + row * NH + t;
 #pragma unroll
-    for (int m = 0; m < 16; ++m)
-      x[m] = (fg < NF && t + A * m < a.kzlive) ? src[A * m] : make_float2(0.0f, 0.0f);
+    for (int m = 0; m < 16; ++m) x[m] = (t + A * m < a.kzlive) ? src[A * m] : make_float2(0.0f, 0.0f);
   }
   __syncthreads();  // the twiddle table
   float2* xr = xb[rl][fg];
@@ -1283,24 +1290,25 @@ __global__ __launch_bounds__(256) void k_c2r_threshold_reg(const float2* __restr
 #pragma unroll
   for (int j = 0; j < 16; ++j) xr[j * XP + t] = z[j];
   __syncthreads();
-  // the cells n = t + A j, j = 4 fg + q: all fields of the row from LDS
+  // all fields of the cells from LDS
   double sum[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int j = 4 * fg + q;
+  for (int q = 0; q < QN; ++q) {
+    if (16 % NF != 0 && q >= nq) break;
+    const int j = j0 + q;
     const int c0 = 2 * (t + A * j);  // first of the two cells
     float c[2][NF];
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
       const float2 p = xb[rl][f][j * XP + t];
-      c[0][f] = clamp_field<XE>(p.x, f);
-      c[1][f] = clamp_field<XE>(p.y, f);
+      c[0][f] = clamp_field<FS>(p.x, f);
+      c[1][f] = clamp_field<FS>(p.y, f);
     }
-    const uint32_t st = threshold_pair<N, NF, false>(c, st_pre[q], row, c0, a, g, sum);
+    const uint32_t st = threshold_pair<N, FS>(c, st_pre[q], row, c0, a, g, sum);
     if (st != st_pre[q] || a.step == 0) *reinterpret_cast<uint16_t*>(g.state + row * N + c0) = (uint16_t)st;
   }
   if (a.last) {
-    block_sum_n<256, 4>(sum, red);
+    block_sum_n<NT, 4>(sum, red);
     if (tid == 0) {
       double* p = partials + (long)blockIdx.x * 4;
 #pragma unroll
@@ -1309,14 +1317,14 @@ __global__ __launch_bounds__(256) void k_c2r_threshold_reg(const float2* __restr
   }
 }
 
-template <int N, int NF, bool REC = false>
-__global__ __launch_bounds__(RowCfg<N>::NT, thr_waves(NF)) void k_c2r_threshold(const float2* __restrict__ T, long fstride,
+template <int N, class FS>
+__global__ __launch_bounds__(RowCfg<N>::NT, thr_waves(FS::N)) void k_c2r_threshold(const float2* __restrict__ T, long fstride,
                                                                  long kstride, int K,
                                                                  const float2* __restrict__ twN,
                                                                  const StepDev* __restrict__ steps, ThrGrids g,
                                                                  double* __restrict__ partials, StepArgs a)
 {
-  c2r_threshold_rows<N, NF, REC>(T, fstride, kstride, K, twN, steps, nullptr, g, partials, a);
+  c2r_threshold_rows<N, FS>(T, fstride, kstride, K, twN, steps, nullptr, g, partials, a);
 }
 
 // Per-box grids and scalars of a batch (device array, one entry per box).
@@ -1335,8 +1343,8 @@ struct BoxDev {
 // The ladder step of every box of a cohort: blockIdx.y is the box.  T holds
 // nfield spectra per box (box stride bstride); state and partials are
 // contiguous per box; J21c_tab[box * nstep + step] is the box's J_21 constant.
-template <int N, int NF>
-__global__ __launch_bounds__(RowCfg<N>::NT, thr_waves(NF)) void k_c2r_threshold_batch(
+template <int N, class FS>
+__global__ __launch_bounds__(RowCfg<N>::NT, thr_waves(FS::N)) void k_c2r_threshold_batch(
   const float2* __restrict__ T, long fstride, long bstride, const float2* __restrict__ twN,
   const BoxDev* __restrict__ boxes, uint8_t* __restrict__ state, const float* __restrict__ Rtab,
   const StepDev* __restrict__ steps, const double* __restrict__ J21c_tab, int nstep, double* __restrict__ partials,
@@ -1349,7 +1357,7 @@ __global__ __launch_bounds__(RowCfg<N>::NT, thr_waves(NF)) void k_c2r_threshold_
   a.bias = bx.bias;
   const ThrGrids g{bx.deltax, state + (long)box * N * N * N, bx.xH, bx.r_bubble, bx.J21, bx.z_in, bx.J21_ion, nullptr,
                    Rtab};
-  c2r_threshold_rows<N, NF, false>(T + box * bstride, fstride, 0, 1, twN, steps, J21c_tab + (long)box * nstep, g,
+  c2r_threshold_rows<N, FS>(T + box * bstride, fstride, 0, 1, twN, steps, J21c_tab + (long)box * nstep, g,
                                    partials + (long)box * gridDim.x * 4, a);
 }
 

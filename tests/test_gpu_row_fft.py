@@ -57,3 +57,21 @@ def test_ladder_rows_against_the_oracle(ctx, N, spin, rec, ftype):
     assert crossed.sum() > 50
     close(g["Gamma12"], o["Gamma12"], "Gamma12", crossed)
     close(g["N_rec"][:, :, :N], o["N_rec"][:, :, :N], "N_rec", ~flips)
+
+
+@pytest.mark.parametrize("N,spin,ftype", [(32, 0, 0), (96, 1, 2), (256, 0, 1), (256, 1, 0)])
+def test_ladder_without_the_uvb_leaves_the_sfr_out(ctx, N, spin, ftype):
+    """The weighted SFR only feeds J_21: without the UVB the ladder transforms one field less
+    (two or three, also where rows of 256^3 go through registers), every other output the same."""
+    print(f"N={N} spin={spin} filter={ftype}", flush=True)
+    d, s, w = synth.snapshot_inputs(N, 80 + N)
+    xe = None
+    if spin:
+        xe = synth.to_padded(np.random.default_rng(5).uniform(0.0, 0.2, (N, N, N)).astype(np.float32))
+    r = [reion.find_hii_bubbles(ctx, P.hii_params(N, 0.8 * N, 8.0, filter_type=ftype, efficiency=30.0, uvb_flag=u,
+                                                  include_spin_temp=spin), d, s, w, x_e=xe) for u in (1, 0)]
+    for k in ("xH", "r_bubble", "z_at_ionization"):
+        assert np.array_equal(r[0][k], r[1][k]), k
+    for k in ("volume_weighted_global_xH", "mass_weighted_global_xH", "n_radii"):
+        assert r[0][k] == r[1][k], k
+    assert (r[0]["r_bubble"] > 0).any()
