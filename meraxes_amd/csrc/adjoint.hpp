@@ -223,25 +223,30 @@ __global__ __launch_bounds__(kNT) void k_snapshot_adjoint_cell(
   }
 }
 
-// Gradient of shell ct, dL/d(shell_ct) on the padded grid: the raw sums'
-// adjoints times their coefficients at the cell's x_e, where the forward's
-// max(v, 0) clamp passed the value (v > 0; the derivative is taken as 0 at
-// v = 0).  `unclamped`, when given, is the padded grid v itself (the
-// unfiltered shell 0 is the working grid, whose zeros the transform's
-// round-off would otherwise make positive or negative at random).
+// Gradients of n <= G shells from ct0 on, dL/d(shell) on padded grids (stride
+// ostride): the raw sums' adjoints times their coefficients at the cell's x_e,
+// where the forward's max(v, 0) clamp passed the value (v > 0; the derivative
+// is taken as 0 at v = 0).  `unclamped`, when given (n = 1), is the padded grid v
+// itself (the unfiltered shell 0 is the working grid, whose zeros the
+// transform's round-off would otherwise make positive or negative at random).
+// Bound by memory: per cell 32 bytes of gS and 8 per shell, so the shells of a
+// group share one read of gS (one shell per launch read 1.9 of its 2.8 ms at
+// 192^3 for it).
+template <int G>
 __global__ __launch_bounds__(kNT) void k_ts_shell_grad(const TsDev* __restrict__ tg, const float* __restrict__ shells,
                                                       const float* __restrict__ xe_prev,
-                                                      const double* __restrict__ gS, float* __restrict__ out, int ct,
-                                                      int N, const float* __restrict__ unclamped)
+                                                      const double* __restrict__ gS, float* __restrict__ out,
+                                                      long ostride, int ct0, int n, int N,
+                                                      const float* __restrict__ unclamped)
 {
-  // this shell's column of the six x_e tables
-  __shared__ double col[6][kNXHII];
+  // these shells' columns of the six x_e tables
+  __shared__ double col[G][6][kNXHII];
   const TsDev& t = *tg;
-  if (threadIdx.x < 6 * kNXHII) {
-    const int tb = threadIdx.x / kNXHII, x = threadIdx.x % kNXHII;
+  for (int e = threadIdx.x; e < n * 6 * kNXHII; e += kNT) {
+    const int g = e / (6 * kNXHII), tb = e / kNXHII % 6, x = e % kNXHII;
     const double(*src)[kTsMaxSteps] =
       tb == 0 ? t.fheat : tb == 1 ? t.fion : tb == 2 ? t.flya : tb == 3 ? t.sheat : tb == 4 ? t.sion : t.slya;
-    col[tb][x] = src[x][ct];
+    col[g][tb][x] = src[x][ct0 + g];
   }
   __syncthreads();
   const long ncell = (long)N * N * N;
@@ -250,21 +255,30 @@ __global__ __launch_bounds__(kNT) void k_ts_shell_grad(const TsDev* __restrict__
   const long r = i / N;
   const int z = (int)(i % N);
   const long ip = r * (N + 2) + z;
-  const float sv = shells[(long)ct * ncell + i];
-  double g = 0.0;
-  if ((unclamped ? unclamped[ip] : sv) > 0.0f) {
-    const XeBracket br = xe_bracket(t, xe_prev[ip]);
-    double dd;
-    const double fh = interp(col[0][br.lo], col[3][br.lo], br, &dd);
-    const double fi = interp(col[1][br.lo], col[4][br.lo], br, &dd);
-    const double fl = interp(col[2][br.lo], col[5][br.lo], br, &dd);
-    const double dSFR = t.sfr_factor;
-    const double w = t.dt_dzpp[ct] * t.dzpp[ct] * t.zpp_pow[ct];
-    const double wl = t.P2 * t.zpp1[ct] * t.sum_lyn[ct] * t.dt_dzpp[ct] * t.dzpp[ct];
-    g = dSFR * (gS[i] * w * fh + gS[ncell + i] * w * fi + gS[2 * ncell + i] * w * fl + gS[3 * ncell + i] * wl);
+  float sv[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) sv[g] = g < n ? shells[(long)(ct0 + g) * ncell + i] : 0.0f;
+  const double s0 = gS[i], s1 = gS[ncell + i], s2 = gS[2 * ncell + i], s3 = gS[3 * ncell + i];
+  const XeBracket br = xe_bracket(t, xe_prev[ip]);
+#pragma unroll
+  for (int k = 0; k < G; ++k) {
+    if (k >= n) break;
+    const int ct = ct0 + k;
+    double g = 0.0;
+    if ((unclamped ? unclamped[ip] : sv[k]) > 0.0f) {
+      double dd;
+      const double fh = interp(col[k][0][br.lo], col[k][3][br.lo], br, &dd);
+      const double fi = interp(col[k][1][br.lo], col[k][4][br.lo], br, &dd);
+      const double fl = interp(col[k][2][br.lo], col[k][5][br.lo], br, &dd);
+      const double dSFR = t.sfr_factor;
+      const double w = t.dt_dzpp[ct] * t.dzpp[ct] * t.zpp_pow[ct];
+      const double wl = t.P2 * t.zpp1[ct] * t.sum_lyn[ct] * t.dt_dzpp[ct] * t.dzpp[ct];
+      g = dSFR * (s0 * w * fh + s1 * w * fi + s2 * w * fl + s3 * wl);
+    }
+    float* o = out + k * ostride;
+    o[ip] = (float)g;
+    if (z == N - 1) o[ip + 1] = o[ip + 2] = 0.0f;
   }
-  out[ip] = (float)g;
-  if (z == N - 1) out[ip + 1] = out[ip + 2] = 0.0f;
 }
 
 // The shell tables' dependence on the two grid means they are built from

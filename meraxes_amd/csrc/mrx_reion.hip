@@ -549,6 +549,39 @@ struct Pipe {
     return check_launch(ctx, "k_unpack_dc");
   }
 
+  // Adds the sharp-k filtered spectra of nf padded fields (in, at stride npad)
+  // to acc, or stores them when init (k_colpass_x_accum); ws by increasing
+  // radius, every ball inside ws[0]'s and that smaller than the grid.  S: nf
+  // spectra of scratch.
+  static int forward_sharpk_sum(mrx_ctx* ctx, const float* in, int nf, const WinArgs* ws, float2* S, float2* acc,
+                                bool init)
+  {
+    constexpr int TW = Cfg<N>::TW;
+    FieldTab t{};
+    SharpkTab k{};
+    for (int f = 0; f < nf; ++f) {
+      t.p[f] = in + (size_t)f * npad(N);
+      k.R[f] = ws[f].R;
+      k.nmax[f] = sharpk_nmax(ws[f], N);
+    }
+    const int lmax = k.nmax[0], nkzb = std::min(NH / TW, lmax / TW + 1);
+    {
+      PROF("r2c_z");
+      k_r2c_z<N><<<dim3(N * N / Cfg<N>::RZ, nf), kNT, 0, ctx->stream>>>(t, S, ctx->tw, nc);
+    }
+    MRX_TRY(check_launch(ctx, "k_r2c_z"));
+    {
+      PROF("colpass_y_fwd");
+      k_colpass_sub<N, false><<<dim3(N * nkzb, nf), Cfg<N>::COL_NT, 0, ctx->stream>>>(S, ctx->tw, nc, (long)N * NH,
+                                                                                      NH, 0.0, nkzb, -1);
+    }
+    MRX_TRY(check_launch(ctx, "k_colpass_sub y"));
+    PROF("colpass_x_accum");
+    k_colpass_x_accum<N><<<std::min(N, 2 * lmax + 1) * nkzb, TileMap<N, TW>::NT, 0, ctx->stream>>>(
+      S, acc, ctx->tw, nc, (float)std::pow((double)N, 3), ws[0].delta_k, k, nf, nkzb, lmax, init ? 1 : 0);
+    return check_launch(ctx, "k_colpass_x_accum");
+  }
+
   // U (+V) filtered at R -> T, then inverse y pass; T then holds the packed
   // spectra of the filtered fields with x and y already transformed, in kz
   // slots below kzlive (the slots above are zero and left unwritten: a
@@ -705,6 +738,11 @@ struct Pipe {
     return N * N / RowCfg<N>::ROWS;
   }
 
+  static int unpack_dc(mrx_ctx* ctx, float2* U, float2* V)
+  {
+    k_unpack_dc<N><<<dim3((N * N + 255) / 256, 1), 256, 0, ctx->stream>>>(U, V, nc, (long)N * N);
+    return check_launch(ctx, "k_unpack_dc");
+  }
   static int pack_herm(mrx_ctx* ctx, const float2* H, float2* U)
   {
     const long n = nc;
@@ -1832,49 +1870,92 @@ struct SnapAdj {
       if (g_sfr) HIP_TRY(hipMemsetAsync(g_sfr, 0, sizeof(float) * np, ctx->stream));
       if (g_hist && tp) HIP_TRY(hipMemsetAsync(g_hist, 0, sizeof(float) * np * (size_t)tp->n_history, ctx->stream));
       if (!shells || !g_sfr) return finish_means();
-      MRX_TRY(ensure_buf(ctx, ctx->adj_work, ctx->adj_work_cap, 2 * np));
+      // Shells G at a time: their gradients share one read of the shell sums'
+      // adjoints, and those that reach the same state of the working grid (no
+      // operations between them) one inverse transform of the sum of their
+      // filtered spectra.  G padded grids and spectra, the summed spectrum and
+      // one grid: at most 12 GiB, two shells at least.
+      const size_t per = np + (size_t)ncell;
+      const int G = (int)std::max<size_t>(2, std::min<size_t>(kMaxFields, ((size_t)12 << 30) / (sizeof(float) * per)));
+      MRX_TRY(ensure_buf(ctx, ctx->adj_work, ctx->adj_work_cap, G * per + (size_t)ncell + np));
       float* gshell = ctx->adj_work;
-      float* tmp = ctx->adj_work + np;
+      float2* spec = reinterpret_cast<float2*>(gshell + G * np);
+      float2* acc = spec + (size_t)G * P::nc;
+      float* tmp = reinterpret_cast<float*>(acc + P::nc);
       const long half = (long)N * N * (N / 2 + 1);
-      for (int ct = s->nsteps - 1; ct >= 0; --ct) {
-        const float* unclamped = nullptr;
-        if (ct == 0) {  // shell 0 is the working grid after its operations: rebuild it
-          HIP_TRY(hipMemcpyAsync(tmp, sfr, sizeof(float) * np, hipMemcpyDeviceToDevice, ctx->stream));
-          for (int k = 0; k < s->n_ops[0]; ++k) {
-            const mrx_sfr_op& o = s->ops[0][k];
-            const long n = (o.kind <= 1) ? half : ncell;
-            const float* hs = (o.kind >= 2) ? hist + (size_t)o.slot * np : nullptr;
-            k_sfr_op<<<(unsigned)((n + 255) / 256), 256, 0, ctx->stream>>>(tmp, hs, o.kind, o.weight,
-                                                                          (float)o.weight, N, half);
-            MRX_TRY(check_launch(ctx, "k_sfr_op"));
-          }
-          unclamped = tmp;
+      auto shell_grad = [&](int ct, int n, const float* unclamped) -> int {
+        PROF("adjoint_shell_grad");
+        if (n == 1)
+          k_ts_shell_grad<1><<<nbc, kNT, 0, ctx->stream>>>(ctx->ts_dev, ctx->ts_shells, xe_prev, ctx->adj_gS, gshell,
+                                                           (long)np, ct, 1, N, unclamped);
+        else
+          k_ts_shell_grad<kMaxFields><<<nbc, kNT, 0, ctx->stream>>>(ctx->ts_dev, ctx->ts_shells, xe_prev, ctx->adj_gS,
+                                                                    gshell, (long)np, ct, n, N, nullptr);
+        return check_launch(ctx, "k_ts_shell_grad");
+      };
+      auto add_sfr = [&](const float* x) -> int {
+        k_axpy<<<(unsigned)((np + 255) / 256), 256, 0, ctx->stream>>>(g_sfr, x, (long)np);
+        return check_launch(ctx, "k_axpy");
+      };
+      auto shell_win = [&](int ct) { return win_args(tp->box_size, (float)s->R[ct], tp->heating_filter_type, 1); };
+      for (int hi = s->nsteps - 1; hi >= 0;) {
+        // the shells lo .. hi see the working grid as the operations of lo left it
+        int lo = hi;
+        while (lo > 0 && s->n_ops[lo] == 0) --lo;
+        // sharp-k shells whose balls of modes are smaller than the grid (the
+        // radii increase, so these are the last of the run) are summed
+        int first_sum = hi + 1;
+        if (tp->heating_filter_type == MRX_FILTER_SHARPK)
+          while (first_sum > std::max(lo, 1) && sharpk_nmax(shell_win(first_sum - 1), N) < N / 2) --first_sum;
+        for (int ct = first_sum; ct <= hi; ct += G) {
+          const int n = std::min(G, hi + 1 - ct);
+          WinArgs ws[kMaxFields];
+          for (int k = 0; k < n; ++k) ws[k] = shell_win(ct + k);
+          MRX_TRY(shell_grad(ct, n, nullptr));
+          MRX_TRY(P::forward_sharpk_sum(ctx, gshell, n, ws, spec, acc, ct == first_sum));
         }
-        {
-          PROF("adjoint_shell_grad");
-          k_ts_shell_grad<<<nbc, kNT, 0, ctx->stream>>>(ctx->ts_dev, ctx->ts_shells, xe_prev, ctx->adj_gS, gshell, ct,
-                                                        N, unclamped);
-        }
-        MRX_TRY(check_launch(ctx, "k_ts_shell_grad"));
-        const float* add = gshell;
-        if (ct > 0) {  // shell 0 is the unfiltered grid
-          MRX_TRY(P::forward(ctx, gshell, true, ctx->U, ctx->V, true));
-          const WinArgs w = win_args(tp->box_size, (float)s->R[ct], tp->heating_filter_type, 1);
+        if (first_sum <= hi) {
+          // acc lies inside the first shell's ball: its window keeps every mode
+          MRX_TRY(P::unpack_dc(ctx, acc, ctx->V));
           int kzlive;
-          MRX_TRY(P::inverse_xy(ctx, ctx->U, ctx->V, ctx->T, 1, w, kzlive));
+          MRX_TRY(P::inverse_xy(ctx, acc, ctx->V, ctx->T, 1, shell_win(first_sum), kzlive));
           MRX_TRY(P::c2r_z(ctx, ctx->T, tmp, 1, -1, N + 2, kzlive));
-          add = tmp;
+          MRX_TRY(add_sfr(tmp));
         }
-        k_axpy<<<(unsigned)((np + 255) / 256), 256, 0, ctx->stream>>>(g_sfr, add, (long)np);
-        MRX_TRY(check_launch(ctx, "k_axpy"));
-        for (int k = s->n_ops[ct] - 1; k >= 0; --k) {
-          const mrx_sfr_op& o = s->ops[ct][k];
+        for (int ct = first_sum - 1; ct >= lo; --ct) {
+          const float* unclamped = nullptr;
+          if (ct == 0) {  // shell 0 is the working grid after its operations: rebuild it
+            HIP_TRY(hipMemcpyAsync(tmp, sfr, sizeof(float) * np, hipMemcpyDeviceToDevice, ctx->stream));
+            for (int k = 0; k < s->n_ops[0]; ++k) {
+              const mrx_sfr_op& o = s->ops[0][k];
+              const long n = (o.kind <= 1) ? half : ncell;
+              const float* hs = (o.kind >= 2) ? hist + (size_t)o.slot * np : nullptr;
+              k_sfr_op<<<(unsigned)((n + 255) / 256), 256, 0, ctx->stream>>>(tmp, hs, o.kind, o.weight,
+                                                                            (float)o.weight, N, half);
+              MRX_TRY(check_launch(ctx, "k_sfr_op"));
+            }
+            unclamped = tmp;
+          }
+          MRX_TRY(shell_grad(ct, 1, unclamped));
+          const float* add = gshell;
+          if (ct > 0) {  // shell 0 is the unfiltered grid
+            MRX_TRY(P::forward(ctx, gshell, true, ctx->U, ctx->V, true));
+            int kzlive;
+            MRX_TRY(P::inverse_xy(ctx, ctx->U, ctx->V, ctx->T, 1, shell_win(ct), kzlive));
+            MRX_TRY(P::c2r_z(ctx, ctx->T, tmp, 1, -1, N + 2, kzlive));
+            add = tmp;
+          }
+          MRX_TRY(add_sfr(add));
+        }
+        for (int k = s->n_ops[lo] - 1; k >= 0; --k) {
+          const mrx_sfr_op& o = s->ops[lo][k];
           const long n = (o.kind <= 1) ? half : ncell;
           float* gh = (o.kind >= 2 && g_hist && o.slot < nslot) ? g_hist + (size_t)o.slot * np : nullptr;
           k_sfr_op_adjoint<<<(unsigned)((n + 255) / 256), 256, 0, ctx->stream>>>(g_sfr, gh, o.kind, o.weight,
                                                                                  (float)o.weight, N, half);
           MRX_TRY(check_launch(ctx, "k_sfr_op_adjoint"));
         }
+        hi = lo - 1;
       }
       return finish_means();
     }

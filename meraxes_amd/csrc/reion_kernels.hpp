@@ -195,9 +195,10 @@ __device__ __forceinline__ void r2c_z_tile(const float* __restrict__ in, float2*
   }
 }
 
-// The input grids of up to five fields (separate allocations), by value.
+// The input grids of up to kMaxFields fields (separate allocations), by value.
+constexpr int kMaxFields = 8;
 struct FieldTab {
-  const float* p[5];
+  const float* p[kMaxFields];
 };
 
 // blockIdx.y selects the field (outputs at stride out_fstride)
@@ -369,6 +370,64 @@ __global__ __launch_bounds__((TileMap<N, TW>::NT), 4) void k_colpass_sub(float2*
   }
 #pragma unroll
   for (int i = 0; i < EPT; ++i) g[(unsigned)(i * RPI) * rs] = r[i];
+}
+
+// Forward x pass of nf spectra (stride fstride), each cut by its own sharp-k
+// window and scaled by 1 / fdiv, summed into `acc` (init: stored, else added):
+// since a filter is its own adjoint and linear, the spectra of several filtered
+// fields that end in the same grid need one inverse transform.  Grid: lines |ky|
+// <= lmax x kz blocks below nkzb (k_colpass_sub's order); R and nmax are per
+// field, nmax[f] <= lmax.  Points |kx| > lmax of acc are not written.
+struct SharpkTab {
+  float R[kMaxFields];
+  int nmax[kMaxFields];
+};
+template <int N, int TW = Cfg<N>::TW>
+__global__ __launch_bounds__((TileMap<N, TW>::NT)) void k_colpass_x_accum(const float2* __restrict__ data,
+                                                                      float2* __restrict__ acc,
+                                                                      const float2* __restrict__ twN, long fstride,
+                                                                      float fdiv, float delta_k, SharpkTab tab, int nf,
+                                                                      int nkzb, int lmax, int init)
+{
+  using M = TileMap<N, TW>;
+  constexpr int NT = M::NT, SP = M::SP, RPI = M::RPI, EPT = M::EPT;
+  constexpr int NH = N / 2;
+  constexpr unsigned rs = (unsigned)N * NH;
+  __shared__ float2 s[N * SP];
+  __shared__ float2 tw[N];
+  const int tid = threadIdx.x;
+  const int c = tid % TW, n0 = tid / TW;
+  const int j = blockIdx.x / nkzb, b = blockIdx.x % nkzb;
+  const int ky = (j <= lmax) ? j : N - (min(N, 2 * lmax + 1) - j);
+  const int aky = ky <= NH ? ky : N - ky;
+  const long base = (long)ky * NH + (long)b * TW + (unsigned)n0 * rs + c;
+  for (int i = tid; i < N; i += NT) tw[i] = twN[i];
+  float2 sum[EPT];
+#pragma unroll
+  for (int i = 0; i < EPT; ++i) sum[i] = make_float2(0.0f, 0.0f);
+  for (int f = 0; f < nf; ++f) {
+    if (aky > tab.nmax[f] || b * TW > tab.nmax[f]) continue;  // outside this field's ball
+    const float2* g = data + f * fstride + base;
+    float2 r[EPT];
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) r[i] = g[(unsigned)(i * RPI) * rs];
+    __syncthreads();  // the twiddle table; the last field's reads of s
+    fft_tile_reg<N, TW, NT, false, SP>(r, s, tw, tid);
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) {
+      const int n = n0 + i * RPI;
+      const int an = n <= NH ? n : N - n;
+      if (an <= tab.nmax[f] && sharpk_window(k_magnitude(an, aky, b * TW + c, N, delta_k), tab.R[f]) != 0.0f)
+        sum[i] = cadd(sum[i], make_float2(r[i].x / fdiv, r[i].y / fdiv));
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < EPT; ++i) {
+    const int n = n0 + i * RPI;
+    if (min(n, N - n) > lmax) continue;
+    float2* o = acc + base + (unsigned)(i * RPI) * rs;
+    *o = init ? sum[i] : cadd(*o, sum[i]);
+  }
 }
 
 // Window table of one radius: W depends on (|nx|, |ny|, nz) only, because
