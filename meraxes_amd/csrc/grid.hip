@@ -4,12 +4,14 @@
 // The reference walks the galaxies in order and adds each one's value to a
 // float buffer cell, `buffer[ind] += v` with v double, so every cell's value is
 // a sequence of float roundings in galaxy order.  Here each galaxy gets its
-// cell as a key (pos_to_ngp of its position, misc_tools.c:163-173; dead
-// galaxies get the key N^3), the (key, galaxy index) pairs are sorted by key
-// with a stable radix sort (rocPRIM), and the first galaxy of every run of
-// equal keys sums its run in galaxy order with the reference's roundings and
-// writes the cell's final values into the padded grids (the reference's final
-// pass, :1530-1600).  The grids are therefore identical to the reference's,
+// cell as a key (pos_to_ngp of its position, misc_tools.c:163-173), the (key,
+// galaxy index) pairs are sorted by key with a stable radix sort (rocPRIM), and
+// the first galaxy of every run of equal keys sums its run in galaxy order with
+// the reference's roundings and writes the cell's final values into the padded
+// grids (the reference's final pass, :1530-1600).  Dead galaxies are dealt over
+// the cells with a mark in their index that the sums skip: a key of their own
+// past the last cell would cost a sort pass where N^3 is a power of 256 and put
+// them all in one run.  The grids are therefore identical to the reference's,
 // bit for bit, whatever the number of galaxies per cell.
 #include <hip/hip_runtime.h>
 
@@ -31,7 +33,7 @@ struct GridArgs {
   int N;
   int bh;    // Flag_BHFeedback
   int spin;  // Flag_IncludeSpinTemp
-  unsigned ncell;  // N^3, also the key of a dead galaxy
+  unsigned ncell;  // N^3
   double box_size;
   double bh_limit;  // BlackHoleMassLimitReion
   double a_bh, a_uv;  // ReionAlphaUVBH, ReionAlphaUV
@@ -50,21 +52,37 @@ __device__ __forceinline__ int ngp(float x, double side, int nx)
   return (int)v;
 }
 
-// Keys and counts: counts[0] dead galaxies, counts[1] galaxies below the black
+constexpr unsigned kDead = 0x80000000u;  // mark of a dead galaxy in its index (n < 2^31)
+
+// The values of one galaxy, side by side: the sums read them in cell order,
+// one 32-byte access per galaxy instead of four scattered ones.
+struct alignas(32) GalVal {
+  double fesc, gross, bhm, ebhm;
+};
+
+// Keys, values and counts: counts[0] dead galaxies, counts[1] galaxies below the black
 // hole mass limit (N_BlackHoleMassLimitReion, :1473-1478); *bad = the lowest
-// index of a galaxy whose grid index is negative.  Grid-stride, with the
-// counts reduced per workgroup (one atomic per workgroup and counter).
+// index of a galaxy whose grid index is negative.  Grid-stride over at most
+// 1024 workgroups, with the counts reduced per workgroup (one atomic per
+// workgroup and counter: the atomics of 4096 workgroups on one line took most
+// of 117 us for 2e6 galaxies).
 __global__ __launch_bounds__(kGT) void k_grid_keys(const float* __restrict__ pos, const int* __restrict__ type,
-                                                   const double* __restrict__ bhm, GridArgs a, long n,
+                                                   const double* __restrict__ fesc,
+                                                   const double* __restrict__ gross,
+                                                   const double* __restrict__ bhm,
+                                                   const double* __restrict__ ebhm, GridArgs a, long n,
                                                    unsigned* __restrict__ keys, unsigned* __restrict__ vals,
+                                                   GalVal* __restrict__ gal,
                                                    unsigned long long* __restrict__ counts, int* __restrict__ bad)
 {
   __shared__ unsigned red[2][kGT / 64];
   unsigned n_dead = 0, n_below = 0;
   for (long g = (long)blockIdx.x * kGT + threadIdx.x; g < n; g += (long)gridDim.x * kGT) {
-    unsigned key = a.ncell;
+    unsigned key = (unsigned)g % a.ncell, val = (unsigned)g;
+    const double m = a.bh ? bhm[g] : 0.0;
     if (type[g] > 2) {
       ++n_dead;
+      val |= kDead;
     } else {
       const int ix = ngp(pos[3 * g], a.box_size, a.N);
       const int iy = ngp(pos[3 * g + 1], a.box_size, a.N);
@@ -73,10 +91,11 @@ __global__ __launch_bounds__(kGT) void k_grid_keys(const float* __restrict__ pos
         atomicMin(bad, (int)g);
       else
         key = (unsigned)iz + (unsigned)a.N * ((unsigned)iy + (unsigned)a.N * (unsigned)ix);
-      if (a.bh && !(bhm[g] >= a.bh_limit)) ++n_below;
+      if (a.bh && !(m >= a.bh_limit)) ++n_below;
     }
     keys[g] = key;
-    vals[g] = (unsigned)g;
+    vals[g] = val;
+    gal[g] = GalVal{fesc[g], a.spin ? gross[g] : 0.0, m, a.bh ? ebhm[g] : 0.0};
   }
   for (int o = 32; o > 0; o >>= 1) {
     n_dead += __shfl_xor(n_dead, o);
@@ -99,66 +118,96 @@ __global__ __launch_bounds__(kGT) void k_grid_keys(const float* __restrict__ pos
   }
 }
 
-// The galaxy values in sorted (cell, galaxy) order, so that each cell's run is
-// summed from contiguous memory.
-__global__ __launch_bounds__(kGT) void k_grid_gather(const unsigned* __restrict__ sval, long n,
-                                                     const double* __restrict__ fesc,
-                                                     const double* __restrict__ gross,
-                                                     const double* __restrict__ bhm,
-                                                     const double* __restrict__ ebhm, GridArgs a,
-                                                     double* __restrict__ f_s, double* __restrict__ g_s,
-                                                     double* __restrict__ m_s, double* __restrict__ e_s)
+// The grids before the sums, in one pass: stars, weighted_sfr and (spin) sfr
+// zeroed, the SFR history ring moved by one slot (:1376-1398, :1580-1600), its
+// slot 0 zeroed at the real cells, its padding kept.  V floats per access: 4
+// when every grid is 16-byte aligned (a grid of N N (N + 2) floats, N even, is a
+// whole number of them, so every slot is aligned as the first), else 1.  A
+// launch per copied slot and per zeroed grid took 370 us for the 1.2 GB of
+// 256^3 grids and 8 slots.
+constexpr int kShift = 4;  // slots in flight per thread
+template <int V>
+struct alignas(4 * V) Floats {
+  float v[V];
+};
+template <int V>
+__global__ __launch_bounds__(kGT) void k_grid_init(float* __restrict__ stars, float* __restrict__ wsfr,
+                                                   float* __restrict__ sfr, float* hist, int nstore, unsigned n,
+                                                   int N)
 {
-  const long q = (long)blockIdx.x * kGT + threadIdx.x;
-  if (q >= n) return;
-  const unsigned g = sval[q];
-  f_s[q] = fesc[g];
-  if (a.spin) g_s[q] = gross[g];
-  if (a.bh) {
-    m_s[q] = bhm[g];
-    e_s[q] = ebhm[g];
+  using P = Floats<V>;
+  const unsigned i = blockIdx.x * kGT + threadIdx.x;  // of n accesses per grid
+  if (i >= n) return;
+  const P zero = {};
+  reinterpret_cast<P*>(stars)[i] = zero;
+  reinterpret_cast<P*>(wsfr)[i] = zero;
+  if (!nstore) return;
+  reinterpret_cast<P*>(sfr)[i] = zero;
+  P* h = reinterpret_cast<P*>(hist) + i;
+  P first = h[0];
+  // slots from the last down, kShift of them loaded before the first is stored
+  for (int s = nstore - 1; s >= 1; s -= kShift) {
+    P v[kShift];
+#pragma unroll
+    for (int u = 0; u < kShift; ++u)
+      if (s - u >= 1) v[u] = h[(size_t)(s - u - 1) * n];
+#pragma unroll
+    for (int u = 0; u < kShift; ++u)
+      if (s - u >= 1) h[(size_t)(s - u) * n] = v[u];
   }
-}
-
-// Real cells of one padded grid set to 0 (the new slot 0 of the history ring
-// is overwritten at every real cell, its padding kept).
-__global__ __launch_bounds__(kGT) void k_zero_real(float* __restrict__ g, int N)
-{
-  const long i = (long)blockIdx.x * kGT + threadIdx.x;
-  if (i >= (long)N * N * N) return;
-  const long r = i / N;
-  g[r * (N + 2) + (i % N)] = 0.0f;
+  const unsigned z0 = (unsigned)((unsigned long long)i * V % (unsigned)(N + 2));
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    const unsigned z = z0 + k, zr = z >= (unsigned)(N + 2) ? z - (N + 2) : z;
+    if (zr < (unsigned)N) first.v[k] = 0.0f;
+  }
+  h[0] = first;
 }
 
 // The first galaxy of each run of equal keys sums the run in galaxy order and
 // writes the cell (reionization.c:1436-1515 accumulation, :1530-1600 final
-// pass); the values come in sorted order from k_grid_gather.
-__global__ __launch_bounds__(kGT) void k_grid_accumulate(const unsigned* __restrict__ skey, long n,
-                                                         const double* __restrict__ f_s,
-                                                         const double* __restrict__ g_s,
-                                                         const double* __restrict__ m_s,
-                                                         const double* __restrict__ e_s, GridArgs a,
+// pass).  The next kAhead entries of the run are loaded before the first is
+// added: a crowded cell's run is one thread's serial chain (128 us of 2e6
+// galaxies on 256^3 went to runs of about a hundred, one load after another).
+constexpr int kAhead = 4;
+__global__ __launch_bounds__(kGT) void k_grid_accumulate(const unsigned* __restrict__ skey,
+                                                         const unsigned* __restrict__ sval, long n,
+                                                         const GalVal* __restrict__ gal, GridArgs a,
                                                          float* __restrict__ stars, float* __restrict__ wsfr,
                                                          float* __restrict__ sfr, float* __restrict__ hist0)
 {
   const long p = (long)blockIdx.x * kGT + threadIdx.x;
   if (p >= n) return;
   const unsigned key = skey[p];
-  if (key >= a.ncell) return;
   if (p > 0 && skey[p - 1] == key) return;
   float st = 0.0f, ws = 0.0f, sf = 0.0f;
-  for (long q = p; q < n && skey[q] == key; ++q) {
-    const double f = f_s[q];
-    st = (float)((double)st + f);  // prop_stellar
-    ws = (float)((double)ws + f);  // prop_weighted_sfr
-    if (a.bh) {
-      if (m_s[q] >= a.bh_limit) {
-        const double e = e_s[q];
-        st = (float)((double)st + e);
-        ws = (float)((double)ws + e * a.a_bh / a.a_uv);
-      }
+  bool more = true;
+  for (long q = p; more; q += kAhead) {
+    bool in[kAhead], alive[kAhead];
+    GalVal g[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      in[u] = q + u < n && skey[q + u] == key;
+      const unsigned v = in[u] ? sval[q + u] : kDead;
+      alive[u] = !(v & kDead);
+      if (alive[u]) g[u] = gal[v];
     }
-    if (a.spin) sf = (float)((double)sf + g_s[q]);  // prop_sfr
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      more = more && in[u];
+      if (!alive[u]) continue;
+      const double f = g[u].fesc;
+      st = (float)((double)st + f);  // prop_stellar
+      ws = (float)((double)ws + f);  // prop_weighted_sfr
+      if (a.bh) {
+        if (g[u].bhm >= a.bh_limit) {
+          const double e = g[u].ebhm;
+          st = (float)((double)st + e);
+          ws = (float)((double)ws + e * a.a_bh / a.a_uv);
+        }
+      }
+      if (a.spin) sf = (float)((double)sf + g[u].gross);  // prop_sfr
+    }
   }
   const unsigned N = (unsigned)a.N;
   const long pad = (long)(key / N) * (N + 2) + key % N;  // INDEX_PADDED of the INDEX_REAL key
@@ -185,7 +234,7 @@ __global__ __launch_bounds__(kGT) void k_grid_accumulate(const unsigned* __restr
 
 // device buffer slots of ctx_buffer used here
 enum { S_KEY, S_VAL, S_KEY2, S_VAL2, S_SORT, S_CNT, S_POS, S_TYPE, S_FESC, S_GROSS, S_BHM, S_EBHM, S_STARS,
-       S_WSFR, S_SFR, S_HIST, S_FS, S_GS, S_MS, S_ES };
+       S_WSFR, S_SFR, S_HIST, S_GAL };
 
 template <class T>
 int stage_in(mrx_ctx* ctx, int slot, const T* host, size_t n, const T** dev)
@@ -282,13 +331,15 @@ extern "C" int mrx_construct_baryon_grids(mrx_ctx* ctx, const mrx_grid_params* p
   unsigned* keys2 = static_cast<unsigned*>(ctx_buffer(ctx, S_KEY2, sizeof(unsigned) * (ng + 1)));
   unsigned* vals2 = static_cast<unsigned*>(ctx_buffer(ctx, S_VAL2, sizeof(unsigned) * (ng + 1)));
   unsigned long long* cnt = static_cast<unsigned long long*>(ctx_buffer(ctx, S_CNT, 64));
-  if (!keys || !vals || !keys2 || !vals2 || !cnt) return MRX_ENOMEM;
+  GalVal* gal = static_cast<GalVal*>(ctx_buffer(ctx, S_GAL, sizeof(GalVal) * ng));
+  if (!keys || !vals || !keys2 || !vals2 || !cnt || !gal) return MRX_ENOMEM;
   int* bad = reinterpret_cast<int*>(cnt + 2);
   const unsigned long long init[3] = {0ull, 0ull, 0x7fffffffull};
   G_TRY(hipMemcpyAsync(cnt, init, sizeof init, hipMemcpyHostToDevice, st));
   const unsigned nb = (unsigned)((ng + kGT - 1) / kGT);
   if (ng) {
-    k_grid_keys<<<nb < 4096 ? nb : 4096, kGT, 0, st>>>(dpos, dtype, dbhm, a, n_gal, keys, vals, cnt, bad);
+    k_grid_keys<<<nb < 1024 ? nb : 1024, kGT, 0, st>>>(dpos, dtype, dfesc, dgross, dbhm, debhm, a, n_gal, keys,
+                                                       vals, gal, cnt, bad);
     G_TRY(hipGetLastError());
   }
   unsigned long long h[3];
@@ -301,36 +352,27 @@ extern "C" int mrx_construct_baryon_grids(mrx_ctx* ctx, const mrx_grid_params* p
                     "misc_tools.c:170)",
                     first_bad);
 
-  // the grids start at zero (:1376-1398); the SFR history ring moves by one slot
-  G_TRY(hipMemsetAsync(dstars, 0, sizeof(float) * np, st));
-  G_TRY(hipMemsetAsync(dwsfr, 0, sizeof(float) * np, st));
-  if (spin) {
-    G_TRY(hipMemsetAsync(dsfr, 0, sizeof(float) * np, st));
-    for (long s = (long)nstore - 2; s >= 0; --s)
-      G_TRY(hipMemcpyAsync(dhist + (size_t)(s + 1) * np, dhist + (size_t)s * np, sizeof(float) * np,
-                           hipMemcpyDeviceToDevice, st));
-    const long nr = (long)N * N * N;
-    k_zero_real<<<(unsigned)((nr + kGT - 1) / kGT), kGT, 0, st>>>(dhist, N);
+  {
+    const uintptr_t align = reinterpret_cast<uintptr_t>(dstars) | reinterpret_cast<uintptr_t>(dwsfr) |
+                            (spin ? reinterpret_cast<uintptr_t>(dsfr) | reinterpret_cast<uintptr_t>(dhist) : 0);
+    const unsigned n4 = (unsigned)(np / 4), n1 = (unsigned)np;
+    if ((align & 15) == 0)
+      k_grid_init<4><<<(n4 + kGT - 1) / kGT, kGT, 0, st>>>(dstars, dwsfr, dsfr, dhist, (int)nstore, n4, N);
+    else
+      k_grid_init<1><<<(unsigned)((np + kGT - 1) / kGT), kGT, 0, st>>>(dstars, dwsfr, dsfr, dhist, (int)nstore, n1, N);
     G_TRY(hipGetLastError());
   }
 
   if (ng) {
-    // stable sort of (cell, galaxy) by cell; the dead galaxies' key N^3 sorts last
+    // stable sort of (cell, galaxy) by cell
     unsigned bits = 1;
-    while (bits < 32 && ((unsigned long long)a.ncell >> bits) != 0) ++bits;
+    while (bits < 32 && ((unsigned long long)(a.ncell - 1) >> bits) != 0) ++bits;
     size_t tmp_bytes = 0;
     G_TRY(rocprim::radix_sort_pairs(nullptr, tmp_bytes, keys, keys2, vals, vals2, (unsigned)ng, 0, bits, st));
     void* tmp = ctx_buffer(ctx, S_SORT, tmp_bytes);
     if (!tmp) return MRX_ENOMEM;
     G_TRY(rocprim::radix_sort_pairs(tmp, tmp_bytes, keys, keys2, vals, vals2, (unsigned)ng, 0, bits, st));
-    double* f_s = static_cast<double*>(ctx_buffer(ctx, S_FS, sizeof(double) * ng));
-    double* g_s = spin ? static_cast<double*>(ctx_buffer(ctx, S_GS, sizeof(double) * ng)) : nullptr;
-    double* m_s = bh ? static_cast<double*>(ctx_buffer(ctx, S_MS, sizeof(double) * ng)) : nullptr;
-    double* e_s = bh ? static_cast<double*>(ctx_buffer(ctx, S_ES, sizeof(double) * ng)) : nullptr;
-    if (!f_s || (spin && !g_s) || (bh && (!m_s || !e_s))) return MRX_ENOMEM;
-    k_grid_gather<<<nb, kGT, 0, st>>>(vals2, n_gal, dfesc, dgross, dbhm, debhm, a, f_s, g_s, m_s, e_s);
-    G_TRY(hipGetLastError());
-    k_grid_accumulate<<<nb, kGT, 0, st>>>(keys2, n_gal, f_s, g_s, m_s, e_s, a, dstars, dwsfr, dsfr, dhist);
+    k_grid_accumulate<<<nb, kGT, 0, st>>>(keys2, vals2, n_gal, gal, a, dstars, dwsfr, dsfr, dhist);
     G_TRY(hipGetLastError());
   }
 
