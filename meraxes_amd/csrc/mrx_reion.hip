@@ -743,17 +743,28 @@ struct Pipe {
     k_unpack_dc<N><<<dim3((N * N + 255) / 256, 1), 256, 0, ctx->stream>>>(U, V, nc, (long)N * N);
     return check_launch(ctx, "k_unpack_dc");
   }
-  static int pack_herm(mrx_ctx* ctx, const float2* H, float2* U)
+  // padded real grid -> half spectrum in the caller's layout
+  static int forward_herm(mrx_ctx* ctx, const float* in, float2* H)
   {
-    const long n = nc;
-    k_herm_to_packed<N><<<(unsigned)((n + 255) / 256), 256, 0, ctx->stream>>>(H, U);
-    return check_launch(ctx, "k_herm_to_packed");
+    FieldTab t{};
+    t.p[0] = in;
+    k_r2c_z<N><<<dim3(N * N / Cfg<N>::RZ, 1), kNT, 0, ctx->stream>>>(t, ctx->U, ctx->tw, nc);
+    MRX_TRY(check_launch(ctx, "k_r2c_z"));
+    const unsigned tiles = N * (NH / Cfg<N>::TW);
+    k_colpass<N, false><<<tiles, Cfg<N>::COL_NT, 0, ctx->stream>>>(ctx->U, ctx->tw, nc, (long)N * NH, NH, 0.0);
+    MRX_TRY(check_launch(ctx, "k_colpass y"));
+    k_colpass_herm<N, false><<<tiles, Cfg<N>::COL_NT, 0, ctx->stream>>>(ctx->U, H, ctx->tw);
+    MRX_TRY(check_launch(ctx, "k_colpass_herm x"));
+    k_unpack_dc_herm<N><<<(N * N + 255) / 256, 256, 0, ctx->stream>>>(H);
+    return check_launch(ctx, "k_unpack_dc_herm");
   }
-  static int unpack_herm(mrx_ctx* ctx, const float2* U, const float2* V, float2* H)
+  // half spectrum in the caller's layout -> packed spectrum with the x and y passes done
+  static int inv_xy_herm(mrx_ctx* ctx, const float2* H, float2* T)
   {
-    const long n = (long)N * N * (NH + 1);
-    k_packed_to_herm<N><<<(unsigned)((n + 255) / 256), 256, 0, ctx->stream>>>(U, V, H);
-    return check_launch(ctx, "k_packed_to_herm");
+    k_colpass_herm<N, true><<<N * (NH / Cfg<N>::TW), Cfg<N>::COL_NT, 0, ctx->stream>>>(H, T, ctx->tw);
+    MRX_TRY(check_launch(ctx, "k_colpass_herm x inv"));
+    colpass_y<true>(ctx, T, 1, 0.0);
+    return check_launch(ctx, "k_colpass y inv");
   }
   // inverse x then y pass on packed spectra in place (no window)
   static int inv_xy_plain(mrx_ctx* ctx, float2* T, int nfield)
@@ -1080,8 +1091,7 @@ struct R2C {
     {
       using P = Pipe<N>;
       MRX_TRY(ensure_buffers(ctx, N, 1));
-      MRX_TRY(P::forward(ctx, in, false, ctx->U, ctx->V));
-      return P::unpack_herm(ctx, ctx->U, ctx->V, out);
+      return P::forward_herm(ctx, in, out);
     }
   };
 };
@@ -1093,8 +1103,7 @@ struct C2R {
     {
       using P = Pipe<N>;
       MRX_TRY(ensure_buffers(ctx, N, 1));
-      MRX_TRY(P::pack_herm(ctx, in, ctx->T));
-      MRX_TRY(P::inv_xy_plain(ctx, ctx->T, 1));
+      MRX_TRY(P::inv_xy_herm(ctx, in, ctx->T));
       return P::c2r_z(ctx, ctx->T, out, 1, -1);
     }
   };
@@ -2270,7 +2279,9 @@ int mrx_filter(mrx_ctx* ctx, float* box, int local_ix_start, int slab_nx, int gr
     HIP_TRY(hipMemcpyAsync(d, box, sizeof(float2) * n, hipMemcpyHostToDevice, ctx->stream));
   }
   const WinArgs w = win_args(box_size, R, filter_type, 1);
-  k_filter_herm<<<(unsigned)((n + 255) / 256), 256, 0, ctx->stream>>>(d, local_ix_start, slab_nx, grid_dim, w);
+  const long waves = (long)slab_nx * (grid_dim / 2 + 1);
+  k_filter_herm<<<(unsigned)((waves + kFilterRows - 1) / kFilterRows), 64 * kFilterRows, 0, ctx->stream>>>(
+    d, local_ix_start, slab_nx, grid_dim, w);
   MRX_TRY(check_launch(ctx, "k_filter_herm"));
   if (!on_device) {
     HIP_TRY(hipMemcpyAsync(box, d, sizeof(float2) * n, hipMemcpyDeviceToHost, ctx->stream));

@@ -328,6 +328,71 @@ __global__ __launch_bounds__((TileMap<N, TW, MAXNT>::NT), 4) void k_colpass(floa
   for (int i = 0; i < EPT; ++i) store_nt(g + (unsigned)(i * RPI) * rs, r[i]);
 }
 
+// The x passes between a packed spectrum and a half spectrum in the caller's
+// layout (rows of N / 2 + 1, INDEX_COMPLEX_HERM): the transform of k_colpass
+// with the conversion in its loads or stores, which saves a pass over the
+// spectrum each way.  Forward: packed `in` to half spectrum `out`, whose kz = 0
+// column gets the packed kz = 0 and N / 2 planes (k_unpack_dc_herm splits
+// them).  Inverse: half spectrum to packed, that column formed as A + i B.
+// Rows of N / 2 + 1 complex start at any 8-byte boundary, so neighbouring tiles
+// share cache lines: the tiles are dealt so that each XCD writes a contiguous
+// range of them (workgroup g runs on XCD g mod 8).
+template <int N, bool INV, int TW = Cfg<N>::TW>
+__global__ __launch_bounds__((TileMap<N, TW>::NT), 4) void k_colpass_herm(const float2* __restrict__ in,
+                                                                    float2* __restrict__ out,
+                                                                    const float2* __restrict__ twN)
+{
+  using M = TileMap<N, TW>;
+  constexpr int NT = M::NT, SP = M::SP, RPI = M::RPI, EPT = M::EPT, NKZB = M::NKZB;
+  constexpr int NH = N / 2, NH1 = NH + 1, T = N * NKZB;
+  constexpr int PI = INV ? NH1 : NH, PO = INV ? NH : NH1;  // row pitches
+  __shared__ float2 s[N * SP];
+  __shared__ float2 tw[N];
+  const int tid = threadIdx.x;
+  const int c = tid % TW, n0 = tid / TW;
+  const int tile = (T % 8 == 0) ? (int)(blockIdx.x % 8) * (T / 8) + (int)(blockIdx.x / 8) : (int)blockIdx.x;
+  const int y = tile / NKZB, kz = (tile % NKZB) * TW + c;
+  const float2* g = in + (long)y * PI + kz + (unsigned)n0 * (unsigned)(N * PI);
+  float2 r[EPT];
+#pragma unroll
+  for (int i = 0; i < EPT; ++i) r[i] = g[(unsigned)(i * RPI) * (unsigned)(N * PI)];
+  if (INV && kz == 0) {
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) {
+      const float2 B = g[(unsigned)(i * RPI) * (unsigned)(N * PI) + NH];
+      r[i] = make_float2(r[i].x - B.y, r[i].y + B.x);
+    }
+  }
+  for (int i = tid; i < N; i += NT) tw[i] = twN[i];
+  fft_tile_reg<N, TW, NT, INV, SP>(r, s, tw, tid);
+  float2* o = out + (long)y * PO + kz + (unsigned)n0 * (unsigned)(N * PO);
+#pragma unroll
+  for (int i = 0; i < EPT; ++i) o[(unsigned)(i * RPI) * (unsigned)(N * PO)] = r[i];
+}
+
+// k_unpack_dc on a half spectrum: column kz = 0 holds P = A + iB; A stays
+// there, B goes to column N / 2.
+template <int N>
+__global__ void k_unpack_dc_herm(float2* __restrict__ H)
+{
+  constexpr int NH = N / 2, NH1 = NH + 1;
+  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= N * N) return;
+  const int kx = idx / N, ky = idx % N;
+  const int midx = (N - kx) % N * N + (N - ky) % N;
+  if (idx > midx) return;  // the pair is handled by its canonical member
+  const float2 P = H[(long)idx * NH1], qc = cconj(H[(long)midx * NH1]);
+  const float2 A = cscale(cadd(P, qc), 0.5f);
+  const float2 d = csub(P, qc);
+  const float2 B = make_float2(0.5f * d.y, -0.5f * d.x);
+  H[(long)idx * NH1] = A;
+  H[(long)idx * NH1 + NH] = B;
+  if (midx != idx) {
+    H[(long)midx * NH1] = cconj(A);
+    H[(long)midx * NH1 + NH] = cconj(B);
+  }
+}
+
 // k_colpass over a subset of its tiles: kz blocks below nkzb only (grid
 // nline x nkzb per field, tile t = line t / nkzb, kz block t % nkzb), and
 // with lmax >= 0 only the lines ky with min(ky, N - ky) <= lmax (line j is ky
@@ -744,47 +809,27 @@ __global__ void k_unpack_dc(float2* __restrict__ U, float2* __restrict__ V, long
   }
 }
 
-// --------------------------------------------------- layout conversions
-// packed spectrum (+ separate Nyquist plane) <-> INDEX_COMPLEX_HERM
-template <int N>
-__global__ void k_packed_to_herm(const float2* __restrict__ U, const float2* __restrict__ V, float2* __restrict__ H)
+// filter() on a reference-layout half spectrum slab, in place.  A wave takes
+// the rows (nx, ny) and (nx, N - ny), whose modes have the same |k|, so the
+// window (bound by its FP64 sines below kR = 4) is evaluated once for both;
+// grid slab_nx x (N / 2 + 1) waves, kFilterRows of them per workgroup.
+constexpr int kFilterRows = 4;
+__global__ __launch_bounds__(64 * kFilterRows) void k_filter_herm(float2* __restrict__ H, int local_ix_start,
+                                                                  int slab_nx, int N, WinArgs w)
 {
-  constexpr int NH = N / 2;
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)N * N * (NH + 1)) return;
-  const long row = idx / (NH + 1);
-  const int kz = (int)(idx % (NH + 1));
-  const int x = (int)(row / N), y = (int)(row % N);
-  H[idx] = (kz < NH) ? U[row * NH + kz] : V[(long)y * N + x];
-}
-
-template <int N>
-__global__ void k_herm_to_packed(const float2* __restrict__ H, float2* __restrict__ U)
-{
-  constexpr int NH = N / 2;
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)N * N * NH) return;
-  const long row = idx / NH;
-  const int kz = (int)(idx % NH);
-  if (kz == 0) {
-    const float2 A = H[row * (NH + 1)], B = H[row * (NH + 1) + NH];
-    U[idx] = make_float2(A.x - B.y, A.y + B.x);  // A + iB
-  } else {
-    U[idx] = H[row * (NH + 1) + kz];
+  const int NH = N / 2, NH1 = NH + 1;
+  const long q = (long)blockIdx.x * kFilterRows + threadIdx.x / 64;
+  if (q >= (long)slab_nx * NH1) return;
+  const int ix = (int)(q / NH1), ny = (int)(q % NH1);
+  float2* a = H + ((long)ix * N + ny) * NH1;
+  const bool two = ny != 0 && 2 * ny != N;
+  float2* b = H + ((long)ix * N + (N - ny)) * NH1;  // used when two
+  for (int nz = threadIdx.x % 64; nz < NH1; nz += 64) {
+    const float wv = window(ix + local_ix_start, ny, nz, N, w);
+    if (wv == 1.0f) continue;
+    a[nz] = cscale(a[nz], wv);
+    if (two) b[nz] = cscale(b[nz], wv);
   }
-}
-
-// filter() on a reference-layout half spectrum slab, in place.
-__global__ void k_filter_herm(float2* __restrict__ H, int local_ix_start, int slab_nx, int N, WinArgs w)
-{
-  const int NH1 = N / 2 + 1;
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)slab_nx * N * NH1) return;
-  const int nz = (int)(idx % NH1);
-  const long r = idx / NH1;
-  const int ny = (int)(r % N), nx = (int)(r / N) + local_ix_start;
-  const float wv = window(nx, ny, nz, N, w);
-  if (wv != 1.0f) H[idx] = cscale(H[idx], wv);
 }
 
 // ------------------------------------------------------------ reductions

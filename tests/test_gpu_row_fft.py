@@ -62,7 +62,9 @@ def test_ladder_rows_against_the_oracle(ctx, N, spin, rec, ftype):
 @pytest.mark.parametrize("N,spin,ftype", [(32, 0, 0), (96, 1, 2), (256, 0, 1), (256, 1, 0)])
 def test_ladder_without_the_uvb_leaves_the_sfr_out(ctx, N, spin, ftype):
     """The weighted SFR only feeds J_21: without the UVB the ladder transforms one field less
-    (two or three, also where rows of 256^3 go through registers), every other output the same."""
+    (two or three, also where rows of 256^3 go through registers), every other grid the same.
+    The cells are dealt to lanes by the number of fields there, so the globals' double sums are
+    formed in another order: some 30 roundings of 2^-53 along each path of the reduction."""
     print(f"N={N} spin={spin} filter={ftype}", flush=True)
     d, s, w = synth.snapshot_inputs(N, 80 + N)
     xe = None
@@ -73,5 +75,5 @@ def test_ladder_without_the_uvb_leaves_the_sfr_out(ctx, N, spin, ftype):
     for k in ("xH", "r_bubble", "z_at_ionization"):
         assert np.array_equal(r[0][k], r[1][k]), k
     for k in ("volume_weighted_global_xH", "mass_weighted_global_xH", "n_radii"):
-        assert r[0][k] == r[1][k], k
+        assert abs(r[0][k] - r[1][k]) <= 30 * 2.0**-53 * abs(r[1][k]), k
     assert (r[0]["r_bubble"] > 0).any()
