@@ -604,8 +604,10 @@ struct Pipe {
       MRX_TRY(check_launch(ctx, "k_ix_filter (sharp-k)"));
       {
         PROF("colpass_y_inv");
-        k_colpass_live<N><<<dim3(N * nkzb, nfield), Cfg<N>::COL_NT, 0, ctx->stream>>>(T, ctx->tw, nc, (long)N * NH,
-                                                                                    NH, nkzb, nmax);
+        SharpkTab t{};
+        for (int f = 0; f < nfield; ++f) t.nmax[f] = nmax;
+        k_colpass_live<N><<<dim3(N * nkzb, nfield), Cfg<N>::COL_NT, 0, ctx->stream>>>(T, ctx->tw, nc, (long)N * NH, NH,
+                                                                                    t);
       }
       MRX_TRY(check_launch(ctx, "k_colpass_live y inv"));
       kzlive = nkzb * TW;
@@ -632,6 +634,34 @@ struct Pipe {
     PROF("colpass_y_inv");
     colpass_y<true>(ctx, T, nfield, 0.0);
     return check_launch(ctx, "k_colpass y inv");
+  }
+
+  // One field's spectrum U filtered by n <= kMaxSharpk sharp-k windows ws, by
+  // increasing radius with every ball smaller than the grid, back to n unpadded
+  // grids in `out` (stride N^3): three launches.  T: n spectra.
+  static int sharpk_shells(mrx_ctx* ctx, const float2* U, float2* T, const WinArgs* ws, int n, float* out, int clamp)
+  {
+    constexpr int TW = Cfg<N>::TW;
+    SharpkTab t{};
+    KzLive live{};
+    for (int f = 0; f < n; ++f) {
+      t.R[f] = ws[f].R;
+      t.nmax[f] = sharpk_nmax(ws[f], N);
+      live.p[f] = (t.nmax[f] / TW + 1) * TW;
+    }
+    const int nkzb = t.nmax[0] / TW + 1;
+    {
+      PROF("ix_filter");
+      k_ix_shells<N><<<dim3((2 * t.nmax[0] + 1) * nkzb, n), TileMap<N, TW>::NT, 0, ctx->stream>>>(
+        U, T, ctx->tw, nc, ws[0].delta_k, t);
+    }
+    MRX_TRY(check_launch(ctx, "k_ix_shells"));
+    {
+      PROF("colpass_y_inv");
+      k_colpass_live<N><<<dim3(N * nkzb, n), Cfg<N>::COL_NT, 0, ctx->stream>>>(T, ctx->tw, nc, (long)N * NH, NH, t);
+    }
+    MRX_TRY(check_launch(ctx, "k_colpass_live y inv"));
+    return c2r_z(ctx, T, out, n, clamp, N, live);
   }
 
   // The inverse x and y passes of K ladder radii with tabulated windows ws[k]
@@ -680,16 +710,22 @@ struct Pipe {
   static int c2r_z(mrx_ctx* ctx, const float2* T, float* out, int nfield, int clamp, int pitch = N + 2,
                    int kzlive = NH)
   {
+    KzLive live;
+    for (int& p : live.p) p = kzlive;
+    return c2r_z(ctx, T, out, nfield, clamp, pitch, live);
+  }
+  static int c2r_z(mrx_ctx* ctx, const float2* T, float* out, int nfield, int clamp, int pitch, const KzLive& live)
+  {
     PROF("c2r_z");
     if constexpr (N == 256 || N == 512) {
       // the row transforms in registers
       constexpr int A = N / 32;
       k_c2r_z_reg<A><<<dim3(N * N / (256 / A), nfield), 256, 0, ctx->stream>>>(T, out, ctx->tw, nc,
-                                                                              (long)N * N * pitch, clamp, pitch, kzlive);
+                                                                              (long)N * N * pitch, clamp, pitch, live);
       return check_launch(ctx, "k_c2r_z_reg");
     }
-    const dim3 gz(N * N / RowCfg<N>::ROWS, nfield);
-    k_c2r_z<N><<<gz, RowCfg<N>::NT, 0, ctx->stream>>>(T, out, ctx->tw, nc, (long)N * N * pitch, clamp, pitch, kzlive);
+    const dim3 gz(N * N / (kCzRows * RowCfg<N>::ROWS), nfield);
+    k_c2r_z<N><<<gz, RowCfg<N>::NT, 0, ctx->stream>>>(T, out, ctx->tw, nc, (long)N * N * pitch, clamp, pitch, live);
     return check_launch(ctx, "k_c2r_z");
   }
 
@@ -1391,7 +1427,11 @@ struct TsRun {
         MRX_TRY(fcoll(kLFactor * box_size / (float)N, 0));
         x_e_ave = 0.0;
       } else {
-        MRX_TRY(ensure_buffers(ctx, N, 1));
+        // shells per group of launches: spectra of half the Infinity Cache, as
+        // the ladder's radii (one from 320^3 up)
+        const int KS = (int)std::max<size_t>(
+          1, std::min<size_t>(kMaxSharpk, kLadderBytes / (sizeof(float2) * (size_t)P::nc)));
+        MRX_TRY(ensure_buffers(ctx, N, KS));
         MRX_TRY(ensure_buf(ctx, ctx->ts_work, ctx->ts_work_cap, np));
         ctx->ts_shells_N = ctx->ts_shells_n = 0;
         MRX_TRY(ensure_buf(ctx, ctx->ts_shells, ctx->ts_shells_cap, (size_t)s->nsteps * ncell));
@@ -1411,7 +1451,7 @@ struct TsRun {
         // the working grid starts as the input sfr grid: it is read in place
         // until the first shell with operations writes ts_work from it
         const float* wgrid = sfr;
-        for (int ct = 0; ct < s->nsteps; ++ct) {
+        for (int ct = 0; ct < s->nsteps;) {
           // a shell's operations in plan order, MRX_TS_MAX_OPS per launch (each
           // launch after the first reads the working grid the previous wrote)
           for (int k0 = 0; k0 < s->n_ops[ct]; k0 += MRX_TS_MAX_OPS) {
@@ -1443,9 +1483,24 @@ struct TsRun {
             else
               MRX_TRY(P::forward(ctx, wgrid, true, ctx->U, ctx->V, true));
           }
+          // the shells after this one that read the same transform, sharp-k with
+          // balls smaller than the grid, come back in the same launches
+          int n = 1;
+          if (KS > 1 && ct > 0 && w.type == MRX_FILTER_SHARPK && sharpk_nmax(w, N) < N / 2) {
+            WinArgs ws[kMaxSharpk];
+            ws[0] = w;
+            while (n < KS && ct + n < s->nsteps && s->n_ops[ct + n] == 0) {
+              ws[n] = win_args(p->box_size, (float)s->R[ct + n], p->heating_filter_type, 1);
+              ++n;
+            }
+            MRX_TRY(P::sharpk_shells(ctx, ctx->U, ctx->T, ws, n, ctx->ts_shells + (size_t)ct * ncell, 3));
+            ct += n;
+            continue;
+          }
           int kzlive;
           MRX_TRY(P::inverse_xy(ctx, ctx->U, ctx->V, ctx->T, 1, w, kzlive));
           MRX_TRY(P::c2r_z(ctx, ctx->T, ctx->ts_shells + (size_t)ct * ncell, 1, 3, N, kzlive));
+          ++ct;
         }
         ctx->ts_shells_N = N;
         ctx->ts_shells_n = s->nsteps;

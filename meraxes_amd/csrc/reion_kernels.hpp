@@ -201,6 +201,15 @@ struct FieldTab {
   const float* p[kMaxFields];
 };
 
+// Sharp-k windows of the spectra of one launch: radius and sharpk_nmax of each,
+// by value.  Of spectrum f only the kz blocks that hold kz <= nmax[f], and in
+// them the lines and points with |k| components <= nmax[f], are live.
+constexpr int kMaxSharpk = 16;
+struct SharpkTab {
+  float R[kMaxSharpk];
+  int nmax[kMaxSharpk];
+};
+
 // blockIdx.y selects the field (outputs at stride out_fstride)
 template <int N>
 __global__ __launch_bounds__(kNT) void k_r2c_z(FieldTab in, float2* __restrict__ out, const float2* __restrict__ twN,
@@ -244,15 +253,25 @@ __device__ __forceinline__ float clamp_kind(float v, int kind)
 
 // ------------------------------------------------------------- z: C2R pass
 // Packed rows -> real rows of pitch floats (the padding zeroed), with an
-// optional clamp; slots kz >= kzlive of the input are zero.  ROWS rows per
-// workgroup (row_fft.hpp); blockIdx.y selects the field.
+// optional clamp; slots kz >= kzlive of the input are zero.  kCzRows times
+// RowCfg's rows per workgroup (row_fft.hpp; those are sized for the ladder's
+// three to five fields, and one field of them leaves three quarters of the
+// threads without a first-stage unit: 121 us at 384^3, 85 with four times the
+// rows); blockIdx.y selects the field.
+constexpr int kCzRows = 4;
+// slots kz >= p[f] of field f are zero
+struct KzLive {
+  int p[kMaxSharpk];
+};
 template <int N>
 __global__ __launch_bounds__(RowCfg<N>::NT) void k_c2r_z(const float2* __restrict__ in, float* __restrict__ out,
                                                          const float2* __restrict__ twN, long in_fstride,
-                                                         long out_fstride, int clamp, int pitch, int kzlive)
+                                                         long out_fstride, int clamp, int pitch, KzLive live)
 {
+  const int kzlive = live.p[blockIdx.y];
   using C = RowCfg<N>;
-  constexpr int NH = C::NH, ROWS = C::ROWS, NT = C::NT, NBL = C::NBL, RL = C::RL;
+  constexpr int NH = C::NH, ROWS = kCzRows * C::ROWS, NT = C::NT, NBL = C::NBL, RL = C::RL;
+  static_assert((N * N) % ROWS == 0, "workgroups must tile the rows");
   __shared__ float2 s[row_lds<N>(ROWS)];
   __shared__ float2 tw[N];
   const int tid = threadIdx.x;
@@ -443,10 +462,6 @@ __global__ __launch_bounds__((TileMap<N, TW>::NT), 4) void k_colpass_sub(float2*
 // fields that end in the same grid need one inverse transform.  Grid: lines |ky|
 // <= lmax x kz blocks below nkzb (k_colpass_sub's order); R and nmax are per
 // field, nmax[f] <= lmax.  Points |kx| > lmax of acc are not written.
-struct SharpkTab {
-  float R[kMaxFields];
-  int nmax[kMaxFields];
-};
 template <int N, int TW = Cfg<N>::TW>
 __global__ __launch_bounds__((TileMap<N, TW>::NT)) void k_colpass_x_accum(const float2* __restrict__ data,
                                                                       float2* __restrict__ acc,
@@ -654,6 +669,47 @@ __global__ __launch_bounds__((TileMap<N, TW, ix_max_threads(N)>::NT)) void k_ix_
   }
 }
 
+// k_ix_filter<N, kWinSharpK> of one field at several radii (blockIdx.y, tab; every
+// nmax < N / 2, so the Nyquist plane is cut): one launch for the shells that
+// share a working grid, whose passes are a few microseconds each up to 160^3
+// (the 128^3 step ran 160 of its 200 launches for them: 1145 -> 942 us).
+// Shell f's spectrum goes to T + f tstride.  Grid: the tiles of the largest ball.
+template <int N, int TW = Cfg<N>::TW>
+__global__ __launch_bounds__((TileMap<N, TW>::NT), 4) void k_ix_shells(const float2* __restrict__ U,
+                                                                 float2* __restrict__ T,
+                                                                 const float2* __restrict__ twN, long tstride,
+                                                                 float delta_k, SharpkTab tab)
+{
+  using M = TileMap<N, TW>;
+  constexpr int NT = M::NT, SP = M::SP, RPI = M::RPI, EPT = M::EPT;
+  constexpr int NH = N / 2;
+  constexpr unsigned rs = (unsigned)N * NH;
+  __shared__ float2 s[N * SP];
+  __shared__ float2 tw[N];
+  const int tid = threadIdx.x;
+  const int c = tid % TW, n0 = tid / TW;
+  const int nmax = tab.nmax[blockIdx.y], nkzb = nmax / TW + 1, nky = 2 * nmax + 1;
+  const float R = tab.R[blockIdx.y];
+  const int j = blockIdx.x / nkzb, b = blockIdx.x % nkzb;
+  if (j >= nky) return;
+  const int ky = (j <= nmax) ? j : N - (nky - j);
+  const int aky = ky <= NH ? ky : N - ky;
+  const long base = (long)ky * NH + (long)b * TW + (unsigned)n0 * rs + c;
+  float2 r[EPT];
+#pragma unroll
+  for (int i = 0; i < EPT; ++i) {
+    const int n = n0 + i * RPI;
+    const int an = n <= NH ? n : N - n;
+    const bool in = an <= nmax && sharpk_window(k_magnitude(an, aky, b * TW + c, N, delta_k), R) != 0.0f;
+    r[i] = in ? U[base + (unsigned)(i * RPI) * rs] : make_float2(0.0f, 0.0f);
+  }
+  for (int i = tid; i < N; i += NT) tw[i] = twN[i];
+  fft_tile_reg<N, TW, NT, true, SP>(r, s, tw, tid);
+  float2* t = T + blockIdx.y * tstride + base;
+#pragma unroll
+  for (int i = 0; i < EPT; ++i) t[(unsigned)(i * RPI) * rs] = r[i];
+}
+
 // Inverse x pass of K consecutive ladder radii at once, for the tabulated
 // windows (top-hat, Gaussian): for each field, each radius k < K windows the
 // field's tile of the unfiltered spectrum U with table k (Wt + k wstride,
@@ -748,15 +804,15 @@ __global__ __launch_bounds__((TileMap<N, TW, MAXNT>::NT)) __attribute__((amdgpu_
   }
 }
 
-// Inverse pass over the live tiles of a sharp-k filtered spectrum left by
-// k_ix_filter<kWinSharpK>: kz blocks below nkzb only (grid N x nkzb per
-// field, tile t = line t / nkzb, kz block t % nkzb), and rows n with
-// min(n, N - n) > nlive read as zero.  Otherwise as k_colpass<N, true>.
+// Inverse pass over the live tiles of sharp-k filtered spectra left by
+// k_ix_filter<kWinSharpK> or k_ix_shells: per field (blockIdx.y, its nmax in
+// tab) the kz blocks that hold kz <= nmax only (grid N x the most blocks of a
+// field, tile t = line t / nkzb, kz block t mod nkzb), and rows n with min(n, N
+// - n) > nmax read as zero.  Otherwise as k_colpass<N, true>.
 template <int N, int TW = Cfg<N>::TW>
 __global__ __launch_bounds__((TileMap<N, TW>::NT), 4) void k_colpass_live(float2* __restrict__ data,
                                                                     const float2* __restrict__ twN, long fstride,
-                                                                    long astride, long rstride, int nkzb,
-                                                                    int nlive)
+                                                                    long astride, long rstride, SharpkTab tab)
 {
   using M = TileMap<N, TW>;
   constexpr int NT = M::NT, SP = M::SP, RPI = M::RPI, EPT = M::EPT;
@@ -765,7 +821,10 @@ __global__ __launch_bounds__((TileMap<N, TW>::NT), 4) void k_colpass_live(float2
   __shared__ float2 tw[N];
   const int tid = threadIdx.x;
   const int c = tid % TW, n0 = tid / TW;
+  const int nlive = tab.nmax[blockIdx.y];
+  const int nkzb = min(M::NKZB, nlive / TW + 1);
   const int a = blockIdx.x / nkzb, b = blockIdx.x % nkzb;
+  if (a >= N) return;
   const unsigned rs = (unsigned)rstride;
   float2* g = data + blockIdx.y * fstride + (long)a * astride + (long)b * TW + (unsigned)n0 * rs + c;
   float2 r[EPT];
@@ -1315,8 +1374,9 @@ __device__ __forceinline__ void row_c2r_reg(const float2 (&x)[16], float2 (&z)[1
 template <int A>
 __global__ __launch_bounds__(256) void k_c2r_z_reg(const float2* __restrict__ in, float* __restrict__ out,
                                                    const float2* __restrict__ twN, long in_fstride, long out_fstride,
-                                                   int clamp, int pitch, int kzlive)
+                                                   int clamp, int pitch, KzLive live)
 {
+  const int kzlive = live.p[blockIdx.y];
   constexpr int NH = 16 * A, N = 2 * NH, RWG = 256 / A, XP = A + 1;
   __shared__ float2 tw[N];
   __shared__ float2 xb[RWG][16 * XP];
