@@ -1671,6 +1671,8 @@ struct TbVel {
         r.cell = box_mpc / (float)N;
         r.half = (sub_w / 2.) / r.cell;
         r.frac_w = sub_w / r.cell;
+        r.r_cell = 1.0 / r.cell;
+        r.r_frac_w = 1.0 / r.frac_w;
         for (int s = 0; s < kRsdSteps; ++s) {
           r.x_off[s] = (float)(sub_w * (float)s + sub_w / 2.);
           r.x_pos[s] = (float)(r.x_off[s] / (box_mpc / (float)N));

@@ -1712,6 +1712,7 @@ struct RsdArgs {
   double cell;    // BoxSize / (float)N  [Mpc]
   double half;    // (subcell_width / 2) / cell
   double frac_w;  // subcell_width / cell
+  double r_cell, r_frac_w;  // 1 / cell, 1 / frac_w
   float x_pos[kRsdSteps];
   float x_off[kRsdSteps];
 };
@@ -1819,7 +1820,8 @@ __global__ __launch_bounds__(kNT) void k_rsd_los(float* __restrict__ dT, const f
 // can form its own sum in that order.  One thread per column kept 4 waves per
 // SIMD busy with dependent read-modify-writes and 6.7e9 FP64 placements at
 // 512^3 (37 ms; at 32^3, 1024 threads in all, 2.3 ms).  At 256^3 the whole
-// delta_T call went from 10.4 to 1.31 ms.
+// delta_T call went from 10.4 to 1.17 ms (this kernel 797 us, 940 with FP64
+// divisions for div_const).
 //
 // Phase 1, one thread per cell: each of the 50 sub-cells gets a class, "whole
 // in bin k + a" or "across k + a and k + a + 1", held as five 64-bit planes in
@@ -1839,6 +1841,18 @@ constexpr int kRsdPlanes = 5;
 constexpr double kRsdMaxDisp = 5.9;  // cells; floor(-5.9) = -6, floor(1 + 5.9) + 1 = 7
 constexpr float kRsdMargin = 1e-4f;
 
+// x / c for a snapshot constant c with r = 1 / c rounded: x r corrected twice by
+// its exact remainder gives the correctly rounded quotient (P. Markstein,
+// "Computation of elementary functions on the IBM RISC System/6000 processor",
+// 1990) for finite x with no overflow or underflow on the way, here positions
+// and widths of order 1e-17 to 10; five operations for the division's eleven.
+__device__ __forceinline__ double div_const(double x, double c, double r)
+{
+  double q = x * r;
+  q = fma(fma(-q, c, x), r, q);
+  return fma(fma(-q, c, x), r, q);
+}
+
 // Class id of a sub-cell: whole in bin a, or divided between a and a + 1.
 __device__ __forceinline__ int rsd_id(int a, bool split) { return 2 * (a + kRsdReach) + (split ? 2 : 1); }
 
@@ -1849,7 +1863,7 @@ __device__ __forceinline__ void rsd_edges(int s, double d1_low, double d2_low, d
   const double xp = a.x_pos[s];
   const double disp = (xp <= 0.5) ? d1_low + ((xp + 0.5) - 0.) * (d2_low - d1_low) / (1. - 0.)
                                   : d2_low + ((xp - 0.5) - 0.) * (d2_high - d2_low) / (1. - 0.);
-  const double pos = ((double)a.x_off[s] + disp) / a.cell;
+  const double pos = div_const((double)a.x_off[s] + disp, a.cell, a.r_cell);
   lo = pos - a.half;
   hi = pos + a.half;
 }
@@ -1871,18 +1885,19 @@ __device__ __forceinline__ int rsd_class(double lo, double hi)
 // The double share of a divided sub-cell in its lower or upper bin.
 __device__ __forceinline__ double rsd_share(double lo, double hi, bool upper, float d, const RsdArgs& a)
 {
+  auto frac = [&](double x) { return div_const(x, a.frac_w, a.r_frac_w); };
   double up, dn;
   if (lo < 0.0 && hi < 0.0) {
-    dn = (fabs(lo) - (ceil(fabs(lo)) - 1.)) / a.frac_w;
+    dn = frac(fabs(lo) - (ceil(fabs(lo)) - 1.));
     up = 1. - dn;
   } else if (lo < 0.0 && (hi > 0.0 && hi < 1.0)) {
-    up = hi / a.frac_w;
+    up = frac(hi);
     dn = 1. - up;
   } else if ((lo >= 0.0 && lo < 1.0) && hi >= 1.0) {
-    up = (hi - 1.) / a.frac_w;
+    up = frac(hi - 1.);
     dn = 1. - up;
   } else {
-    up = (hi - floor(fabs(hi))) / a.frac_w;
+    up = frac(hi - floor(fabs(hi)));
     dn = 1. - up;
   }
   return (upper ? up : dn) * (double)d / (double)(float)kRsdSteps;
@@ -1999,9 +2014,10 @@ __global__ __launch_bounds__(kNT) void k_rsd_gather(float* __restrict__ dT, cons
       while (m) {
         const int s = __ffsll((unsigned long long)m) - 1;
         if ((mf >> s) & 1) {
-          const int run = __ffsll((unsigned long long)~(mf >> s)) - 1;
-          for (int i = 0; i < run; ++i) acc = acc + share;
+          int run = __ffsll((unsigned long long)~(mf >> s)) - 1;
           m &= ~(((1ull << run) - 1) << s);
+          for (; run >= 4; run -= 4) acc = (((acc + share) + share) + share) + share;
+          for (; run > 0; --run) acc = acc + share;
         } else {
           const double dl = dsp[k == 0 ? src + N - 1 : src - 1], dc = dsp[src],
                        dh = dsp[k == N - 1 ? src - (N - 1) : src + 1];
