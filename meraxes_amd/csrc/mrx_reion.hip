@@ -1322,12 +1322,12 @@ int quad_launch(mrx_ctx* ctx, const mrx_ts_params* p, const mrx_ts_snap* s, int 
   } on_side(ctx);
   {
     PROF("nu_lower");
-    k_ts_nu_lower<<<dim3(s->nsteps, nbuild), 64, 0, ctx->stream>>>(ctx->quad_dev, a, ctx->quad_out);
+    k_ts_nu_lower<<<dim3(s->nsteps, nbuild), 128, 0, ctx->stream>>>(ctx->quad_dev, a, ctx->quad_out);
   }
   MRX_TRY(check_launch(ctx, "k_ts_nu_lower"));
   {
     PROF("freq_integrals");
-    k_ts_freq_integrals<<<dim3(s->nsteps, 3 * kNXHII, nbuild), 64, 0, ctx->stream>>>(ctx->quad_dev, a, ctx->quad_out);
+    k_ts_freq_integrals<<<dim3(s->nsteps, 3 * kNXHII, nbuild), 128, 0, ctx->stream>>>(ctx->quad_dev, a, ctx->quad_out);
   }
   MRX_TRY(check_launch(ctx, "k_ts_freq_integrals"));
   HIP_TRY(hipMemcpyAsync(ctx->quad_host, ctx->quad_out, sizeof(double) * nbuild * kQuadOut, hipMemcpyDeviceToHost,

@@ -6,13 +6,15 @@
 // integrals over frequency.  On 16 host threads that is 2.5-3 ms, more than
 // the device needs for the whole step up to 192^3, and the adjoint builds the
 // tables five times.  A 61-point Gauss-Kronrod rule fits a wave of 64 lanes:
-// here one wave is one integral (or one root), its lanes the nodes, the sums
-// wave butterflies, and the bisection's bookkeeping is uniform over the wave.
-// All integrals of all shells (and of several builds) run at once: about 9000
-// rules of some 4000 vector instructions, 60 us of the whole chip; the time is
-// the longest chain, 60 rules in a row (434 us, after 119 us of roots), hidden
-// behind the shells' launches.  The 128^3 step went from 3.47 to 1.14 ms, a
-// 192^3 training step from 29.5 (27.9 with the rows of row_fft.hpp) to 19.5.
+// here one workgroup of two waves is one integral (or one root), a wave's lanes
+// the nodes of a rule, its sums butterflies; the waves take the two halves of a
+// bisected interval, and the bookkeeping is uniform.  All integrals of all
+// shells (and of several builds) run at once: about 9000 rules of some 4000
+// vector instructions, 60 us of the whole chip.  The time is the longest chain,
+// 60 rules, two at a time: 302 us (434 with one wave), after 121 us of roots,
+// beside the shells' passes.  The 128^3 step went from 3.47 to 1.14 ms with one
+// wave per integral (0.94 to 0.79 with the second, the shells grouped), a 192^3
+// training step from 27.9 to 19.5.
 //
 // The algorithms, tolerances and interval order are ts_tables.c's (the host
 // build, which mrx_ts_snapshot_tables still serves); sums run over the wave in
@@ -107,9 +109,11 @@ __device__ __forceinline__ double xsec_HeI(double nu)
          pow(1.0 + sqrt(y / 1.469), -3.188);
 }
 
-// The interval lists of one wave (one workgroup).
+// The interval lists of one integral (a workgroup of two waves), and the two
+// halves' rules on their way from wave to wave.
 struct Lists {
   double a[kMaxIntervals], b[kMaxIntervals], r[kMaxIntervals], e[kMaxIntervals];
+  double half_r[2], half_e[2], half_asc[2];
 };
 
 struct Rule {
@@ -149,7 +153,8 @@ __device__ __forceinline__ double gk61(const F& f, const Rule& q, double a, doub
 }
 
 // QAG: bisects the interval with the largest error until the summed error is
-// below epsrel |result|.  Uniform over the wave; at most kMaxIntervals rules.
+// below epsrel |result|; each of the workgroup's two waves takes the rule of one
+// half.  Uniform over the workgroup; at most kMaxIntervals intervals.
 template <class F>
 __device__ double qag61(const F& f, const Rule& q, Lists& l, double a, double b, double epsrel)
 {
@@ -160,8 +165,8 @@ __device__ double qag61(const F& f, const Rule& q, Lists& l, double a, double b,
   const double round_off = 50 * DBL_EPSILON * resabs;
   if ((e0 <= round_off && e0 > tolerance) || (e0 <= tolerance && e0 != resasc) || e0 == 0.0) return r0;
   int n = 1;
-  __syncthreads();  // one wave: orders the lists' reuse
-  if (lane == 0) {
+  __syncthreads();  // the last integral's reads of the lists
+  if (threadIdx.x == 0) {
     l.a[0] = a;
     l.b[0] = b;
     l.r[0] = r0;
@@ -190,9 +195,19 @@ __device__ double qag61(const F& f, const Rule& q, Lists& l, double a, double b,
     }
     k = __builtin_amdgcn_readfirstlane(k);
     const double a1 = l.a[k], b2 = l.b[k], b1 = 0.5 * (a1 + b2), a2 = b1, rk = l.r[k], ek = l.e[k];
-    double e1, e2, ra, rs1, rs2;
-    const double r1 = gk61(f, q, a1, b1, e1, ra, rs1);
-    const double r2 = gk61(f, q, a2, b2, e2, ra, rs2);
+    const int w = threadIdx.x >> 6;
+    {
+      double e, ra, rs;
+      const double r = gk61(f, q, w ? a2 : a1, w ? b2 : b1, e, ra, rs);
+      if (lane == 0) {
+        l.half_r[w] = r;
+        l.half_e[w] = e;
+        l.half_asc[w] = rs;
+      }
+    }
+    __syncthreads();
+    const double r1 = l.half_r[0], r2 = l.half_r[1], e1 = l.half_e[0], e2 = l.half_e[1], rs1 = l.half_asc[0],
+                 rs2 = l.half_asc[1];
     const double area12 = r1 + r2, error12 = e1 + e2;
     errsum += (error12 - ek);
     area += area12 - rk;
@@ -202,8 +217,7 @@ __device__ double qag61(const F& f, const Rule& q, Lists& l, double a, double b,
       if (iteration >= 10 && error12 > ek) roundoff2++;
     }
     tolerance = epsrel * fabs(area);
-    __syncthreads();
-    if (lane == 0) {
+    if (threadIdx.x == 0) {  // every read of entry k and of the halves' slots' last values is past
       l.b[k] = b1;
       l.r[k] = r1;
       l.e[k] = e1;
@@ -385,9 +399,9 @@ struct NuIntegrand {
 
 }  // namespace quad
 
-// The shells' lower frequency limits (ComputeTs.c:560-580): one wave per shell
+// The shells' lower frequency limits (ComputeTs.c:560-580): one workgroup per shell
 // (blockIdx.x) and build (blockIdx.y).
-__global__ __launch_bounds__(64) void k_ts_nu_lower(const TsQuadDev* __restrict__ tg, TsQuadArgs a,
+__global__ __launch_bounds__(128) void k_ts_nu_lower(const TsQuadDev* __restrict__ tg, TsQuadArgs a,
                                                    double* __restrict__ out)
 {
   __shared__ quad::Lists lists;
@@ -409,9 +423,9 @@ __global__ __launch_bounds__(64) void k_ts_nu_lower(const TsQuadDev* __restrict_
   if (threadIdx.x == 0) out[(long)bd * kQuadOut + ct] = fmax(nu, a.nu_min);
 }
 
-// The frequency integrals: one wave per shell (blockIdx.x), integrand and x_e
+// The frequency integrals: one workgroup per shell (blockIdx.x), integrand and x_e
 // entry (blockIdx.y) and build (blockIdx.z), from the shell's lower limit.
-__global__ __launch_bounds__(64) void k_ts_freq_integrals(const TsQuadDev* __restrict__ tg, TsQuadArgs a,
+__global__ __launch_bounds__(128) void k_ts_freq_integrals(const TsQuadDev* __restrict__ tg, TsQuadArgs a,
                                                          double* __restrict__ out)
 {
   __shared__ quad::Lists lists;
