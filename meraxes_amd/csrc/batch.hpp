@@ -157,6 +157,8 @@ struct BatchPipe {
     mrx_ctx* ctx;
     Cohort* c;
     const WinArgs* w;  // NULL: the unfiltered last step
+    // the filtered steps' y pass is in the threshold kernel where planes fit in LDS
+    bool y_pass() const { return !w || !plane_ok<N>(); }
     template <int TW, int SV>
     int go()
     {
@@ -180,6 +182,7 @@ struct BatchPipe {
                                                                       (long)N * N, c->F, bs, bvs, WinArgs{}, N,
                                                                       M::NKZB);
       MRX_TRY(check_launch(ctx, "k_ix_filter (batch)"));
+      if (!y_pass()) return MRX_OK;
       const dim3 gy(N * M::NKZB, c->nbox * c->F);
       k_colpass<N, true, TW, SV><<<gy, M::NT, 0, c->stream>>>(c->T, c->tw, nc, (long)N * NH, NH, 0.0);
       return check_launch(ctx, "k_colpass y inv (batch)");
@@ -222,6 +225,15 @@ struct BatchPipe {
       a.last = last ? 1 : 0;
       constexpr int NT = RowCfg<N>::NT;
       auto thr = [&](auto fs) {
+        if constexpr (plane_ok<N>()) {
+          if (!last) {
+            using FS = decltype(fs);
+            using C = PlaneCfg<N, FS::N>;
+            k_plane_threshold_batch<N, FS><<<dim3(N * C::PARTS, c.nbox), C::NT, 0, c.stream>>>(
+              c.T, nc, (long)c.F * nc, c.tw, c.boxes_dev, c.state, c.Rtab, c.steps, c.J21c, c.S, a);
+            return;
+          }
+        }
         k_c2r_threshold_batch<N, decltype(fs)><<<dim3(nb, c.nbox), NT, 0, c.stream>>>(
           c.T, nc, (long)c.F * nc, c.tw, c.boxes_dev, c.state, c.Rtab, c.steps, c.J21c, c.S, c.partials, a);
       };
@@ -300,7 +312,7 @@ struct BatchPipe {
     return MRX_OK;
   }
 
-  // Times every variant's window table + filtered inverse x+y passes over the whole cohort
+  // Times every variant's window table + filtered inverse x (+ y) passes over the whole cohort
   // (the radius of step 0, real spectra from one forward transform) and keeps
   // the fastest.
   static int tune(mrx_ctx* ctx, Cohort& c)

@@ -22,6 +22,7 @@
 #include "../../include/mrx_reion.h"
 #include "ctx.hpp"
 #include "reion_kernels.hpp"
+#include "plane_fft.hpp"
 #include "ts_kernels.hpp"
 #include "adjoint.hpp"
 #include "ts_quad.hpp"
@@ -149,6 +150,9 @@ struct mrx_ctx {
   int ladder_radii = 0;  // radii per group; 0: chosen by size (kLadderBytes)
   float2* TK = nullptr;
   size_t TK_cap = 0;  // float2
+  // a group's crossings and J_21 candidates (plane_fft.hpp)
+  float* plane = nullptr;
+  size_t plane_cap = 0;
   float ts_h_xe0 = 0.f, ts_h_T0 = 0.f;  // RECFAST x_e, T_K of the homogeneous branch
   // adjoint work buffers
   float* adj_work = nullptr;
@@ -668,9 +672,10 @@ struct Pipe {
   // (not sharp-k): one x pass reads U once and writes the K spectra TK + k
   // tstride, then one y pass runs in place over them all.  Per radius the
   // spectra are inverse_xy's.
-  // wpre: the K radii's window tables already built (window_tables), or null
+  // wpre: the K radii's window tables already built (window_tables), or null;
+  // y_pass false: the x pass only (threshold_plane has the y pass in it)
   static int inverse_xy_k(mrx_ctx* ctx, const float2* U, const float2* V, float2* TK, long tstride, int nfield,
-                          const WinArgs* ws, int K, const float* wpre = nullptr)
+                          const WinArgs* ws, int K, const float* wpre = nullptr, bool y_pass = true)
   {
     constexpr int TW = Cfg<N>::TW;
     const long nt = (long)(NH + 1) * (NH + 1) * (NH + 1);
@@ -686,6 +691,7 @@ struct Pipe {
         U, V, TK, ctx->tw, wt, nt, nc, (long)N * N, tstride, nfield, K);
     }
     MRX_TRY(check_launch(ctx, "k_ix_filter_k"));
+    if (!y_pass) return MRX_OK;
     PROF("colpass_y_inv");
     colpass_y<true>(ctx, TK, K * nfield, 0.0);  // the group's spectra lie back to back (tstride = nfield nc)
     return check_launch(ctx, "k_colpass y inv");
@@ -764,6 +770,40 @@ struct Pipe {
                 : threshold_fs<Fields<false, true, false>>(ctx, Tsrc, tstride, K, g, a);
     return xe ? threshold_fs<Fields<true, false, false>>(ctx, Tsrc, tstride, K, g, a)
               : threshold_fs<Fields<false, false, false>>(ctx, Tsrc, tstride, K, g, a);
+  }
+
+  // The y pass and the last pass of K filtered steps together, step k's
+  // x-passed spectra at T + k tstride (plane_fft.hpp; N <= 128 without
+  // recombinations); cross and cand hold K N^3 / 2 entries.
+  template <class FS>
+  static int plane_fs(mrx_ctx* ctx, const float2* T, long tstride, int K, const ThrGrids& g, uint8_t* cross,
+                      float2* cand, const StepArgs& a)
+  {
+    using C = PlaneCfg<N, FS::N>;
+    {
+      PROF("plane_threshold");
+      k_plane_threshold<N, FS><<<dim3(N * C::PARTS, K), C::NT, 0, ctx->stream>>>(
+        T, nc, tstride, ctx->tw, ctx->steps, g, cross, cand, a);
+    }
+    MRX_TRY(check_launch(ctx, "k_plane_threshold"));
+    PROF("ladder_combine");
+    k_ladder_combine<<<(unsigned)((nc / 4 + kNT - 1) / kNT), kNT, 0, ctx->stream>>>(
+      reinterpret_cast<const uint32_t*>(cross), reinterpret_cast<const float*>(cand),
+      reinterpret_cast<uint64_t*>(ctx->state), g.J21, nc, K, a.step, a.uvb);
+    return check_launch(ctx, "k_ladder_combine");
+  }
+  static int threshold_plane(mrx_ctx* ctx, const float2* T, long tstride, int K, const ThrGrids& g, uint8_t* cross,
+                             float2* cand, bool xe, bool sfr, const StepArgs& a)
+  {
+    if constexpr (plane_ok<N>()) {
+      if (sfr)
+        return xe ? plane_fs<Fields<true, true, false>>(ctx, T, tstride, K, g, cross, cand, a)
+                  : plane_fs<Fields<false, true, false>>(ctx, T, tstride, K, g, cross, cand, a);
+      return xe ? plane_fs<Fields<true, false, false>>(ctx, T, tstride, K, g, cross, cand, a)
+                : plane_fs<Fields<false, false, false>>(ctx, T, tstride, K, g, cross, cand, a);
+    } else {
+      return set_err(ctx, MRX_EUNSUPPORTED, "no plane kernel for %d^3", N);
+    }
   }
 
   static int nblocks_threshold(bool rec)
@@ -1046,6 +1086,11 @@ struct HiiRun {
         KL = std::max(1, std::min(KL, S - 1));
       }
       if (KL > 1 && ensure_tk(ctx, (size_t)KL * tstride) != MRX_OK) KL = 1;
+      // a group's crossings and J_21 candidates, when the y pass and the test
+      // run together
+      bool plane = plane_ok<N>() && !rec && KL >= 1;
+      const size_t ncand = wsfr ? (size_t)2 * KL * P::nc : 0;  // floats
+      plane = plane && ensure_buf(ctx, ctx->plane, ctx->plane_cap, ncand + (size_t)KL * P::nc / 4) == MRX_OK;
       for (int s = 0; s < S;) {
         const bool last = (s == S - 1);
         int K = 1;
@@ -1055,7 +1100,8 @@ struct HiiRun {
           std::vector<WinArgs> ws(wpre ? 0 : K);
           for (int k = 0; k < (int)ws.size(); ++k) ws[k] = win_args(box_size, (float)R[s + k], p->filter_type, 1);
           float2* TK = KL > 1 ? ctx->TK : ctx->T;
-          MRX_TRY(P::inverse_xy_k(ctx, ctx->U, ctx->V, TK, tstride, nfield, ws.data(), K, wpre ? wpre + s * nt : nullptr));
+          MRX_TRY(P::inverse_xy_k(ctx, ctx->U, ctx->V, TK, tstride, nfield, ws.data(), K,
+                                  wpre ? wpre + s * nt : nullptr, !plane));
           a.kzlive = N / 2;
           Tsrc = TK;
         } else {
@@ -1064,7 +1110,13 @@ struct HiiRun {
         }
         a.step = s;
         a.last = last ? 1 : 0;
-        MRX_TRY(P::threshold(ctx, Tsrc, tstride, K, grids, xe, wsfr, rec, a));
+        if (plane && !last) {
+          float2* cand = reinterpret_cast<float2*>(ctx->plane);
+          uint8_t* cross = reinterpret_cast<uint8_t*>(ctx->plane + ncand);
+          MRX_TRY(P::threshold_plane(ctx, Tsrc, tstride, K, grids, cross, wsfr ? cand : nullptr, xe, wsfr, a));
+        } else {
+          MRX_TRY(P::threshold(ctx, Tsrc, tstride, K, grids, xe, wsfr, rec, a));
+        }
         s += K;
       }
       if (rec) {
@@ -2200,6 +2252,7 @@ int mrx_free(mrx_ctx* ctx)
     if (e) (void)hipEventDestroy(e);
   dfree(ctx->wtab_all);
   if (ctx->TK) (void)hipFree(ctx->TK);
+  dfree(ctx->plane);
   dfree(ctx->adj_work);
   dfree(ctx->adj_gS);
   dfree(ctx->adj_E);

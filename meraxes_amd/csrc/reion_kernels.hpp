@@ -1029,6 +1029,58 @@ struct Fields {
   static constexpr int N = 2 + SFR + XE + REC;
 };
 
+// The quantities of a cell's test (find_HII_bubbles.c:313-372) from its clamped
+// filtered fields v (Fields' order); the double ones are formed only where used.
+template <class FS>
+struct CellTest {
+  const float* v;
+  const StepArgs& a;
+  __device__ __forceinline__ double density_over_mean() const { return 1.0 + (double)v[0]; }
+  __device__ __forceinline__ double neutral_fraction() const { return FS::XE ? 1.0 - (double)v[FS::X] : 1.0; }
+  // recombinations in the cell (:360-363)
+  __device__ __forceinline__ double rec() const
+  {
+#pragma clang fp contract(off)
+    return FS::REC ? (double)v[FS::R] / density_over_mean() : 0.0;
+  }
+  // the reference's f_coll (four roundings of its exact value), evaluated
+  // where needed: the last step's partial xH and near-threshold cells
+  __device__ __forceinline__ double f_coll() const
+  {
+#pragma clang fp contract(off)
+    return (double)v[1] / (a.M_mean * density_over_mean()) * (4.0 / 3.0) * M_PI * a.R_cubed / a.pixel_volume;
+  }
+  // the weighted SFR is clamped here, where it is used (the clamp is
+  // idempotent, so a caller may pass it clamped or not)
+  __device__ __forceinline__ float sfr() const { return FS::SFR ? clamp_kind(v[FS::W], 1) : 0.0f; }
+  // J_21 of the cell at this radius (:317-320, :331-337)
+  __device__ __forceinline__ float j21() const
+  {
+#pragma clang fp contract(off)
+    return a.uvb ? (float)((double)sfr() / a.pixel_volume * a.J21c) : 0.0f;
+  }
+  // f_coll*eff > n_f as stars*kfc*eff vs n_f*(1+delta), both positive sides
+  // within 1e-14 of their exact values: a relative gap above 1e-12 fixes the
+  // reference's outcome, closer cells take its own expression
+  __device__ __forceinline__ bool cross() const
+  {
+#pragma clang fp contract(off)
+    if constexpr (!FS::REC) {
+      // the same test in single precision first: lf and rf lie within 2e-7
+      // (relative) of the exact sides, so a gap above the band's 9.5e-7 gives
+      // the double test's outcome; cells inside the band take the double test
+      const float kfe = (float)(a.kfc * a.eff);
+      const float lf = v[1] * kfe, rf = (FS::XE ? 1.0f - v[FS::X] : 1.0f) * (1.0f + v[0]);
+      if (lf > rf * 1.000001f) return true;
+      if (lf < rf * 0.999999f) return false;
+    }
+    const double lhs = (double)v[1] * a.kfc * a.eff, rhs = neutral_fraction() * (1. + rec()) * density_over_mean();
+    if (lhs > rhs * (1.0 + 1e-12)) return true;
+    if (lhs < rhs * (1.0 - 1e-12)) return false;
+    return f_coll() * a.eff > neutral_fraction() * (1. + rec());
+  }
+};
+
 // The ladder step's test of one cell (find_HII_bubbles.c:313-443).  v: the
 // cell's clamped filtered fields (Fields' order); st: its state byte.  The
 // first crossing writes the cell's J_21 (and Gamma_12 with REC); on the last
@@ -1048,59 +1100,16 @@ __device__ __forceinline__ uint32_t threshold_cell(const float* v, uint32_t st, 
                                                    float& jflag, bool& zcheck, float& jaux)
 {
 #pragma clang fp contract(off)
-  constexpr bool XE = FS::XE, REC = FS::REC;
-  // the double quantities are formed in the branches that use them: the
-  // single-precision test below decides almost every cell without them
-  auto density_over_mean = [&]() { return 1.0 + (double)v[0]; };
-  auto neutral_fraction = [&]() { return XE ? 1.0 - (double)v[FS::X] : 1.0; };
-  // recombinations in the cell (:360-363)
-  auto rec = [&]() { return REC ? (double)v[FS::R] / density_over_mean() : 0.0; };
-  // the reference's f_coll (four roundings of its exact value), evaluated
-  // where needed: the last step's partial xH and near-threshold cells
-  auto f_coll = [&]() {
-    return (double)v[1] / (a.M_mean * density_over_mean()) * (4.0 / 3.0) * M_PI * a.R_cubed / a.pixel_volume;
-  };
-  // the test f_coll*eff > n_f as stars*kfc*eff vs n_f*(1+delta), both
-  // positive sides within 1e-14 of their exact values: a relative gap
-  // above 1e-12 fixes the reference's outcome, closer cells take its
-  // own expression
-  bool cross, decided = false;
-  if constexpr (!REC) {
-    // the same test in single precision first: lf and rf lie within 2e-7
-    // (relative) of the exact sides, so a gap above the band's 9.5e-7 gives
-    // the double test's outcome; cells inside the band take the double test
-    const float kfe = (float)(a.kfc * a.eff);
-    const float lf = v[1] * kfe, rf = (XE ? 1.0f - v[FS::X] : 1.0f) * (1.0f + v[0]);
-    if (lf > rf * 1.000001f) {
-      cross = true;
-      decided = true;
-    } else if (lf < rf * 0.999999f) {
-      cross = false;
-      decided = true;
-    }
-  }
-  if (!decided) {
-    const double lhs = (double)v[1] * a.kfc * a.eff, rhs = neutral_fraction() * (1. + rec()) * density_over_mean();
-    if (lhs > rhs * (1.0 + 1e-12))
-      cross = true;
-    else if (lhs < rhs * (1.0 - 1e-12))
-      cross = false;
-    else
-      cross = f_coll() * a.eff > neutral_fraction() * (1. + rec());
-  }
-  // the weighted SFR is clamped here, where it is used (the clamp is
-  // idempotent, so a caller may pass it clamped or not)
-  auto sfr = [&]() { return FS::SFR ? clamp_kind(v[FS::W], 1) : 0.0f; };
-  // J_21 of the cell at this radius (:317-320, :331-337)
-  auto j21_aux = [&]() { return a.uvb ? (float)((double)sfr() / a.pixel_volume * a.J21c) : 0.0f; };
+  const CellTest<FS> t{v, a};
+  const bool cross = t.cross();
   const bool never = (st == 0xFFu);
   zcheck = false;
   jaux = 0.0f;
   uint32_t st_new = st;
   if (cross) {
     if (never) {
-      if (a.uvb) J21[ir] = j21_aux();
-      if (REC) Gamma12[ir] = (float)(a.gamma_pref * ((double)sfr() / a.pixel_volume));  // :398-404
+      if (a.uvb) J21[ir] = t.j21();
+      if (FS::REC) Gamma12[ir] = (float)(a.gamma_pref * ((double)t.sfr() / a.pixel_volume));  // :398-404
     }
     st_new = (uint32_t)a.step;
   }
@@ -1109,12 +1118,12 @@ __device__ __forceinline__ uint32_t threshold_cell(const float* v, uint32_t st, 
     if (ion) {
       xh = 0.0f;
     } else {
-      xh = (float)(neutral_fraction() - f_coll() * a.eff);
+      xh = (float)(t.neutral_fraction() - t.f_coll() * a.eff);
       if (xh < 0.f)
         xh = 0.f;
       else if (xh > 1.0f)
         xh = 1.f;
-      if (xh < kRelTol) jaux = j21_aux();
+      if (xh < kRelTol) jaux = t.j21();
     }
     zcheck = xh < kRelTol;  // every ionised cell, and the partial ones below REL_TOL
     rb = ion ? Rtab[cross ? a.step : (int)st] : 0.0f;

@@ -109,12 +109,13 @@ __device__ __forceinline__ void untwist_unit(float2* a, float2* b, const float2*
 }
 
 // Loads, untwists and first stage of P rows into s; load(pencil, k) returns
-// point k of a row.  Ends with a barrier.
-template <int N, int P, class Load>
+// point k of a row.  INPLACE: load reads s itself, so every point is loaded
+// before the first is overwritten.  Ends with a barrier.
+template <int N, int P, int NT = RowCfg<N>::NT, bool INPLACE = false, class Load>
 __device__ __forceinline__ void rows_first(float2* s, const float2* tw, int tid, Load load)
 {
   using C = RowCfg<N>;
-  constexpr int NH = C::NH, R1 = C::R1, Q = C::Q, U = C::U, NT = C::NT;
+  constexpr int NH = C::NH, R1 = C::R1, Q = C::Q, U = C::U;
   constexpr int NU = P * U, PT = (NU + NT - 1) / NT;
   float2 a[PT][R1], b[PT][R1];
 #pragma unroll
@@ -130,6 +131,7 @@ __device__ __forceinline__ void rows_first(float2* s, const float2* tw, int tid,
       }
     }
   }
+  if (INPLACE) __syncthreads();
 #pragma unroll
   for (int p = 0; p < PT; ++p) {
     const int e = tid + p * NT;
@@ -150,14 +152,14 @@ __device__ __forceinline__ void rows_first(float2* s, const float2* tw, int tid,
   __syncthreads();
 }
 
-template <int N, int P, int I, int NS>
+template <int N, int P, int I, int NS, int NT = RowCfg<N>::NT>
 __device__ __forceinline__ void rows_middle(float2* s, const float2* tw, int tid)
 {
   using C = RowCfg<N>;
   if constexpr (I + 1 < C::NR) {
     constexpr int R = C::S::radix[I];
-    stockham_stage<C::NH, R, NS, P, C::NT, true, 1, C::NH, false, 2, true>(s, tw, tid);
-    rows_middle<N, P, I + 1, NS * R>(s, tw, tid);
+    stockham_stage<C::NH, R, NS, P, NT, true, 1, C::NH, false, 2, true>(s, tw, tid);
+    rows_middle<N, P, I + 1, NS * R, NT>(s, tw, tid);
   }
 }
 
@@ -178,15 +180,15 @@ __device__ __forceinline__ void rows_last(const float2* s, const float2* tw, int
 // The last stage of P rows in place (a butterfly's outputs replace its
 // inputs): real cells 2n, 2n + 1 of row c are float2 lds_addr(c NH + n).  Ends
 // with a barrier.
-template <int N, int P>
+template <int N, int P, int NT = RowCfg<N>::NT>
 __device__ __forceinline__ void rows_last_lds(float2* s, const float2* tw, int tid)
 {
   using C = RowCfg<N>;
-  constexpr int NB = P * C::NBL, PT = (NB + C::NT - 1) / C::NT;
+  constexpr int NB = P * C::NBL, PT = (NB + NT - 1) / NT;
 #pragma unroll
   for (int p = 0; p < PT; ++p) {
-    const int e = tid + p * C::NT;
-    if ((NB % C::NT == 0) || e < NB) {
+    const int e = tid + p * NT;
+    if ((NB % NT == 0) || e < NB) {
       const int c = e / C::NBL, j = e % C::NBL;
       float2 v[C::RL];
       rows_last<N>(s, tw, c, j, v);
