@@ -103,13 +103,14 @@ def ladder_radii(name, S, prof, steps):
 def path_bytes_hii(N, F, S):
     """The bubble finder's algorithmic bytes for one box, the sum of its kernels'
     (kernel_bytes): F forward transforms, then per radius the windowed inverse x
-    pass, the inverse y pass and the z pass + threshold; the window tables
-    (shared by the boxes of a batch cohort) are left out."""
+    pass, the inverse y pass and the z pass + threshold (up to 128^3 the filtered
+    radii's y pass happens in the threshold's kernel and moves nothing); the
+    window tables (shared by the boxes of a batch cohort) are left out."""
     spec = 8 * N * N * (N // 2)
     fwd = kernel_bytes("r2c_z", N, F) + F * 2 * 2 * spec
-    per_radius = kernel_bytes("ix_filter", N, F) + kernel_bytes("colpass_y_inv", N, F) + kernel_bytes(
-        "c2r_threshold", N, F)
-    return fwd + S * per_radius
+    per_radius = kernel_bytes("ix_filter", N, F) + kernel_bytes("c2r_threshold", N, F)
+    y_passes = 1 if N <= 128 else S
+    return fwd + S * per_radius + y_passes * kernel_bytes("colpass_y_inv", N, F)
 
 
 def cpu_info():

@@ -79,12 +79,12 @@ double* resolve_scratch(int device)
 // otherwise it is as many as keep the group's spectra within kLadderBytes, two
 // at least.  Two bring the x pass to the y pass's rate at 512^3 (more gain
 // nothing there).  On small grids a pass over one radius is a few microseconds
-// of work behind a launch of the same length: 64^3 with three fields runs all
-// 37 filtered radii in one group (711 -> 315 us per call; 373 with 8 per
-// group).  The bound keeps a group's spectra in the 256 MB Infinity Cache from
-// pass to pass: 128^3 with four fields takes 1553, 1440, 1485, 1588 and 1684
-// us with 2, 4, 6, 8 and 12 radii per group; from 160^3 up the number matters
-// by less than 3 %.
+// of work behind a launch of the same length: 64^3 with three fields takes 451,
+// 344, 286, 261 and 207 us per call with 2, 4, 8, 12 and all 38 filtered radii
+// in a group.  The bound keeps a group's spectra in the 256 MB Infinity Cache
+// from pass to pass: 128^3 with four fields takes 1365, 1251, 1265, 1387 and
+// 1381 us with 2, 4, 6, 8 and 12 radii per group; from 160^3 up the number
+// matters by less than 3 %.
 constexpr int kLadderRadiiMax = 64;
 constexpr size_t kLadderBytes = (size_t)128 << 20;
 
