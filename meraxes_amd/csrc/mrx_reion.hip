@@ -123,8 +123,9 @@ struct mrx_ctx {
   mrx_ts_data* tsd = nullptr;
   std::string ts_key;
   mrx_ts_snap* tss = nullptr;
-  TsDev* ts_host = nullptr;  // pinned: its upload does not stop the host
+  TsDev* ts_host = nullptr;  // pinned: its upload does not stop the host (ts_upload)
   TsDev* ts_dev = nullptr;
+  hipEvent_t ts_uploaded = nullptr;  // the last upload of ts_host
   // the frequency integrals on the device (ts_quad.hpp): their tables, for the
   // table set quad_key, and the results of up to kQuadBuilds builds
   TsQuadDev* quad_dev = nullptr;
@@ -1405,6 +1406,26 @@ int quad_results(mrx_ctx* ctx, int b, mrx_ts_snap* s)
   return MRX_OK;
 }
 
+// The constants of the planned snapshot (ctx->tsd, ctx->tss, p) into ts_host, and
+// their copy to ts_dev queued.  The buffer is pinned: the copy reads it when the
+// stream gets there, which on a caller's stream can be after the call that
+// queued it has returned (an adjoint whose grid means are not measured waits
+// for nothing), so the last copy is waited for before the buffer is filled again.
+// A captured copy reads it at every replay and has no event to wait for.
+int ts_upload(mrx_ctx* ctx, const mrx_ts_params* p)
+{
+  if (!ctx->ts_uploaded)
+    HIP_TRY(hipEventCreateWithFlags(&ctx->ts_uploaded, hipEventDisableTiming));
+  else
+    HIP_TRY(hipEventSynchronize(ctx->ts_uploaded));
+  fill_ts_dev(*ctx->ts_host, ctx->tsd, ctx->tss, p);
+  HIP_TRY(hipMemcpyAsync(ctx->ts_dev, ctx->ts_host, sizeof(TsDev), hipMemcpyHostToDevice, ctx->stream));
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(ctx->stream, &capture));
+  if (capture == hipStreamCaptureStatusNone) HIP_TRY(hipEventRecord(ctx->ts_uploaded, ctx->stream));
+  return MRX_OK;
+}
+
 struct TsRun {
   template <int N>
   struct At {
@@ -1463,8 +1484,7 @@ struct TsRun {
         const float zp = (float)s->zp;
         const float xe0 = (float)mrx_ts_xion_RECFAST(d, zp);
         const float T0 = (float)mrx_ts_T_RECFAST(d, zp);
-        fill_ts_dev(*ctx->ts_host, d, s, p);
-        HIP_TRY(hipMemcpyAsync(ctx->ts_dev, ctx->ts_host, sizeof(TsDev), hipMemcpyHostToDevice, ctx->stream));
+        MRX_TRY(ts_upload(ctx, p));
         ctx->ts_h_xe0 = xe0;
         ctx->ts_h_T0 = T0;
         if (prepare_only) return MRX_OK;
@@ -1558,8 +1578,7 @@ struct TsRun {
         ctx->ts_shells_n = s->nsteps;
         if (mrx_ts_finish_tables(s, d, p) != MRX_OK) return set_err(ctx, MRX_EINVAL, "spin-temperature tables failed");
         MRX_TRY(quad_results(ctx, 0, s));
-        fill_ts_dev(*ctx->ts_host, d, s, p);
-        HIP_TRY(hipMemcpyAsync(ctx->ts_dev, ctx->ts_host, sizeof(TsDev), hipMemcpyHostToDevice, ctx->stream));
+        MRX_TRY(ts_upload(ctx, p));
         if (prepare_only) return MRX_OK;
         {
           PROF("cell");
@@ -2263,6 +2282,7 @@ int mrx_free(mrx_ctx* ctx)
   delete ctx->tsd;
   delete ctx->tss;
   if (ctx->ts_host) (void)hipHostFree(ctx->ts_host);
+  if (ctx->ts_uploaded) (void)hipEventDestroy(ctx->ts_uploaded);
   dfree(ctx->quad_dev);
   dfree(ctx->quad_out);
   if (ctx->quad_host) (void)hipHostFree(ctx->quad_host);
