@@ -88,6 +88,11 @@ double* resolve_scratch(int device)
 constexpr int kLadderRadiiMax = 64;
 constexpr size_t kLadderBytes = (size_t)128 << 20;
 
+// Work space of the adjoint's groups of shells: eight of them at 512^3 take 9.7
+// GB.  The MRX_ADJOINT_SHELLS environment variable (0..8), read when a context
+// is created, sets the shells of a group instead.
+constexpr size_t kAdjointBytes = (size_t)12 << 30;
+
 struct mrx_ctx {
   int device = 0;
   hipStream_t own_stream = nullptr;
@@ -156,6 +161,7 @@ struct mrx_ctx {
   size_t plane_cap = 0;
   float ts_h_xe0 = 0.f, ts_h_T0 = 0.f;  // RECFAST x_e, T_K of the homogeneous branch
   // adjoint work buffers
+  int adj_shells = -1;  // shells per group; -1: chosen by size (kAdjointBytes)
   float* adj_work = nullptr;
   size_t adj_work_cap = 0;
   double* adj_gS = nullptr;
@@ -2011,14 +2017,21 @@ struct SnapAdj {
       // adjoints, and those that reach the same state of the working grid (no
       // operations between them) one inverse transform of the sum of their
       // filtered spectra.  G padded grids and spectra, the summed spectrum and
-      // one grid: at most 12 GiB, two shells at least.
+      // one grid, at most kAdjointBytes and as many as there is memory for; G = 0
+      // takes each shell by itself, with two padded grids.
       const size_t per = np + (size_t)ncell;
-      const int G = (int)std::max<size_t>(2, std::min<size_t>(kMaxFields, ((size_t)12 << 30) / (sizeof(float) * per)));
-      MRX_TRY(ensure_buf(ctx, ctx->adj_work, ctx->adj_work_cap, G * per + (size_t)ncell + np));
+      int G = ctx->adj_shells >= 0
+                ? ctx->adj_shells
+                : (int)std::min<size_t>(kMaxFields, std::max<size_t>(1, kAdjointBytes / (sizeof(float) * per)) - 1);
+      for (;; G /= 2) {
+        const int rc = ensure_buf(ctx, ctx->adj_work, ctx->adj_work_cap, G > 0 ? (G + 1) * per : 2 * np);
+        if (rc == MRX_OK) break;
+        if (rc != MRX_ENOMEM || G == 0) return rc;
+      }
       float* gshell = ctx->adj_work;
       float2* spec = reinterpret_cast<float2*>(gshell + G * np);
       float2* acc = spec + (size_t)G * P::nc;
-      float* tmp = reinterpret_cast<float*>(acc + P::nc);
+      float* tmp = G > 0 ? reinterpret_cast<float*>(acc + P::nc) : gshell + np;
       const long half = (long)N * N * (N / 2 + 1);
       auto shell_grad = [&](int ct, int n, const float* unclamped) -> int {
         PROF("adjoint_shell_grad");
@@ -2042,7 +2055,7 @@ struct SnapAdj {
         // sharp-k shells whose balls of modes are smaller than the grid (the
         // radii increase, so these are the last of the run) are summed
         int first_sum = hi + 1;
-        if (tp->heating_filter_type == MRX_FILTER_SHARPK)
+        if (G > 0 && tp->heating_filter_type == MRX_FILTER_SHARPK)
           while (first_sum > std::max(lo, 1) && sharpk_nmax(shell_win(first_sum - 1), N) < N / 2) --first_sum;
         for (int ct = first_sum; ct <= hi; ct += G) {
           const int n = std::min(G, hi + 1 - ct);
@@ -2234,6 +2247,10 @@ int mrx_init(int device, mrx_ctx** out)
   if (const char* e = getenv("MRX_LADDER_RADII")) {
     const int k = atoi(e);
     if (k >= 1 && k <= kLadderRadiiMax) ctx->ladder_radii = k;
+  }
+  if (const char* e = getenv("MRX_ADJOINT_SHELLS")) {
+    const int k = atoi(e);
+    if (*e && k >= 0 && k <= kMaxFields) ctx->adj_shells = k;
   }
   *out = ctx;
   return MRX_OK;
