@@ -1505,11 +1505,15 @@ struct TsRun {
         MRX_TRY(fcoll(kLFactor * box_size / (float)N, 0));
         x_e_ave = 0.0;
       } else {
-        // shells per group of launches: spectra of half the Infinity Cache, as
-        // the ladder's radii (one from 320^3 up)
-        const int KS = (int)std::max<size_t>(
-          1, std::min<size_t>(kMaxSharpk, kLadderBytes / (sizeof(float2) * (size_t)P::nc)));
-        MRX_TRY(ensure_buffers(ctx, N, KS));
+        // sharp-k shells per group of launches, their spectra in TK: as many as
+        // the ladder has radii in a group for one field (one from 320^3 up), one
+        // where TK cannot be had
+        int KS = 1;
+        if (p->heating_filter_type == MRX_FILTER_SHARPK)
+          KS = (int)std::min<size_t>(
+            kMaxSharpk, ctx->ladder_radii ? ctx->ladder_radii : kLadderBytes / (sizeof(float2) * (size_t)P::nc));
+        MRX_TRY(ensure_buffers(ctx, N, 1));
+        if (KS > 1 && ensure_tk(ctx, (size_t)KS * P::nc) != MRX_OK) KS = 1;
         MRX_TRY(ensure_buf(ctx, ctx->ts_work, ctx->ts_work_cap, np));
         ctx->ts_shells_N = ctx->ts_shells_n = 0;
         MRX_TRY(ensure_buf(ctx, ctx->ts_shells, ctx->ts_shells_cap, (size_t)s->nsteps * ncell));
@@ -1571,7 +1575,7 @@ struct TsRun {
               ws[n] = win_args(p->box_size, (float)s->R[ct + n], p->heating_filter_type, 1);
               ++n;
             }
-            MRX_TRY(P::sharpk_shells(ctx, ctx->U, ctx->T, ws, n, ctx->ts_shells + (size_t)ct * ncell, 3));
+            MRX_TRY(P::sharpk_shells(ctx, ctx->U, ctx->TK, ws, n, ctx->ts_shells + (size_t)ct * ncell, 3));
             ct += n;
             continue;
           }
