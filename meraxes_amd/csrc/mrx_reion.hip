@@ -2941,8 +2941,8 @@ int mrx_hii_batch_describe(const mrx_hii_batch* b, char* buf, int len)
     (void)cohort_dispatch(c.N, sh);
     char tmp[256];
     snprintf(tmp, sizeof tmp, "%s{\"grid_dim\": %d, \"boxes\": %d, \"fields\": %d, \"radii\": %d, \"variant\": %d, "
-             "\"tile_width\": %d, \"radix_schedule\": %d, \"tune_ms\": [", k ? ", " : "", c.N, c.nbox, c.p0.include_spin_temp ? 4 : 3, c.S,
-             c.variant, sh.tw, sh.sv);
+             "\"tile_width\": %d, \"radix_schedule\": %d, \"tune_ms\": [", k ? ", " : "", c.N, c.nbox, c.F, c.S, c.variant, sh.tw,
+             sh.sv);
     s += tmp;
     for (size_t v = 0; v < c.tune_ms.size(); ++v) {
       snprintf(tmp, sizeof tmp, "%s%.4f", v ? ", " : "", c.tune_ms[v]);

@@ -106,6 +106,19 @@ def test_tuned_batch_parity_with_oracle(ctx):
     batch.close()
 
 
+@pytest.mark.parametrize("spin,uvb,fields", [(0, 0, 2), (0, 1, 3), (1, 0, 3), (1, 1, 4)])
+def test_described_fields_are_those_transformed(ctx, spin, uvb, fields):
+    """deltax and stars, the weighted SFR only with the UVB (it enters J_21 alone), x_e with spin temperature."""
+    d, s, w = (torch.from_numpy(a).cuda() for a in synth.snapshot_inputs(32, 4))
+    p = P.hii_params(32, 50.0, 8.0, uvb_flag=uvb, include_spin_temp=spin)
+    box = {"params": p, "deltax": d, "stars": s, "weighted_sfr": w}
+    if spin:
+        box["x_e"] = torch.full_like(d, 1e-3)
+    batch = reion.HiiBatch(ctx, [box], graph=False, tune=False)
+    assert [c["fields"] for c in batch.describe()["cohorts"]] == [fields]
+    batch.close()
+
+
 def test_batch_rejects_host_grids_and_bad_params(ctx):
     d, s, w = synth.snapshot_inputs(32, 1)
     p = P.hii_params(32, 50.0, 8.0)
