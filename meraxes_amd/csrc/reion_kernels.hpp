@@ -1843,11 +1843,16 @@ __global__ __launch_bounds__(kNT) void k_rsd_los(float* __restrict__ dT, const f
 // reference's order of k (the wrapped ones where the reference meets them),
 // the runs of whole sub-cells are float additions of d / 50 and the divided
 // ones take the reference's double fractions.
-// Reach: kRsdReach bins either way; a column with a larger (or non-finite)
-// displacement is flagged in `todo` and left untouched for k_rsd_los.
-constexpr int kRsdReach = 7;         // 2 (2 * 7 + 1) - 1 = 29 classes, ids 1..29 in five bits
-constexpr int kRsdPlanes = 5;
-constexpr double kRsdMaxDisp = 5.9;  // cells; floor(-5.9) = -6, floor(1 + 5.9) + 1 = 7
+// Reach: a column with a displacement above kRsdMaxDisp (or a non-finite one) is
+// flagged in `todo` and left untouched for k_rsd_los.  The others' sub-cells lie
+// in the bins -(kRsdReach - 1) to kRsdReach - 1 of their cell: their edges within
+// [-kRsdMaxDisp, 1 + kRsdMaxDisp].  Offset -kRsdReach has ids, but no sub-cell may
+// reach it: a bin that far away would ask for id 0, every sub-cell without a class.
+constexpr int kRsdReach = 7;
+constexpr int kRsdPlanes = 5;        // bits of an id
+constexpr double kRsdMaxDisp = 5.9;  // cells
+static_assert(kRsdMaxDisp < kRsdReach - 1, "a sub-cell's bins lie closer than kRsdReach");
+static_assert(2 * (2 * kRsdReach - 1) + 2 < 1 << kRsdPlanes, "ids must fit the planes");
 constexpr float kRsdMargin = 1e-4f;
 
 // x / c for a snapshot constant c with r = 1 / c rounded: x r corrected twice by
