@@ -59,7 +59,10 @@ def kernel_bytes(name, N, F, radii=1.0):
     ``radii`` is the average number of ladder radii one launch of this kernel
     covers (ladder_radii): ix_filter_k reads each field's spectrum once and
     writes one per radius, the y pass reads and writes each radius's, and the
-    threshold pass reads each radius's and one byte of state per cell once.
+    threshold pass reads each radius's and one byte of state per cell once.  Up
+    to 128^3 plane_threshold reads each filtered radius's spectra and the state
+    and writes a byte of crossings per cell pair, which ladder_combine reads (the
+    J_21 of first crossings depends on the data and is left out).
     """
     if name.startswith("ts_"):
         name, F = name[3:], 1
@@ -85,19 +88,29 @@ def kernel_bytes(name, N, F, radii=1.0):
         # inverse z pass + threshold: read each field's spectrum, 1 byte of step state per cell
         "c2r_threshold": F * spec * radii + 2 * Nr,
         "r2c_z": F * (4 * N * N * (N + 2) + spec),
-        "window_table": 4 * (N // 2 + 1) ** 3,
+        "plane_threshold": (F * spec + Nr // 2) * radii + Nr,
+        "ladder_combine": Nr // 2 * radii + 2 * Nr,
+        "window_table": 4 * (N // 2 + 1) ** 3 * radii,
         "brightness_temp": 4 * N * N * (N + 2) + 2 * 4 * Nr,
     }
     return table.get(name)
 
 
 def ladder_radii(name, S, prof, steps):
-    """Ladder radii per launch of a kernel, from the launches of a profiled run:
-    the S - 1 filtered radii over ix_filter_k's, all S over the y and threshold passes'."""
+    """Ladder radii per launch of a kernel, from the launches of a profiled run.
+
+    The S - 1 filtered radii over the launches of the tables and of the x pass,
+    and up to 128^3 of the plane and combining kernels (the y and threshold
+    passes then take the unfiltered last step alone); otherwise all S over the
+    y and threshold passes'."""
     n = prof.get(name, (0, 0))[1] / steps
-    if not n or name not in ("ix_filter_k", "colpass_y_inv", "c2r_threshold"):
+    if not n:
         return 1.0
-    return (S - 1 if name == "ix_filter_k" else S) / n
+    if name in ("window_table", "ix_filter_k", "plane_threshold", "ladder_combine"):
+        return (S - 1) / n
+    if name in ("colpass_y_inv", "c2r_threshold"):
+        return (1 if "plane_threshold" in prof else S) / n
+    return 1.0
 
 
 def path_bytes_hii(N, F, S):
@@ -506,7 +519,8 @@ BATCH_PER_SIZE = 32
 
 def bench_batched(ctx, steps, warmup, per_size=BATCH_PER_SIZE):
     """96 uneven boxes (32 each of 64^3, 128^3, 192^3, 100 Mpc/h, z=8, top-hat,
-    three fields, efficiency U[10, 40], own seed each): the batch replayed as one
+    without the UVB, which leaves two fields to transform, efficiency U[10, 40], own
+    seed each): the batch replayed as one
     graph launch, against the per-box plain loop over the same boxes."""
     import numpy as np
     import torch
@@ -527,7 +541,7 @@ def bench_batched(ctx, steps, warmup, per_size=BATCH_PER_SIZE):
             p = P.hii_params(N, 100.0, 8.0, filter_type=0, efficiency=float(rng.uniform(10.0, 40.0)))
             S = len(P.radius_ladder(p))
             cells_radii += N**3 * S
-            mbytes += model_bytes_hii(N, 3, S, False)
+            mbytes += model_bytes_hii(N, 2, S, False)
             boxes.append({"params": p, "deltax": d, "stars": s, "weighted_sfr": w})
     torch.cuda.synchronize()
     t0 = time.perf_counter()
@@ -601,7 +615,7 @@ def bench_batched(ctx, steps, warmup, per_size=BATCH_PER_SIZE):
         "graph_nodes": info["graph_nodes"],
         "cohorts": [{k: c[k] for k in ("grid_dim", "boxes", "radii", "variant", "tile_width", "radix_schedule")}
                     for c in info["cohorts"]],
-        "config": {"workload": "32 x 64^3 + 32 x 128^3 + 32 x 192^3 boxes, 100 Mpc/h, z=8, top-hat, 3 fields, "
+        "config": {"workload": "32 x 64^3 + 32 x 128^3 + 32 x 192^3 boxes, 100 Mpc/h, z=8, top-hat, no UVB (2 fields), "
                                "eps U[10,40], synthetic (torch generator)"},
     }
 
