@@ -365,7 +365,7 @@ int mrx_power_spectrum_adjoint(mrx_ctx* ctx, int grid_dim, double box_size_mpc, 
  * xH = n_f - eff f_coll.  `ts` NULL: no spin temperature (tb and hii must not
  * use it).  With ts, the gradient reaches through the shell tables' two grid
  * means (the collapse fraction and <x_e>, ComputeTs.c:413-475): their
- * derivatives are taken by central differences of the host table build and
+ * derivatives are taken by central differences of the table build and
  * spread back over the cells the means are taken from.  ts->fixed_globals
  * holds them at ts->fixed_collapse_fraction and ts->fixed_x_e_ave instead,
  * forward and adjoint alike (a stop-gradient on the means).

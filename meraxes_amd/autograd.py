@@ -6,8 +6,8 @@
 (BrightnessTemperature.c:24-124) - on the HIP path and returns delta_T as a
 torch tensor whose backward is the library's hand-written adjoint
 (mrx_snapshot_adjoint): the ionisation mask is a stop-gradient, per-radius
-fields are recomputed in the backward rather than stored, and the shell
-tables' two grid means are held fixed.  ``power_spectrum(...)`` is Compute_PS
+fields are recomputed in the backward rather than stored, and the gradient
+reaches through the shell tables' two grid means unless ts_params fixes them.  ``power_spectrum(...)`` is Compute_PS
 (ComputePowerSpectrum.c:44-255) with mrx_power_spectrum_adjoint as its
 backward.  Gradients flow to deltax, stars, sfr, the SFR history, x_e_prev and
 T_K; weighted_sfr only feeds J_21, so its gradient is zero.

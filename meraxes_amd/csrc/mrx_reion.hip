@@ -2367,7 +2367,7 @@ int mrx_find_hii_bubbles_rec(mrx_ctx* ctx, const mrx_hii_params* p, const float*
   const float* in[5] = {deltax, stars, weighted_sfr, x_e, rec ? N_rec : nullptr};
   float* outp[6] = {xH, r_bubble, J_21, z_at_ionization, J_21_at_ionization, rec ? Gamma12 : nullptr};
   if (p->pointers_on_device) {
-    // the kernels move four cells per 16-byte access
+    // the last step moves two cells per 8-byte access; 16 bytes are asked for at every size alike
     for (const float* q : {deltax, stars, weighted_sfr, x_e, (const float*)xH, (const float*)r_bubble,
                            (const float*)J_21, (const float*)z_at_ionization, (const float*)J_21_at_ionization,
                            (const float*)in[4], (const float*)outp[5]})

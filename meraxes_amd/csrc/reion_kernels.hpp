@@ -1309,20 +1309,6 @@ __device__ __forceinline__ void c2r_threshold_rows(const float2* __restrict__ T,
   }
 }
 
-// The fused z pass + threshold with the row transforms in registers, for
-// rows of NH = 16 A complex (A = 16: 512^3, A = 8: 256^3) and two to four
-// fields (no N_rec).  A field's packed row is held by A lanes, lane t holding
-// points t + A m, m < 16.  The C2R untwist pairs point k with NH - k, held by
-// lane (A - t) mod A (a lane shuffle); the length-NH inverse transform is a
-// 16-point DFT of each lane's registers, a twiddle, one exchange through LDS,
-// and A-point DFTs, after which lane t holds z[t + A j], j < 16, the real
-// cells 2n and 2n + 1 of n = t + A j.  A workgroup is one wave per field, its
-// groups of A lanes dealt to (row, field) pairs, so no lane idles with two or
-// three fields; the fields of a cell meet through LDS, and the points j of a
-// row are split over its lane groups.  Three barriers per workgroup and two LDS round trips, where staging the rows in LDS for a
-// Stockham transform takes eight and five.  Per cell the test is
-// threshold_cell's, as in c2r_threshold_rows, one step per launch (a loop over
-// two steps spilled at four waves per SIMD: 541 -> 560 us per step at 512^3).
 // Inverse real transform (C2R) of packed rows of NH = 16 A complex held by A
 // lanes each: lane t = lane mod A holds points t + A m of its row in x[m] (m <
 // 16), and gets z[j] = point t + A j of the row's complex output (real cells
@@ -1409,6 +1395,16 @@ __global__ __launch_bounds__(256) void k_c2r_z_reg(const float2* __restrict__ in
   if (pitch > N && t == 0) *reinterpret_cast<float2*>(o + N) = make_float2(0.0f, 0.0f);
 }
 
+// The fused z pass + threshold with the row transforms in registers (row_c2r_reg),
+// for rows of NH = 16 A complex (A = 16: 512^3, A = 8: 256^3) and two to four
+// fields (no N_rec).  A workgroup is one wave per field, its groups of A lanes
+// dealt to (row, field) pairs, so no lane idles with two or three fields.  The
+// fields of a cell meet through LDS, and the points j of a row are split over
+// the row's lane groups.  Four barriers per workgroup and two LDS round trips,
+// where staging the rows in LDS for a Stockham transform takes eight and five.
+// Per cell the test is threshold_cell's, as in c2r_threshold_rows, one step per
+// launch (a loop over two steps spilled at four waves per SIMD: 541 -> 560 us per
+// step at 512^3).
 template <int A, int NF>
 struct RegThr {
   static constexpr int NH = 16 * A, N = 2 * NH;

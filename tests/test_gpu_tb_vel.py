@@ -117,8 +117,8 @@ def test_tb_vel_large_displacements_rebinning_exact(ctx):
 def test_tb_vel_rebinning_gather_exact(ctx, N, disp, width):
     """The gathered re-binning against the oracle's serial one, bit for bit, on the GPU's own
     pec_vels 2 field: one to sixteen columns per workgroup, cells that cross each other
-    (steep velocities), and columns on either side of the gather's reach of 7 cells
-    (displacements of 4 and 30 cells rms: some and nearly all beyond it)."""
+    (steep velocities), and columns on either side of the gather's largest displacement, 5.9
+    cells (4 and 30 cells rms: some and nearly all beyond it)."""
     xH, d, TS, vel = inputs(N, 100.0 * N / 64, 51 + N, 0, disp_rms=disp, width=width)
     p2 = P.tb_vel_params(N, 100.0 * N / 64, 8.0, pec_vels=2, trees_id=0)
     p3 = P.tb_vel_params(N, 100.0 * N / 64, 8.0, pec_vels=3, trees_id=0)
